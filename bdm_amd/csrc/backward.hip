@@ -24,8 +24,7 @@
 // S-wide column reductions use permlane swaps and DPP row sums
 // (reduce-scatter: each output ends in one lane, no LDS round trip).
 //
-// routed_backward_kernel: the general path (any S <= 32, intervals 4/8/16).
-// Same arithmetic; pieces of SUB events, operands loaded per event.
+// staged_backward_kernel: every other S <= 32 and interval of 4, 8 or 16.
 //
 // token_grad_kernel: one workgroup per token, one wave per head.  Lane
 // (j, r) = (lane / 8, lane % 8) handles route slot j and state row r of the
@@ -98,258 +97,6 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
     const int hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(x) >> 32)));
     return int64_t((uint64_t(uint32_t(hi)) << 32) | uint64_t(uint32_t(lo)));
 }
-
-template <int N>
-__device__ __forceinline__ void wave_reduce(float (&x)[N]) {
-    // Butterfly: every lane ends with the same total (each step adds the
-    // same two operands on both partners, and FP32 addition commutes).
-#pragma unroll
-    for (int m = kLanes / 2; m >= 1; m >>= 1) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) x[i] += __shfl_xor(x[i], m, kLanes);
-    }
-}
-
-template <int S, typename E>
-__device__ __forceinline__ void load_s(const E *p, int s_real, float (&out)[S]) {
-#pragma unroll
-    for (int r = 0; r < S; ++r) out[r] = r < s_real ? to_f32(p[r]) : 0.f;
-}
-
-template <int CPL, typename E>
-__device__ __forceinline__ void load_cols(const E *row, int col0, int width, float (&out)[CPL]) {
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) out[c] = col0 + c < width ? to_f32(row[col0 + c]) : 0.f;
-}
-
-template <int S, int CPL>
-__device__ __forceinline__ void load_state_cols(const void *base, int dtype, int64_t offset, int width, int s_real,
-                                                int col0, float (&h)[S][CPL]) {
-#pragma unroll
-    for (int r = 0; r < S; ++r)
-#pragma unroll
-        for (int c = 0; c < CPL; ++c) {
-            const bool live = r < s_real && col0 + c < width;
-            const int64_t at = offset + int64_t(r) * width + c;
-            h[r][c] = !live ? 0.f
-                            : (dtype == BDM_BF16 ? to_f32(static_cast<const bf16_t *>(base)[at])
-                                                 : static_cast<const float *>(base)[at]);
-        }
-}
-
-template <typename T, int S, int CPL>
-struct WriteEvent {
-    WriteRows<S> rows;
-    float ew[CPL], value[CPL];
-};
-
-template <typename T, int S, int CPL>
-__device__ __forceinline__ void load_write(const BackwardParams<T> &p, int64_t token, float pw, int head, int col0,
-                                           WriteEvent<T, S, CPL> &ev) {
-    const int64_t row = token * p.heads + head;
-    float k[S], g[S], b[S], wv[CPL];
-    load_s<S>(p.k + row * p.s_real, p.s_real, k);
-    load_s<S>(p.g + row * p.s_real, p.s_real, g);
-    load_s<S>(p.b + row * p.s_real, p.s_real, b);
-    prepare_write_rows<T, S>(k, g, b, pw, p.routed_decay, ev.rows);
-    load_cols<CPL>(p.v + row * p.width, col0, p.width, ev.value);
-    load_cols<CPL>(p.w + row * p.width, col0, p.width, wv);
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) ev.ew[c] = round_to<T>(wv[c] * pw);
-}
-
-template <typename T, int S, int CPL, int C>
-__global__ __launch_bounds__(64) void routed_backward_kernel(BackwardParams<T> p) {
-    constexpr int SUB = C < 4 ? C : 4;
-    constexpr int NCK = C / SUB;
-    __shared__ int64_t s_token[C];
-    __shared__ int64_t s_slot[C];  // write: token*KW + j; read: token*KR + j
-    __shared__ float s_weight[C];
-    __shared__ int s_read[C];
-
-    int seg, head, tile;
-    block_item(p, seg, head, tile);
-    const int bank = seg % p.banks;
-    const int64_t bidx = seg / p.banks;
-    const int lane = threadIdx.x;
-    const int col0 = (tile * kLanes + lane) * CPL;
-    const int64_t start = p.cu[seg], end = p.cu[seg + 1];
-    const int64_t write_events = p.nt * p.kw;
-    const int64_t events = p.nt * (p.kw + p.kr);
-
-    float dm[S][CPL];
-#pragma unroll
-    for (int r = 0; r < S; ++r)
-#pragma unroll
-        for (int c = 0; c < CPL; ++c) dm[r][c] = 0.f;
-
-    const int64_t count = (end - start + C - 1) / C;
-    for (int64_t chunk = count - 1; chunk >= 0; --chunk) {
-        const int64_t base = start + chunk * C;
-        const int len = int(min(int64_t(C), end - base));
-        __syncthreads();
-        if (lane < len) {
-            int64_t o = p.order[base + lane];
-            o = o < 0 ? 0 : (o >= events ? events - 1 : o);
-            const bool rd = o >= write_events;
-            const int64_t route = rd ? o - write_events : o;
-            s_token[lane] = rd ? route / p.kr : route / p.kw;
-            s_slot[lane] = route;
-            s_weight[lane] = rd ? to_f32(p.rw[route]) : to_f32(p.ww[route]);
-            s_read[lane] = rd;
-        }
-        __syncthreads();
-
-        // state before the chunk's first event
-        float m0[S][CPL];
-        if (chunk == 0) {
-            const int64_t off = bidx * p.init_bstride + (int64_t(bank) * p.heads + head) * p.s_real * p.width + col0;
-            load_state_cols<S, CPL>(p.initial, p.init_dtype, off, p.width, p.s_real, col0, m0);
-            if (p.rounding) {
-#pragma unroll
-                for (int r = 0; r < S; ++r)
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c) m0[r][c] = round_bf16(m0[r][c]);
-            }
-        } else {
-            const int64_t row = base / C - 1;
-            load_state_cols<S, CPL>(p.snap, p.snap_dtype, (row * p.heads + head) * p.s_real * p.width + col0,
-                                    p.width, p.s_real, col0, m0);
-        }
-
-        // The state before each event of piece sc (events sc*SUB .. sc*SUB+SUB-1)
-        // is rebuilt from m0 by replaying the chunk's earlier writes; pieces
-        // are visited in reverse.  The piece loop is not unrolled, so no
-        // register array is indexed by it.
-#pragma unroll 1
-        for (int sc = NCK - 1; sc >= 0; --sc) {
-            float m[S][CPL];
-#pragma unroll
-            for (int r = 0; r < S; ++r)
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) m[r][c] = m0[r][c];
-#pragma unroll 1
-            for (int j = 0; j < sc * SUB; ++j) {
-                if (j < len && !s_read[j]) {
-                    WriteEvent<T, S, CPL> ev;
-                    load_write<T, S, CPL>(p, uniform64(s_token[j]), s_weight[j], head, col0, ev);
-                    apply_write<S, CPL>(m, ev.rows, ev.ew, ev.value);
-                }
-            }
-            float st[SUB][S][CPL];
-#pragma unroll
-            for (int jj = 0; jj < SUB; ++jj) {
-#pragma unroll
-                for (int r = 0; r < S; ++r)
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c) st[jj][r][c] = m[r][c];
-                const int j = sc * SUB + jj;
-                if (jj + 1 < SUB && j < len && !s_read[j]) {
-                    WriteEvent<T, S, CPL> ev;
-                    load_write<T, S, CPL>(p, uniform64(s_token[j]), s_weight[j], head, col0, ev);
-                    apply_write<S, CPL>(m, ev.rows, ev.ew, ev.value);
-                }
-            }
-#pragma unroll
-            for (int jj = SUB - 1; jj >= 0; --jj) {
-                const int j = sc * SUB + jj;
-                if (j >= len) continue;
-                const int64_t token = uniform64(s_token[j]);
-                const int64_t slot = uniform64(s_slot[j]);
-                const float pw = s_weight[j];
-                if (!s_read[j]) {
-                    WriteEvent<T, S, CPL> ev;
-                    load_write<T, S, CPL>(p, token, pw, head, col0, ev);
-                    // hd, u exactly as the forward computed them
-                    float hd[S][CPL], u[CPL], du[CPL];
-                    float red[3 * S];  // U = sum dm*u, X = sum hd*du, P = sum dm*hd, per row
-#pragma unroll
-                    for (int i = 0; i < 3 * S; ++i) red[i] = 0.f;
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
-                        float erase = 0.f;
-#pragma unroll
-                        for (int r = 0; r < S; ++r) {
-                            hd[r][c] = st[jj][r][c] * ev.rows.decay[r];
-                            erase = fmaf(ev.rows.a[r], hd[r][c], erase);
-                        }
-                        u[c] = fmaf(ev.ew[c], ev.value[c], -erase);
-                        float acc = 0.f;
-#pragma unroll
-                        for (int r = 0; r < S; ++r) acc = fmaf(dm[r][c], ev.rows.key[r], acc);
-                        du[c] = acc;
-                    }
-#pragma unroll
-                    for (int r = 0; r < S; ++r)
-#pragma unroll
-                        for (int c = 0; c < CPL; ++c) {
-                            red[r] = fmaf(dm[r][c], u[c], red[r]);
-                            red[S + r] = fmaf(hd[r][c], du[c], red[S + r]);
-                            red[2 * S + r] = fmaf(dm[r][c], hd[r][c], red[2 * S + r]);
-                            // dh <- (dh - a du^T) * decay (role_bank_kernel.py:130-138)
-                            dm[r][c] = (dm[r][c] - ev.rows.a[r] * du[c]) * ev.rows.decay[r];
-                        }
-                    float *du_row = p.du + (slot * p.heads + head) * p.width;
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c)
-                        if (col0 + c < p.width) du_row[col0 + c] = du[c];
-                    wave_reduce<3 * S>(red);
-                    // U, X, P of row `lane` (the token kernel forms dk, db, dg)
-                    float out_u = 0.f, out_x = 0.f, out_p = 0.f;
-#pragma unroll
-                    for (int r = 0; r < S; ++r) {
-                        if (lane == r) {
-                            out_u = red[r];
-                            out_x = red[S + r];
-                            out_p = red[2 * S + r];
-                        }
-                    }
-                    if (lane < p.s_real) {
-                        const int64_t nslots = p.nt * p.kw;
-                        float *wp = p.wpart + ((int64_t(tile) * nslots + slot) * p.heads + head) * 3 * p.s_real;
-                        wp[lane] = out_u;
-                        wp[p.s_real + lane] = out_x;
-                        wp[2 * p.s_real + lane] = out_p;
-                    }
-                } else {
-                    const int64_t row = token * p.heads + head;
-                    float q[S], eq[S], dy[CPL];
-                    load_s<S>(p.q + row * p.s_real, p.s_real, q);
-#pragma unroll
-                    for (int r = 0; r < S; ++r) eq[r] = round_to<T>(q[r] * pw);
-                    load_cols<CPL>(p.dy + row * p.width, col0, p.width, dy);
-                    float red[S];
-#pragma unroll
-                    for (int r = 0; r < S; ++r) {
-                        red[r] = 0.f;
-#pragma unroll
-                        for (int c = 0; c < CPL; ++c) red[r] = fmaf(st[jj][r][c], dy[c], red[r]);
-                    }
-                    // dh += scale * q do^T (role_bank_kernel.py:141-143)
-#pragma unroll
-                    for (int r = 0; r < S; ++r)
-#pragma unroll
-                        for (int c = 0; c < CPL; ++c) dm[r][c] += eq[r] * dy[c] * p.scale;
-                    wave_reduce<S>(red);
-                    float out_q = 0.f;
-#pragma unroll
-                    for (int r = 0; r < S; ++r)
-                        if (lane == r) out_q = red[r] * p.scale;
-                    if (lane < p.s_real)
-                        p.rpart[((int64_t(tile) * p.nt * p.kr + slot) * p.heads + head) * p.s_real + lane] = out_q;
-                }
-            }
-        }
-    }
-    // adjoint of the segment's initial state (FP32, per sequence)
-    const int64_t off = ((bidx * p.banks + bank) * p.heads + head) * p.s_real * p.width + col0;
-#pragma unroll
-    for (int r = 0; r < S; ++r)
-#pragma unroll
-        for (int c = 0; c < CPL; ++c)
-            if (r < p.s_real && col0 + c < p.width) p.dinit[off + int64_t(r) * p.width + c] = dm[r][c];
-}
-
 
 // ------------------------------------------------- S = 8, replay interval 16
 
@@ -457,9 +204,10 @@ struct Pair<float> {
     static __device__ __forceinline__ raw zero() { return make_float2(0.f, 0.f); }
 };
 
-// One entry per event of the packed order: token, route slot, is_read and
-// the route weight (FP32 bits), shared by every head.
-template <typename T>
+// One entry per event of the packed order: token, route slot (PER_TOKEN: the
+// route's index within its token), is_read and the route weight (FP32 bits),
+// shared by every head.
+template <typename T, bool PER_TOKEN>
 __global__ __launch_bounds__(256) void event_meta_kernel(const int64_t *order, int64_t events, int64_t write_events,
                                                          int kw, int kr, const T *ww, const T *rw, int4 *meta) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -470,7 +218,7 @@ __global__ __launch_bounds__(256) void event_meta_kernel(const int64_t *order, i
     const int64_t route = rd ? o - write_events : o;
     const int64_t token = rd ? route / kr : route / kw;
     const float weight = to_f32(rd ? rw[route] : ww[route]);
-    meta[e] = make_int4(int(token), int(route), rd ? 1 : 0, __float_as_int(weight));
+    meta[e] = make_int4(int(token), int(PER_TOKEN ? route - token * (rd ? kr : kw) : route), rd ? 1 : 0, __float_as_int(weight));
 }
 
 template <typename T, typename SNAP>
@@ -876,6 +624,352 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
     }
 }
 
+// ------------------------------------------- other bank sizes and intervals
+
+// Sums each of N values over the columns of a row group: the 64 / RG lanes of
+// equal lane * RG / 64.  Value o ends in the lane of the group for which
+// `at` = o and `mine` is set; other lanes return a partial sum.
+template <int RG, int N>
+__device__ __forceinline__ float reduce_columns(const float (&x)[N], int lane, int &at, bool &mine) {
+    const int pos = lane & 15;
+    if constexpr (RG == 1) {
+        mine = pos < N / 4;
+        at = (N / 4) * (lane >> 4) + (mine ? pos : 0);
+        return reduce_scatter<N>(x, lane);
+    } else {
+        constexpr int M = RG == 2 ? N / 2 : N;
+        mine = pos < M;
+        at = (mine ? pos : 0) + (RG == 2 ? M * ((lane >> 4) & 1) : 0);
+        float out = 0.f;
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            const float z = row_total(RG == 2 ? row_pair_sum(x[i], x[i + N - M]) : x[i]);
+            out = pos == i ? z : out;
+        }
+        asm volatile("" : "+v"(out));  // computed in every lane, as in reduce_scatter
+        return out;
+    }
+}
+
+// Sum over the row groups of a column, in every lane.
+template <int RG>
+__device__ __forceinline__ float sum_row_groups(float x) {
+    if constexpr (RG >= 2) x = half_pair_sum(x, x);
+    if constexpr (RG >= 4) x = row_pair_sum(x, x);
+    return x;
+}
+
+// Columns of T as loaded: a pair (CPL = 2, one load) or one.
+template <typename T, int CPL>
+struct RawCols {
+    T x;
+    __device__ __forceinline__ void load(const T *at) { x = *at; }
+    __device__ __forceinline__ float get(int) const { return to_f32(x); }
+};
+template <typename T>
+struct RawCols<T, 2> {
+    typename Pair<T>::raw x;
+    __device__ __forceinline__ void load(const T *at) { x = Pair<T>::load(at); }
+    __device__ __forceinline__ float get(int c) const { return c ? Pair<T>::hi(x) : Pair<T>::lo(x); }
+};
+
+// Chunk replay for the shapes the S = 8 chunk kernel does not take: S in {4,
+// 8, 16, 32} padded rows (s_real of them live), replay intervals C of 4, 8 or
+// 16 events.  One wave per (segment, head, tile of columns); chunks in
+// reverse.  A lane owns CPL value columns and R = S / RG rows (at most 8): RG
+// groups of 64 / RG lanes share a column's rows.
+//  * All C states of a chunk sit in registers (C*R*CPL of them, at most 128),
+//    so each write is replayed once.
+//  * The operands of the next chunk (columns, row operands, start state) are
+//    loaded when half of the chunk's events remain and put in LDS after them,
+//    so no event waits for a load; the row operands (exp, bf(b p) k, bf(q r))
+//    are formed once per event, spread over the lanes, not by every lane.
+//  * The sums over columns (U, X, P, dq) are permlane swaps and DPP adds.
+// Bound: instruction issue of the event loop.  Before it, one kernel loaded
+// every operand at its event and reduced by shuffles: 813 -> 115 us at 16,384
+// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 1,934 -> 239
+// us at 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events).  Two
+// row groups at S = 16 (32 columns per wave) double the waves, which the
+// second size needs to fill the chip, and halve a lane's states.
+template <typename T, int S, int RG, int CPL, int C>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void staged_backward_kernel(
+    BackwardParams<T> p) {
+    constexpr int R = S / RG, kCols = kLanes / RG;
+    constexpr int NR = (C * S + kLanes - 1) / kLanes;  // (event, row) operands per lane
+    constexpr int kKey = 0, kDecay = S, kErase = 2 * S, kStride = 3 * S + 4;
+    struct Staged {
+        RawCols<T, CPL> a[C], b[C];  // write: v, w; read: dy, dy
+        T x[NR], bb[NR];             // write: k, b; read: q
+        float g[NR];
+        uint32_t m0[R][CPL];  // start state (BF16 or FP32 bits)
+    };
+    __shared__ int4 s_meta[2][C];
+    __shared__ __align__(16) float s_rows[C][kStride];
+    __shared__ float s_cols[C][2 * CPL][kCols];  // write: v, bf(w p); read: dy
+
+    int seg, head, tile;
+    block_item(p, seg, head, tile);
+    const int bank = seg % p.banks;
+    const int64_t bidx = seg / p.banks;
+    const int lane = threadIdx.x;
+    const int row0 = lane / kCols * R, col = lane % kCols;
+    const int col0 = (tile * kCols + col) * CPL;
+    const bool live = col0 < p.width;
+    const int colc = live ? col0 : p.width - CPL;  // lanes past the width load valid columns and zero them
+    const int64_t start = p.cu[seg], end = p.cu[seg + 1];
+    const int count = int((end - start + C - 1) / C);
+    const int64_t hw = int64_t(p.heads) * p.width;
+    const int lane_col = head * p.width + colc;
+
+    auto chunk_len = [&](int c) { return int(min(int64_t(C), end - (start + int64_t(c) * C))); };
+    auto load_meta = [&](int c) {
+        const int len = chunk_len(c);
+        return p.meta[start + int64_t(c) * C + (lane < len ? lane : len - 1)];
+    };
+    auto store_meta = [&](int c, const int4 &m) {
+        if (lane < C) s_meta[c & 1][lane] = m;
+    };
+    // Loads of chunk c's operands and start state (its meta is in LDS).
+    auto issue_stage = [&](int c, Staged &sg) {
+        const int len = chunk_len(c);
+        const int4 *mt = s_meta[c & 1];
+#pragma unroll
+        for (int e = 0; e < C; ++e) {
+            const int4 m = mt[e < len ? e : len - 1];
+            const int64_t row = int64_t(__builtin_amdgcn_readfirstlane(m.x)) * hw;
+            const bool rd = __builtin_amdgcn_readfirstlane(m.z) != 0;
+            sg.a[e].load((rd ? p.dy : p.v) + row + lane_col);
+            sg.b[e].load((rd ? p.dy : p.w) + row + lane_col);
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int idx = (lane + i * kLanes) & (C * S - 1), e = idx / S, r = idx % S;
+            const int4 m = mt[e < len ? e : len - 1];
+            const int64_t at = (int64_t(m.x) * p.heads + head) * p.s_real + (r < p.s_real ? r : 0);
+            sg.x[i] = (m.z ? p.q : p.k)[at];
+            sg.bb[i] = p.b[at];
+            sg.g[i] = p.g[at];
+        }
+        const bool first = c == 0;
+        const void *base = first ? p.initial : p.snap;
+        const int64_t off = first ? bidx * p.init_bstride + (int64_t(bank) * p.heads + head) * p.s_real * p.width
+                                  : (((start + int64_t(c) * C) / C - 1) * p.heads + head) * p.s_real * p.width;
+        const bool half = (first ? p.init_dtype : p.snap_dtype) == BDM_BF16;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc) {
+                const int64_t at = off + int64_t(row0 + r < p.s_real ? row0 + r : 0) * p.width + colc + cc;
+                if (half) sg.m0[r][cc] = static_cast<const uint16_t *>(base)[at];
+                else sg.m0[r][cc] = static_cast<const uint32_t *>(base)[at];
+            }
+    };
+    // Operand rows and columns of chunk c into LDS, its start state into m0.
+    auto finish_stage = [&](int c, const Staged &sg, float (&m0)[R][CPL]) {
+        const int len = chunk_len(c);
+        const int4 *mt = s_meta[c & 1];
+#pragma unroll
+        for (int e = 0; e < C; ++e) {
+            const float pw = __int_as_float(mt[e < len ? e : len - 1].w);
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc) {  // (the row groups of a column store the same values)
+                s_cols[e][cc][col] = live ? sg.a[e].get(cc) : 0.f;
+                s_cols[e][CPL + cc][col] = live ? round_to<T>(sg.b[e].get(cc) * pw) : 0.f;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int idx = (lane + i * kLanes) & (C * S - 1), e = idx / S, r = idx % S;
+            const int4 m = mt[e < len ? e : len - 1];
+            const float pw = __int_as_float(m.w);
+            const float x = r < p.s_real ? to_f32(sg.x[i]) : 0.f;
+            if (m.z) {
+                s_rows[e][kKey + r] = round_to<T>(x * pw) * p.scale;
+            } else {  // prepare_write_rows of row r
+                s_rows[e][kKey + r] = x;
+                s_rows[e][kDecay + r] = r < p.s_real ? __expf(p.routed_decay ? sg.g[i] * pw : sg.g[i]) : 0.f;
+                s_rows[e][kErase + r] = round_to<T>(to_f32(sg.bb[i]) * pw) * x;
+            }
+        }
+        const bool half = (c == 0 ? p.init_dtype : p.snap_dtype) == BDM_BF16;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc) {
+                float x = __uint_as_float(half ? sg.m0[r][cc] << 16 : sg.m0[r][cc]);
+                if (c == 0 && p.rounding) x = round_bf16(x);
+                m0[r][cc] = live && row0 + r < p.s_real ? x : 0.f;
+            }
+    };
+    auto rows_of = [&](int e, int at, float (&x)[R]) {
+        const float4 *row = reinterpret_cast<const float4 *>(&s_rows[e][at + row0]);
+#pragma unroll
+        for (int i = 0; i < R / 4; ++i) {
+            const float4 f = row[i];
+            x[4 * i] = f.x, x[4 * i + 1] = f.y, x[4 * i + 2] = f.z, x[4 * i + 3] = f.w;
+        }
+    };
+    // One write on the state m before it (apply_write, its row sum over the row groups).
+    auto apply = [&](int e, float (&m)[R][CPL]) {
+        float kk[R], dd[R], a[R];
+        rows_of(e, kKey, kk);
+        rows_of(e, kDecay, dd);
+        rows_of(e, kErase, a);
+#pragma unroll
+        for (int cc = 0; cc < CPL; ++cc) {
+            float erase = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                m[r][cc] *= dd[r];
+                erase = fmaf(a[r], m[r][cc], erase);
+            }
+            const float u = fmaf(s_cols[e][CPL + cc][col], s_cols[e][cc][col], -sum_row_groups<RG>(erase));
+#pragma unroll
+            for (int r = 0; r < R; ++r) m[r][cc] = fmaf(kk[r], u, m[r][cc]);
+        }
+    };
+
+    float dm[R][CPL];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int cc = 0; cc < CPL; ++cc) dm[r][cc] = 0.f;
+
+    auto slot_of = [&](int e, int buf, int per_token) {
+        const int4 m = s_meta[buf][e];
+        return int64_t(__builtin_amdgcn_readfirstlane(m.x)) * per_token + __builtin_amdgcn_readfirstlane(m.y);
+    };
+    // Adjoint of write e with the state st before it.
+    auto write_back = [&](int e, int buf, float (&st)[R][CPL]) {
+        float kk[R], dd[R], a[R];
+        rows_of(e, kKey, kk);
+        rows_of(e, kDecay, dd);
+        rows_of(e, kErase, a);
+        float u[CPL], du[CPL];
+#pragma unroll
+        for (int cc = 0; cc < CPL; ++cc) {
+            float erase = 0.f, acc = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                st[r][cc] *= dd[r];  // hd
+                erase = fmaf(a[r], st[r][cc], erase);
+                acc = fmaf(dm[r][cc], kk[r], acc);
+            }
+            u[cc] = fmaf(s_cols[e][CPL + cc][col], s_cols[e][cc][col], -sum_row_groups<RG>(erase));
+            du[cc] = sum_row_groups<RG>(acc);
+        }
+        const int64_t slot = slot_of(e, buf, p.kw);
+        if (live && row0 == 0) {
+            float *du_row = p.du + slot * hw + head * p.width + col0;
+            if constexpr (CPL == 2) *reinterpret_cast<float2 *>(du_row) = make_float2(du[0], du[1]);
+            else du_row[0] = du[0];
+        }
+        float *wp = p.wpart + ((int64_t(tile) * p.nt * p.kw + slot) * p.heads + head) * 3 * p.s_real;
+#pragma unroll
+        for (int g = 0; g < R / 4; ++g) {  // the group's rows 4g .. 4g + 3: red = U[4], X[4], P[4]
+            float red[12];
+#pragma unroll
+            for (int i = 0; i < 12; ++i) red[i] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 4 * g + i;
+#pragma unroll
+                for (int cc = 0; cc < CPL; ++cc) {
+                    red[i] = fmaf(dm[r][cc], u[cc], red[i]);
+                    red[4 + i] = fmaf(st[r][cc], du[cc], red[4 + i]);
+                    red[8 + i] = fmaf(dm[r][cc], st[r][cc], red[8 + i]);
+                    // dh <- (dh - a du^T) * decay (role_bank_kernel.py:130-138)
+                    dm[r][cc] = (dm[r][cc] - a[r] * du[cc]) * dd[r];
+                }
+            }
+            int at;
+            bool mine;
+            const float o = reduce_columns<RG, 12>(red, lane, at, mine);
+            const int r = row0 + 4 * g + (at & 3);
+            if (mine && r < p.s_real) wp[(at >> 2) * p.s_real + r] = o;
+        }
+    };
+    // Adjoint of read e with the state st it read: dq = scale st dy, dm += scale eq dy^T.
+    auto read_back = [&](int e, int buf, const float (&st)[R][CPL]) {
+        float eq[R], dy[CPL], red[R];
+        rows_of(e, kKey, eq);
+#pragma unroll
+        for (int cc = 0; cc < CPL; ++cc) dy[cc] = s_cols[e][cc][col];
+        float *rp = p.rpart + ((int64_t(tile) * p.nt * p.kr + slot_of(e, buf, p.kr)) * p.heads + head) * p.s_real;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            red[r] = 0.f;
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc) {
+                red[r] = fmaf(st[r][cc], dy[cc], red[r]);
+                dm[r][cc] = fmaf(eq[r], dy[cc], dm[r][cc]);
+            }
+        }
+        int at;
+        bool mine;
+        const float o = reduce_columns<RG, R>(red, lane, at, mine) * p.scale;
+        if (mine && row0 + at < p.s_real) rp[row0 + at] = o;
+    };
+
+    float m0[R][CPL];
+    if (count > 0) {
+        store_meta(count - 1, load_meta(count - 1));
+        int4 prev = make_int4(0, 0, 0, 0);
+        if (count > 1) prev = load_meta(count - 2);
+        __syncthreads();
+        Staged sg;
+        issue_stage(count - 1, sg);
+        if (count > 1) store_meta(count - 2, prev);
+        __syncthreads();
+        finish_stage(count - 1, sg, m0);
+    }
+#pragma unroll 1
+    for (int c = count - 1; c >= 0; --c) {
+        __syncthreads();
+        const int buf = c & 1;
+        const int len = chunk_len(c);
+        const int4 mine = s_meta[buf][lane & (C - 1)];
+        const uint32_t wmask = uint32_t(__ballot(lane < len && mine.z == 0)) & ((1u << C) - 1);
+        const uint32_t rmask = uint32_t(__ballot(lane < len && mine.z != 0)) & ((1u << C) - 1);
+        float st[C][R][CPL];
+#pragma unroll
+        for (int e = 0; e < C; ++e) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int cc = 0; cc < CPL; ++cc) st[e][r][cc] = e ? st[e - 1][r][cc] : m0[r][cc];
+            if (e && (wmask & (1u << (e - 1)))) apply(e - 1, st[e]);
+        }
+#pragma unroll
+        for (int e = C - 1; e >= C / 2; --e) {
+            if (wmask & (1u << e)) write_back(e, buf, st[e]);
+            else if (rmask & (1u << e)) read_back(e, buf, st[e]);
+        }
+        // the next chunk's loads, in flight while the first half is differentiated
+        int4 meta2 = make_int4(0, 0, 0, 0);
+        Staged sg;
+        if (c >= 2) meta2 = load_meta(c - 2);
+        if (c >= 1) issue_stage(c - 1, sg);
+#pragma unroll
+        for (int e = C / 2 - 1; e >= 0; --e) {
+            if (wmask & (1u << e)) write_back(e, buf, st[e]);
+            else if (rmask & (1u << e)) read_back(e, buf, st[e]);
+        }
+        __syncthreads();
+        if (c >= 2) store_meta(c - 2, meta2);
+        if (c >= 1) finish_stage(c - 1, sg, m0);
+    }
+    // adjoint of the segment's initial state (FP32, per sequence)
+    if (live) {
+        const int64_t off = ((bidx * p.banks + bank) * p.heads + head) * p.s_real * p.width + col0;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc)
+                if (row0 + r < p.s_real) p.dinit[off + int64_t(row0 + r) * p.width + cc] = dm[r][cc];
+    }
+}
+
 
 template <typename T>
 struct VjpParams {
@@ -1172,14 +1266,12 @@ __global__ __launch_bounds__(256) void token_vjp_kernel(VjpParams<T> p) {
 
 struct Workspace {
     float *du, *wpart, *rpart;
-    int4 *meta;  // per-event meta of the S = 8 chunk kernel (null otherwise)
-    int *seg_order;  // the chunk kernel's segment order (null: bank order)
+    int4 *meta;      // per-event meta
+    int *seg_order;  // longest-first segment order (null: bank order)
     size_t bytes;
 };
 
 constexpr size_t align256(size_t x) { return (x + 255) / 256 * 256; }
-
-int column_lanes_per_tile(int bank_size) { return bank_size <= 8 ? 2 : 1; }
 
 int replay_interval(const bdm_backward_args &a) {
     return a.round_interval > 0 ? a.round_interval : a.snapshot_interval;
@@ -1192,6 +1284,23 @@ bool chunk_path(const bdm_backward_args &a) {
     const int64_t k = a.write_banks > a.read_banks ? a.write_banks : a.read_banks;
     return a.bank_size == 8 && replay_interval(a) == 16 && a.head_width % 2 == 0 && a.write_banks >= 1 &&
            a.read_banks >= 1 && nt * k < INT32_MAX;
+}
+
+// Row groups of the staged kernel: at most 8 rows per lane.
+int row_groups(const bdm_backward_args &a) { return a.bank_size <= 8 ? 1 : (a.bank_size <= 16 ? 2 : 4); }
+
+// Value columns of a lane: pairs in the chunk kernel and, in the staged one,
+// for banks of up to 4 rows whose heads fill more than 64 lanes (16 states of
+// 4 x 2 values then take the registers that 8 x 1 values of larger banks
+// take); loads of a pair need an even width.
+int columns_per_lane(const bdm_backward_args &a) {
+    if (chunk_path(a)) return 2;
+    return a.bank_size <= 4 && a.head_width % 2 == 0 && a.head_width > kLanes ? 2 : 1;
+}
+
+int column_tiles(const bdm_backward_args &a) {
+    const int columns = kLanes / (chunk_path(a) ? 1 : row_groups(a)) * columns_per_lane(a);
+    return (a.head_width + columns - 1) / columns;
 }
 
 // The per-token gradient kernel: one wave per head and one lane per (slot, row).
@@ -1209,27 +1318,27 @@ bool token_grad_path(const bdm_backward_args &a) {
 Workspace carve(const bdm_backward_args &a, void *base) {
     const size_t nt = size_t(a.batch) * size_t(a.time);
     const size_t hs = size_t(a.heads) * size_t(a.bank_size);
-    const int cpl = column_lanes_per_tile(a.bank_size);
-    const size_t tiles = (size_t(a.head_width) + kLanes * cpl - 1) / (kLanes * cpl);
+    const size_t tiles = size_t(column_tiles(a));
     const size_t du = align256(nt * a.write_banks * a.heads * size_t(a.head_width) * sizeof(float));
     const size_t wp = align256(tiles * 3 * nt * a.write_banks * hs * sizeof(float));
     const size_t rp = align256(tiles * nt * a.read_banks * hs * sizeof(float));
-    const size_t mt = chunk_path(a) ? align256(nt * size_t(a.write_banks + a.read_banks) * sizeof(int4)) : 0;
+    const size_t mt = align256(nt * size_t(a.write_banks + a.read_banks) * sizeof(int4));
     const int64_t nseg = int64_t(a.batch) * a.bank_count;
-    const size_t so = chunk_path(a) && order_geometry(nseg) ? align256(size_t(nseg) * sizeof(int)) : 0;
+    const size_t so = order_geometry(nseg) ? align256(size_t(nseg) * sizeof(int)) : 0;
     char *c = static_cast<char *>(base);
     Workspace w{};
     w.du = reinterpret_cast<float *>(c);
     w.wpart = reinterpret_cast<float *>(c ? c + du : nullptr);
     w.rpart = reinterpret_cast<float *>(c ? c + du + wp : nullptr);
-    w.meta = reinterpret_cast<int4 *>(c && mt ? c + du + wp + rp : nullptr);
+    w.meta = reinterpret_cast<int4 *>(c ? c + du + wp + rp : nullptr);
     w.seg_order = reinterpret_cast<int *>(c && so && order_enabled() ? c + du + wp + rp + mt : nullptr);
     w.bytes = du + wp + rp + mt + so;
     return w;
 }
 
-template <typename T, int S, int CPL, int C>
-int launch_backward(const bdm_backward_args &a, const Workspace &ws, hipStream_t stream) {
+template <typename T, bool CHUNK>
+int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kernel)(BackwardParams<T>),
+                    hipStream_t stream) {
     BackwardParams<T> p{};
     p.q = static_cast<const T *>(a.q);
     p.k = static_cast<const T *>(a.k);
@@ -1256,7 +1365,7 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, hipStream_t
     p.banks = a.bank_count;
     p.kw = a.write_banks;
     p.kr = a.read_banks;
-    p.tiles = (a.head_width + kLanes * CPL - 1) / (kLanes * CPL);
+    p.tiles = column_tiles(a);
     p.init_dtype = a.initial_dtype;
     p.snap_dtype = a.snapshot_dtype;
     p.routed_decay = a.routed_decay;
@@ -1265,36 +1374,21 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, hipStream_t
     const int64_t nseg = a.batch * a.bank_count;
     p.xcd_remap = (nseg % 8 == 0) ? 1 : 0;
     const dim3 grid(unsigned(nseg), unsigned(a.heads), unsigned(p.tiles));
-    if constexpr (S == 8 && C == 16) {
-        if (chunk_path(a)) {
-            const int64_t events = p.nt * (p.kw + p.kr);
-            const unsigned blocks = unsigned((events + 255) / 256);
-            event_meta_kernel<T><<<blocks, 256, 0, stream>>>(p.order, events, p.nt * p.kw, p.kw, p.kr, p.ww, p.rw,
-                                                            ws.meta);
-            if (int rc = check_launch("event_meta_kernel")) return rc;
-            p.meta = ws.meta;
-            if (ws.seg_order) {
-                launch_segment_order(p.cu, nseg, ws.seg_order, stream);
-                if (int rc = check_launch("segment_order_kernel")) return rc;
-                p.seg_order = ws.seg_order;
-                const void *kernel = a.snapshot_dtype == BDM_BF16
-                                         ? reinterpret_cast<const void *>(&chunk_backward_kernel<T, bf16_t>)
-                                         : reinterpret_cast<const void *>(&chunk_backward_kernel<T, float>);
-                p.order_gpr = order_groups_per_round(kernel, kLanes, nseg, int(grid.y * grid.z));
-            }
-            if (a.snapshot_dtype == BDM_BF16)
-                chunk_backward_kernel<T, bf16_t><<<grid, kLanes, 0, stream>>>(p);
-            else
-                chunk_backward_kernel<T, float><<<grid, kLanes, 0, stream>>>(p);
-            if (int rc = check_launch("chunk_backward_kernel")) return rc;
-        } else {
-            routed_backward_kernel<T, S, CPL, C><<<grid, kLanes, 0, stream>>>(p);
-            if (int rc = check_launch("routed_backward_kernel")) return rc;
-        }
-    } else {
-        routed_backward_kernel<T, S, CPL, C><<<grid, kLanes, 0, stream>>>(p);
-        if (int rc = check_launch("routed_backward_kernel")) return rc;
+    const int64_t events = p.nt * (p.kw + p.kr);
+    if ((events + 255) / 256 > int64_t(UINT32_MAX)) return fail(BDM_ERR_UNSUPPORTED, "backward: too many events");
+    event_meta_kernel<T, !CHUNK><<<unsigned((events + 255) / 256), 256, 0, stream>>>(p.order, events, p.nt * p.kw, p.kw,
+                                                                                    p.kr, p.ww, p.rw, ws.meta);
+    if (int rc = check_launch("event_meta_kernel")) return rc;
+    p.meta = ws.meta;
+    if (ws.seg_order) {
+        launch_segment_order(p.cu, nseg, ws.seg_order, stream);
+        if (int rc = check_launch("segment_order_kernel")) return rc;
+        p.seg_order = ws.seg_order;
+        p.order_gpr = order_groups_per_round(reinterpret_cast<const void *>(kernel), kLanes, nseg,
+                                             int(grid.y * grid.z));
     }
+    kernel<<<grid, kLanes, 0, stream>>>(p);
+    if (int rc = check_launch(CHUNK ? "chunk_backward_kernel" : "staged_backward_kernel")) return rc;
 
     VjpParams<T> v{};
     v.q = p.q;
@@ -1354,18 +1448,36 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, hipStream_t
     return check_launch("token_vjp_kernel");
 }
 
+template <typename T, int S, int C>
+int launch_staged(const bdm_backward_args &a, const Workspace &ws, hipStream_t stream) {
+    constexpr int RG = S <= 8 ? 1 : S / 8;  // row_groups
+    if constexpr (S == 4) {
+        if (columns_per_lane(a) == 2) return launch_backward<T, false>(a, ws, &staged_backward_kernel<T, S, 1, 2, C>, stream);
+    }
+    return launch_backward<T, false>(a, ws, &staged_backward_kernel<T, S, RG, 1, C>, stream);
+}
+
 template <typename T>
 int dispatch_backward(const bdm_backward_args &a, const Workspace &ws, hipStream_t stream) {
-    const int c = a.round_interval > 0 ? a.round_interval : a.snapshot_interval;
-    if (a.bank_size <= 8) {
-        if (c == 16) return launch_backward<T, 8, 2, 16>(a, ws, stream);
-        if (c == 8) return launch_backward<T, 8, 2, 8>(a, ws, stream);
-        if (c == 4) return launch_backward<T, 8, 2, 4>(a, ws, stream);
+    const int c = replay_interval(a);
+    if (chunk_path(a))
+        return launch_backward<T, true>(a, ws,
+                                        a.snapshot_dtype == BDM_BF16 ? &chunk_backward_kernel<T, bf16_t>
+                                                                     : &chunk_backward_kernel<T, float>,
+                                        stream);
+    if (a.bank_size <= 4) {
+        if (c == 16) return launch_staged<T, 4, 16>(a, ws, stream);
+        if (c == 8) return launch_staged<T, 4, 8>(a, ws, stream);
+        if (c == 4) return launch_staged<T, 4, 4>(a, ws, stream);
+    } else if (a.bank_size <= 8) {
+        if (c == 16) return launch_staged<T, 8, 16>(a, ws, stream);
+        if (c == 8) return launch_staged<T, 8, 8>(a, ws, stream);
+        if (c == 4) return launch_staged<T, 8, 4>(a, ws, stream);
     } else if (a.bank_size <= 16) {
-        if (c == 8) return launch_backward<T, 16, 1, 8>(a, ws, stream);
-        if (c == 4) return launch_backward<T, 16, 1, 4>(a, ws, stream);
+        if (c == 8) return launch_staged<T, 16, 8>(a, ws, stream);
+        if (c == 4) return launch_staged<T, 16, 4>(a, ws, stream);
     } else if (a.bank_size <= 32) {
-        if (c == 4) return launch_backward<T, 32, 1, 4>(a, ws, stream);
+        if (c == 4) return launch_staged<T, 32, 4>(a, ws, stream);
     }
     return fail(BDM_ERR_UNSUPPORTED, "backward: bank_size %d with replay interval %d", a.bank_size, c);
 }

@@ -134,6 +134,31 @@ def test_backward_decay_regimes(device, regime, sdt):
     check_against_oracle(device, case, 300, DECAYS[regime])
 
 
+# The staged replay kernel: padded rows (3 of 4, 5 of 8, 12 of 16, 20 of 32), one and two columns per lane, column
+# tiles with a remainder, odd widths, chunks of 16, 8 and 4 events with ragged ends, empty segments.
+STAGED_CASES = [
+    # batch, time, heads, S, v, J, K
+    (2, 21, 1, 4, 130, 6, 2), (1, 40, 2, 4, 128, 4, 4), (1, 19, 2, 3, 33, 16, 4), (2, 17, 1, 4, 129, 6, 2),
+    (1, 33, 2, 5, 66, 6, 2), (1, 37, 1, 8, 65, 4, 4), (1, 37, 2, 16, 33, 4, 4), (2, 9, 1, 12, 100, 16, 4),
+    (1, 23, 2, 32, 17, 4, 4), (1, 21, 1, 20, 48, 6, 2), (1, 1, 1, 16, 1, 6, 2),
+]
+
+
+@pytest.mark.parametrize('case', STAGED_CASES, ids=[str(i) for i in range(len(STAGED_CASES))])
+def test_staged_backward_fp32(device, case):
+    """FP32 controllers and state, held to 1e-4 as the other FP32 gradients."""
+    announce('staged backward', case)
+    check_against_oracle(device, (*case, True, torch.float32, torch.float32), 500 + case[3] + case[4])
+
+
+@pytest.mark.parametrize('s,compact', [(4, None), (4, True), (8, True), (16, None), (32, None)])
+def test_staged_backward_bf16(device, s, compact):
+    """BF16 state rounded every 16, 8 or 4 events (an odd width keeps S = 8 off the chunk kernel)."""
+    case = (2, 30, 2, s, 63 if s == 8 else 64, 8, 2, s != 16, torch.bfloat16, torch.bfloat16)
+    announce('staged backward bf16', case, compact)
+    check_against_oracle(device, case, 600 + s, compact_replay=compact)
+
+
 def test_backward_per_head_layout_matches_multi_head(device):
     """The reference's per-head call (q [B,T,S], state [J,S,v]) and the
     multi-head layout give the same gradients for one head."""
