@@ -69,52 +69,7 @@ struct BackwardParams {
     int order_gpr;
 };
 
-// The (segment, head, column tile) of this block.  In order: segments
-// remapped so each XCD takes a contiguous range, head = y, tile = z.  With
-// p.seg_order: blocks reach the XCDs round-robin in dispatch order (x
-// fastest), and the k-th block of XCD x runs item k of its range
-// (order_item): rounds of (head, tile) groups, segments longest first.
-template <typename T>
-__device__ __forceinline__ void block_item(const BackwardParams<T> &p, int &seg, int &head, int &tile) {
-    const int nseg = gridDim.x;
-    if (p.seg_order) {
-        const int64_t linear = (int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-        const int range = nseg / 8;
-        int rank, group;
-        order_item(linear / 8, range, int(gridDim.y * gridDim.z), p.order_gpr, rank, group);
-        seg = p.seg_order[int(linear % 8) * range + rank];
-        head = group / int(gridDim.z);
-        tile = group % int(gridDim.z);
-    } else {
-        seg = p.xcd_remap ? int((blockIdx.x % 8) * (nseg / 8) + blockIdx.x / 8) : int(blockIdx.x);
-        head = blockIdx.y;
-        tile = blockIdx.z;
-    }
-}
-
-__device__ __forceinline__ int64_t uniform64(int64_t x) {
-    const int lo = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(x))));
-    const int hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(x) >> 32)));
-    return int64_t((uint64_t(uint32_t(hi)) << 32) | uint64_t(uint32_t(lo)));
-}
-
 // ------------------------------------------------- S = 8, replay interval 16
-
-// Sums over lane pairs l, l + 32: lanes 0..31 return a(l) + a(l + 32), lanes
-// 32..63 return b(l - 32) + b(l) (v_permlane32_swap exchanges a's upper half
-// with b's lower half).
-__device__ __forceinline__ float half_pair_sum(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Sums over 16-lane row pairs (0, 1) and (2, 3): rows 0 and 2 return a
-// summed with the next row, rows 1 and 3 return b summed with the previous
-// row (v_permlane16_swap exchanges a's odd rows with b's even rows).
-__device__ __forceinline__ float row_pair_sum(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float x) {
@@ -180,29 +135,6 @@ __device__ __forceinline__ float reduce_scatter(const float (&x)[N], int lane) {
     asm volatile("" : "+v"(out));
     return out;
 }
-
-// Two adjacent columns of T as loaded (BF16 pairs stay packed).
-template <typename T>
-struct Pair;
-template <>
-struct Pair<bf16_t> {
-    using raw = uint32_t;
-    static __device__ __forceinline__ raw load(const bf16_t *p) { return *reinterpret_cast<const uint32_t *>(p); }
-    static __device__ __forceinline__ float lo(raw r) { return __uint_as_float(r << 16); }
-    static __device__ __forceinline__ float hi(raw r) { return __uint_as_float(r & 0xffff0000u); }
-    // bf(x*p) of both halves, packed
-    static __device__ __forceinline__ raw scaled(raw r, float pw) { return pack_bf16x2(lo(r) * pw, hi(r) * pw); }
-    static __device__ __forceinline__ raw zero() { return 0u; }
-};
-template <>
-struct Pair<float> {
-    using raw = float2;
-    static __device__ __forceinline__ raw load(const float *p) { return *reinterpret_cast<const float2 *>(p); }
-    static __device__ __forceinline__ float lo(raw r) { return r.x; }
-    static __device__ __forceinline__ float hi(raw r) { return r.y; }
-    static __device__ __forceinline__ raw scaled(raw r, float pw) { return make_float2(r.x * pw, r.y * pw); }
-    static __device__ __forceinline__ raw zero() { return make_float2(0.f, 0.f); }
-};
 
 // One entry per event of the packed order: token, route slot (PER_TOKEN: the
 // route's index within its token), is_read and the route weight (FP32 bits),
@@ -650,28 +582,6 @@ __device__ __forceinline__ float reduce_columns(const float (&x)[N], int lane, i
         return out;
     }
 }
-
-// Sum over the row groups of a column, in every lane.
-template <int RG>
-__device__ __forceinline__ float sum_row_groups(float x) {
-    if constexpr (RG >= 2) x = half_pair_sum(x, x);
-    if constexpr (RG >= 4) x = row_pair_sum(x, x);
-    return x;
-}
-
-// Columns of T as loaded: a pair (CPL = 2, one load) or one.
-template <typename T, int CPL>
-struct RawCols {
-    T x;
-    __device__ __forceinline__ void load(const T *at) { x = *at; }
-    __device__ __forceinline__ float get(int) const { return to_f32(x); }
-};
-template <typename T>
-struct RawCols<T, 2> {
-    typename Pair<T>::raw x;
-    __device__ __forceinline__ void load(const T *at) { x = Pair<T>::load(at); }
-    __device__ __forceinline__ float get(int c) const { return c ? Pair<T>::hi(x) : Pair<T>::lo(x); }
-};
 
 // Chunk replay for the shapes the S = 8 chunk kernel does not take: S in {4,
 // 8, 16, 32} padded rows (s_real of them live), replay intervals C of 4, 8 or

@@ -5,14 +5,11 @@
 // _readout (role_bank_dispatch.py:201-231); stateful variants in
 // forward_rows.py:10-194 (final state) and inference.py:70-85.
 //
-// Layout of the work (MI355X): one workgroup per (batch, bank) segment runs
-// that segment's events in packed order for every head at once.  A lane owns
-// CPL value columns of one head and keeps all S rows of those columns in
-// registers (S*CPL FP32 values), so the erase reduction over rows is in-lane
-// and a write costs three FMA-class ops per state element.  The per-event
-// metadata (token, route weight, role) is shared by all heads and staged
-// through LDS 64 events at a time; the per-token controller rows are
-// prefetched one event ahead in registers.
+// Layout of the work (MI355X): one wave runs a (batch, bank) segment's events
+// in packed order for a head (lazy_forward_kernel: two) or a tile of its
+// columns.  A lane owns a few value columns and keeps their rows in registers,
+// so a write is a handful of FMAs per column.  lazy_forward_kernel takes S = 8
+// with 16-event stages, staged_forward_kernel the rest.
 //
 // Segments of one batch are mapped to one XCD where the grid allows it
 // (segment = (blockIdx % 8) * (segments / 8) + blockIdx / 8): the 16 events of
@@ -46,8 +43,6 @@ __device__ void raw_buffer_store_x2(i32x2_t data, i32x4_t rsrc, int32_t voffset,
 
 namespace bdm {
 namespace {
-
-constexpr int kStage = 64;  // events staged per LDS batch
 
 template <typename T>
 struct ForwardParams {
@@ -106,17 +101,6 @@ struct ForwardParams {
 // Events per piece when long segments are cut (a multiple of the stage size).
 constexpr int kPieceEvents = 512;
 
-// Load `S` per-row controller values of one (token, head); rows >= s_real are 0.
-template <int S, typename E>
-__device__ __forceinline__ void load_rows(const E *p, int s_real, float (&out)[S]) {
-    if (s_real == S) {
-        load_row<S>(p, out);
-    } else {
-#pragma unroll
-        for (int r = 0; r < S; ++r) out[r] = r < s_real ? to_f32(p[r]) : 0.f;
-    }
-}
-
 template <int S, int CPL>
 __device__ __forceinline__ void load_state(const void *base, int dtype, int64_t offset, int width, int s_real,
                                            float (&h)[S][CPL]) {
@@ -148,132 +132,212 @@ __device__ __forceinline__ void store_state(void *base, int dtype, int64_t offse
     }
 }
 
-// Registers of one event's per-lane operands (one head).
-template <int S, int CPL>
-struct EventOperands {
-    float key[S];   // k for a write, q for a read
-    float gate[S];  // g
-    float erase[S]; // b
-    float value[CPL];
-    float wgate[CPL];
-};
+// Bank sizes and intervals the S = 8 lazy kernel does not take: S in {4, 8,
+// 16, 32} padded rows (s_real of them live), any rounding or snapshot
+// interval, any width.  One wave per (segment, head, tile of columns); a lane
+// owns CPL value columns and R = S / RG rows (at most 8): RG groups of 64 / RG
+// lanes share a column's rows.
+//  * Stages of 16 events.  Lane e of the wave decodes event e; the loads of the
+//    next stage (columns into registers, row operands) go out before this
+//    stage's events run, the packed order one stage earlier still, so no event
+//    waits for a load.
+//  * The row operands (k, exp(g p), bf(b p) k, or bf(q r)) are formed once per
+//    event, spread over the lanes, and read back from LDS by broadcast.
+// Bound: instruction issue of the event loop.  Before it, one kernel formed the
+// row operands in every lane from loads one event ahead: 273 -> 49 us at 16,384
+// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 433 -> 104 us at
+// 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events; 32 columns
+// per wave make 1,024 waves of them, which the chip holds at once).
+template <typename T, int S, int RG, int CPL>
+__global__ __launch_bounds__(64) void staged_forward_kernel(ForwardParams<T> p) {
+    constexpr int E = 16;  // events per stage
+    constexpr int R = S / RG, kCols = kWave / RG, NR = E * S / kWave;
+    constexpr int kKey = 0, kDecay = S, kErase = 2 * S;
+    __shared__ __align__(16) float s_rows[E][3 * S + 4];
+    struct Meta {  // of event lane % 16 of a stage
+        int token, route, read;
+        float weight;
+    };
+    struct Staged {
+        RawCols<T, CPL> a[E], b[E];  // v and w of a write
+        T x[NR], bb[NR];             // write: k, b; read: q
+        float g[NR];
+    };
 
-template <typename T, int S, int CPL>
-__device__ __forceinline__ void fetch_event(const ForwardParams<T> &p, int64_t token, bool is_read, int head,
-                                            int col0, EventOperands<S, CPL> &ev) {
-    const int64_t row = token * p.heads + head;
-    if (is_read) {
-        load_rows<S>(p.q + row * p.s_real, p.s_real, ev.key);
-    } else {
-        load_rows<S>(p.k + row * p.s_real, p.s_real, ev.key);
-        load_rows<S>(p.g + row * p.s_real, p.s_real, ev.gate);
-        load_rows<S>(p.b + row * p.s_real, p.s_real, ev.erase);
-        load_row<CPL>(p.v + row * p.width + col0, ev.value);
-        load_row<CPL>(p.w + row * p.width + col0, ev.wgate);
-    }
-}
-
-template <typename T, int S, int CPL>
-__global__ __launch_bounds__(256) void routed_forward_kernel(ForwardParams<T> p) {
-    __shared__ int64_t s_token[kStage];
-    __shared__ int64_t s_slot[kStage];  // read: original read slot; write: -1
-    __shared__ float s_weight[kStage];
-
-    const int nseg = gridDim.x;
-    const int seg = p.xcd_remap ? int((blockIdx.x % 8) * (nseg / 8) + blockIdx.x / 8) : int(blockIdx.x);
+    int seg, head, tile;
+    block_item(p, seg, head, tile);
     const int bank = seg % p.banks;
     const int64_t bidx = seg / p.banks;
-    const int head = blockIdx.y * p.heads_per_block + int(threadIdx.x) / p.lanes_per_head;
-    const bool active = int(threadIdx.x) < p.heads_per_block * p.lanes_per_head && head < p.heads;
-    const int col0 = (int(threadIdx.x) % p.lanes_per_head) * CPL;
+    const int lane = threadIdx.x;
+    const int row0 = lane / kCols * R;
+    const int col0 = (tile * kCols + lane % kCols) * CPL;
+    const bool live = col0 < p.width;
+    const int colc = live ? col0 : p.width - CPL;  // lanes past the width load valid columns and store nothing
     const int64_t start = p.cu[seg], end = p.cu[seg + 1];
-    // event and route indices fit in 32 bits (checked by the launcher)
-    const int write_events = int(p.nt * p.kw);
-    const int events = int(p.nt * (p.kw + p.kr));
+    const int count = int((end - start + E - 1) / E);
+    const int64_t hw = int64_t(p.heads) * p.width;
+    const int64_t write_events = p.nt * p.kw, events = p.nt * (int64_t(p.kw) + p.kr);
+    const int lane_col = head * p.width + colc;
     const bool rounding = p.round_interval > 0;
+    const int64_t state_offset = (int64_t(bank) * p.heads + head) * p.s_real * p.width + col0;
 
-    float h[S][CPL];
-    const int64_t state_offset = ((int64_t(bank) * p.heads + head) * p.s_real) * p.width + col0;
-    if (active) {
-        load_state<S, CPL>(p.initial, p.init_dtype, bidx * p.init_bstride + state_offset, p.width, p.s_real, h);
-        if (rounding) {
+    auto load_order = [&](int s) {
+        const int64_t at = start + int64_t(s) * E + (lane & (E - 1));
+        return p.order[at < end ? at : end - 1];
+    };
+    auto decode = [&](int64_t o) {
+        Meta m;
+        o = o < 0 ? 0 : (o >= events ? events - 1 : o);
+        m.read = o >= write_events;
+        const int64_t route = m.read ? o - write_events : o;
+        m.token = int(p.k_shift >= 0 ? route >> p.k_shift : route / (m.read ? p.kr : p.kw));
+        m.route = int(route - int64_t(m.token) * (m.read ? p.kr : p.kw));
+        m.weight = to_f32(m.read ? p.rw[route] : p.ww[route]);
+        return m;
+    };
+    auto issue_stage = [&](const Meta &m, Staged &sg) {
 #pragma unroll
-            for (int r = 0; r < S; ++r)
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) h[r][c] = round_bf16(h[r][c]);
+        for (int e = 0; e < E; ++e) {
+            const int64_t at = int64_t(__builtin_amdgcn_readlane(m.token, e)) * hw + lane_col;
+            sg.a[e].load(p.v + at);
+            sg.b[e].load(p.w + at);
         }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int idx = lane + i * kWave, e = idx / S, r = idx % S;
+            const int64_t at = (int64_t(__shfl(m.token, e)) * p.heads + head) * p.s_real + (r < p.s_real ? r : 0);
+            sg.x[i] = (__shfl(m.read, e) ? p.q : p.k)[at];
+            sg.bb[i] = p.b[at];
+            sg.g[i] = p.g[at];
+        }
+    };
+    auto finish_stage = [&](const Meta &m, const Staged &sg) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int idx = lane + i * kWave, e = idx / S, r = idx % S;
+            const float pw = __shfl(m.weight, e);
+            const float x = r < p.s_real ? to_f32(sg.x[i]) : 0.f;
+            // prepare_write_rows of row r; a read's key is bf(q r)
+            s_rows[e][kKey + r] = __shfl(m.read, e) ? round_to<T>(x * pw) : x;
+            s_rows[e][kDecay + r] = r < p.s_real ? __expf(p.routed_decay ? sg.g[i] * pw : sg.g[i]) : 0.f;
+            s_rows[e][kErase + r] = round_to<T>(to_f32(sg.bb[i]) * pw) * x;
+        }
+    };
+    auto rows_of = [&](int e, int at, float (&x)[R]) {
+        const float4 *row = reinterpret_cast<const float4 *>(&s_rows[e][at + row0]);
+#pragma unroll
+        for (int i = 0; i < R / 4; ++i) {
+            const float4 f = row[i];
+            x[4 * i] = f.x, x[4 * i + 1] = f.y, x[4 * i + 2] = f.z, x[4 * i + 3] = f.w;
+        }
+    };
+    auto store_rows = [&](void *base, int dtype, int64_t offset, const float (&m)[R][CPL]) {
+        if (!live) return;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (row0 + r < p.s_real) {
+                const int64_t at = offset + int64_t(row0 + r) * p.width;
+                if (dtype == BDM_BF16) store_cols(static_cast<bf16_t *>(base) + at, m[r]);
+                else store_cols(static_cast<float *>(base) + at, m[r]);
+            }
+        }
+    };
+
+    float h[R][CPL];
+    {
+        const int64_t offset = bidx * p.init_bstride + state_offset - col0 + colc;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                const int64_t at = offset + int64_t(row0 + r < p.s_real ? row0 + r : 0) * p.width + c;
+                const float x = p.init_dtype == BDM_BF16 ? to_f32(static_cast<const bf16_t *>(p.initial)[at])
+                                                         : static_cast<const float *>(p.initial)[at];
+                h[r][c] = row0 + r < p.s_real ? (rounding ? round_bf16(x) : x) : 0.f;
+            }
     }
-
-    for (int64_t base = start; base < end; base += kStage) {
-        const int n = int(min(int64_t(kStage), end - base));
-        __syncthreads();
-        if (int(threadIdx.x) < n) {
-            int64_t o = p.order[base + threadIdx.x];
-            o = o < 0 ? 0 : (o >= events ? events - 1 : o);
-            const bool rd = o >= write_events;
-            const int64_t route = rd ? o - write_events : o;
-            s_token[threadIdx.x] = rd ? route / p.kr : route / p.kw;
-            s_slot[threadIdx.x] = rd ? route : -1;  // a read's row of zbuf: its route
-            s_weight[threadIdx.x] = rd ? to_f32(p.rw[route]) : to_f32(p.ww[route]);
-        }
-        __syncthreads();
-        if (!active) continue;
-
-        EventOperands<S, CPL> cur, nxt;
-        fetch_event<T, S, CPL>(p, s_token[0], s_slot[0] >= 0, head, col0, cur);
-        for (int i = 0; i < n; ++i) {
-            const int64_t slot = s_slot[i];
-            const float pw = s_weight[i];
-            if (i + 1 < n) fetch_event<T, S, CPL>(p, s_token[i + 1], s_slot[i + 1] >= 0, head, col0, nxt);
-            const int64_t offset = base + i - start;
-            if (p.snap_interval > 0 && offset > 0 && offset % p.snap_interval == 0) {
-                if (rounding) {
+    if (count > 0) {
+        Meta meta = decode(load_order(0));
+        int64_t ahead = load_order(count > 1 ? 1 : 0);
+        Staged cur;
+        issue_stage(meta, cur);
+#pragma unroll 1
+        for (int s = 0; s < count; ++s) {
+            const int64_t base = start + int64_t(s) * E;
+            const int len = int(min(int64_t(E), end - base));
+            __syncthreads();
+            finish_stage(meta, cur);
+            __syncthreads();
+            const Meta next = decode(ahead);
+            Staged nxt;
+            issue_stage(next, nxt);
+            ahead = load_order(s + 2 < count ? s + 2 : count - 1);
+            const bool valid = lane < len;
+            const uint32_t wmask = uint32_t(__ballot(valid && !meta.read)), rmask = uint32_t(__ballot(valid && meta.read));
+            // events that start a rounding / snapshot interval of the segment
+            const int64_t mine = base - start + lane;
+            const uint32_t bmask = p.snap_interval > 0 ? uint32_t(__ballot(valid && mine > 0 && mine % p.snap_interval == 0)) : 0u;
 #pragma unroll
-                    for (int r = 0; r < S; ++r)
+            for (int e = 0; e < E; ++e) {
+                if (bmask & (1u << e)) {
+                    if (rounding) {
 #pragma unroll
-                        for (int c = 0; c < CPL; ++c) h[r][c] = round_bf16(h[r][c]);
+                        for (int r = 0; r < R; ++r)
+#pragma unroll
+                            for (int c = 0; c < CPL; ++c) h[r][c] = round_bf16(h[r][c]);
+                    }
+                    // Snapshot of the state before event base+e, the start of a replay chunk
+                    // (role_bank_kernel.py:59-66).  Boundaries of one segment are snap_interval
+                    // apart and segments are disjoint, so slot = position / interval - 1 is
+                    // unique per boundary.
+                    if (p.snap)
+                        store_rows(p.snap, p.snap_dtype,
+                                   (((base + e) / p.snap_interval - 1) * p.heads + head) * p.s_real * p.width + col0, h);
                 }
-                // Snapshot of the state before event base+i, the start of a
-                // replay chunk (role_bank_kernel.py:59-66).  Boundaries of one
-                // segment are snap_interval apart and segments are disjoint,
-                // so slot = position / interval - 1 is unique per boundary.
-                if (p.snap) {
-                    const int64_t slot = (base + i) / p.snap_interval - 1;
-                    store_state<S, CPL>(p.snap, p.snap_dtype,
-                                        ((slot * p.heads + head) * p.s_real) * p.width + col0, p.width,
-                                        p.s_real, h);
+                if (wmask & (1u << e)) {
+                    // hd = exp(eg) M ; u = bf(w p) v - (bf(b p) k)^T hd ; M = hd + k u^T
+                    float kk[R], dd[R], a[R];
+                    rows_of(e, kKey, kk);
+                    rows_of(e, kDecay, dd);
+                    rows_of(e, kErase, a);
+                    const float pw = __uint_as_float(
+                        __builtin_amdgcn_readlane(__float_as_uint(meta.weight), e));
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) {
+                        float erase = 0.f;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            h[r][c] *= dd[r];
+                            erase = fmaf(a[r], h[r][c], erase);
+                        }
+                        const float u = fmaf(round_to<T>(cur.b[e].get(c) * pw), cur.a[e].get(c),
+                                             -sum_row_groups<RG>(erase));
+#pragma unroll
+                        for (int r = 0; r < R; ++r) h[r][c] = fmaf(kk[r], u, h[r][c]);
+                    }
+                } else if (rmask & (1u << e)) {
+                    // z = scale * bf(q r)^T M, stored in the value dtype
+                    float qr[R], z[CPL];
+                    rows_of(e, kKey, qr);
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) {
+                        float acc = 0.f;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) acc = fmaf(qr[r], h[r][c], acc);
+                        z[c] = sum_row_groups<RG>(acc) * p.scale;
+                    }
+                    const int64_t slot = int64_t(__builtin_amdgcn_readlane(meta.token, e)) * p.kr +
+                                         __builtin_amdgcn_readlane(meta.route, e);
+                    if (live && row0 == 0) store_cols(p.zbuf + slot * hw + head * p.width + col0, z);
                 }
             }
-            if (slot < 0) {
-                // write: hd = exp(eg) M ; u = bf(w p) v - (bf(b p) k)^T hd ; M = hd + k u^T
-                WriteRows<S> rows;
-                prepare_write_rows<T, S>(cur.key, cur.gate, cur.erase, pw, p.routed_decay, rows);
-                float ew[CPL];
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) ew[c] = round_to<T>(cur.wgate[c] * pw);
-                apply_write<S, CPL>(h, rows, ew, cur.value);
-            } else {
-                // read: z = scale * bf(q r)^T M, stored in the value dtype
-                float qr[S];
-#pragma unroll
-                for (int r = 0; r < S; ++r) qr[r] = round_to<T>(cur.key[r] * pw);
-                float z[CPL];
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) {
-                    float acc = 0.f;
-#pragma unroll
-                    for (int r = 0; r < S; ++r) acc = fmaf(qr[r], h[r][c], acc);
-                    z[c] = acc * p.scale;
-                }
-                store_row<CPL>(p.zbuf + (slot * p.heads + head) * p.width + col0, z);
-            }
+            meta = next;
             cur = nxt;
         }
     }
-    if (active && p.final_state) {
-        const int64_t final_offset = bidx * (int64_t(p.banks) * p.heads * p.s_real * p.width) + state_offset;
-        store_state<S, CPL>(p.final_state, p.final_dtype, final_offset, p.width, p.s_real, h);
-    }
+    if (p.final_state)
+        store_rows(p.final_state, p.final_dtype,
+                   bidx * (int64_t(p.banks) * p.heads * p.s_real * p.width) + state_offset, h);
 }
 
 // ----------------------------------------------------------------------------
@@ -1990,11 +2054,9 @@ int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void 
     return record_phase(a, 2, stream);
 }
 
-template <typename T, int S, int CPL, bool kLazy = false>
-int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, hipStream_t stream) {
-    const int split = kLazy ? lazy_split(a) : 1;
-    if (a.head_width / split / CPL > 256)
-        return fail(BDM_ERR_UNSUPPORTED, "forward: head_width %d needs more than 256 lanes", a.head_width);
+// Operands and geometry of a forward whose heads run as `split` column parts each.
+template <typename T>
+ForwardParams<T> forward_params(const bdm_forward_args &a, T *zbuf, int split) {
     ForwardParams<T> p{};
     p.q = static_cast<const T *>(a.q);
     p.k = static_cast<const T *>(a.k);
@@ -2024,12 +2086,6 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
     p.k_shift = -1;
     for (int sh = 0; sh < 8; ++sh)
         if (a.write_banks == (1 << sh) && a.read_banks == (1 << sh)) p.k_shift = sh;
-    p.lanes_per_head = p.width / CPL;
-    p.heads_per_block = 256 / p.lanes_per_head;
-    // lazy kernel: 2 heads per one-wave workgroup when a head has 32 lanes, else 8 per 256 threads
-    const int lazy_hb = p.lanes_per_head == 32 ? 2 : 8;
-    if (kLazy && p.heads_per_block > lazy_hb) p.heads_per_block = lazy_hb;
-    if (p.heads_per_block > p.heads) p.heads_per_block = p.heads;
     p.round_interval = a.round_interval;
     p.routed_decay = a.routed_decay;
     p.snap = a.snapshots;
@@ -2040,11 +2096,55 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
     p.scale = a.scale;
     const int64_t nseg = a.batch * a.bank_count;
     p.xcd_remap = (nseg % 8 == 0) ? 1 : 0;
-    const int threads = ((p.heads_per_block * p.lanes_per_head + kWave - 1) / kWave) * kWave;
-    const dim3 grid(unsigned(nseg), unsigned((p.heads + p.heads_per_block - 1) / p.heads_per_block));
     p.nseg = int(nseg);
+    return p;
+}
+
+// Columns that a head's width counts in where it is limited: at most 256
+// units of 8, 4 or 2 columns for banks of up to 8, 16 and 32 rows where the
+// width and the state's batch stride are multiples of it, else single columns.
+int width_unit(const bdm_forward_args &a) {
+    const int unit = a.bank_size <= 8 ? 8 : (a.bank_size <= 16 ? 4 : 2);
+    return a.initial_batch_stride % 8 == 0 && a.head_width % unit == 0 ? unit : 1;
+}
+
+// Any bank size, width and interval on staged_forward_kernel.
+template <typename T, int S, int RG, int CPL>
+int launch_staged_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, hipStream_t stream) {
+    ForwardParams<T> p = forward_params(a, zbuf, 1);
+    if (a.batch * a.time > int64_t(INT32_MAX)) return fail(BDM_ERR_UNSUPPORTED, "forward: more than 2^31 tokens");
+    if (a.head_width > 256 * width_unit(a))
+        return fail(BDM_ERR_UNSUPPORTED, "forward: head_width %d needs more than 256 lanes", a.head_width);
+    const int columns = kWave / RG * CPL;
+    const dim3 grid(unsigned(p.nseg), unsigned(a.heads), unsigned((a.head_width + columns - 1) / columns));
+    if (a.heads > 65535 || grid.z > 65535) return fail(BDM_ERR_UNSUPPORTED, "forward: grid too large");
     if (int rc = record_phase(a, 0, stream)) return rc;
-    if constexpr (kLazy) {
+    if (pb.seg_order) {
+        if (!pb.order_given) {
+            launch_segment_order(a.cu_seqlens, p.nseg, pb.seg_order, stream);
+            if (int rc = check_launch("segment_order_kernel")) return rc;
+        }
+        p.seg_order = pb.seg_order;
+        p.order_gpr = order_groups_per_round(reinterpret_cast<const void *>(&staged_forward_kernel<T, S, RG, CPL>),
+                                             kWave, p.nseg, int(grid.y * grid.z));
+    }
+    staged_forward_kernel<T, S, RG, CPL><<<grid, kWave, 0, stream>>>(p);
+    if (int rc = check_launch("staged_forward_kernel")) return rc;
+    return launch_combine<T>(a, zbuf, stream);
+}
+
+// S = 8 with 16-event stages on lazy_forward_kernel.
+template <typename T, int CPL>
+int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, hipStream_t stream) {
+    ForwardParams<T> p = forward_params(a, zbuf, lazy_split(a));
+    const int64_t nseg = p.nseg;
+    p.lanes_per_head = p.width / CPL;
+    // 2 heads per one-wave workgroup when a head has 32 lanes, else 8 per 256 threads
+    const int lazy_hb = p.lanes_per_head == 32 ? 2 : 8;
+    p.heads_per_block = std::min({256 / p.lanes_per_head, lazy_hb, p.heads});
+    const dim3 grid(unsigned(nseg), unsigned((p.heads + p.heads_per_block - 1) / p.heads_per_block));
+    if (int rc = record_phase(a, 0, stream)) return rc;
+    {
         // the prep role needs one lane per (event, head, half): 32 per head
         const int lthreads = lazy_hb == 2 ? 64 : 256;
         if (pb.max_pieces > 0) {
@@ -2113,9 +2213,6 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             if (int rc = launch_mode0<T>(kernel, grid, lthreads, p, stream)) return rc;
         }
         if (int rc = check_launch("lazy_forward_kernel")) return rc;
-    } else {
-        routed_forward_kernel<T, S, CPL><<<grid, threads, 0, stream>>>(p);
-        if (int rc = check_launch("routed_forward_kernel")) return rc;
     }
 
     return launch_combine<T>(a, zbuf, stream);
@@ -2169,10 +2266,11 @@ int64_t stage_slots(const bdm_forward_args &a) {
     return events / kLazyStage + a.batch * a.bank_count + 1;
 }
 
-// Whether the lazy kernel takes each XCD range's segments longest first
-// (segment_order_kernel; MODE 0, and MODE 1's segment blocks): ranges that
-// the XCD remap forms, at most kOrderMaxRange segments each.
-bool order_path(const bdm_forward_args &a) { return lazy_path(a) && order_geometry(a.batch * a.bank_count); }
+// Whether the recurrence takes each XCD range's segments longest first
+// (segment_order_kernel; the lazy kernel's MODE 0 and MODE 1's segment blocks,
+// and the staged kernel): ranges that the XCD remap forms, at most
+// kOrderMaxRange segments each.
+bool order_path(const bdm_forward_args &a) { return order_geometry(a.batch * a.bank_count); }
 
 // BDM_FORWARD_KERNEL=mfma selects the matrix-core recurrence where it
 // applies; the vector-ALU kernel is the default (both are complete
@@ -2229,23 +2327,20 @@ int launch_chunked(const bdm_forward_args &a, bf16_t *zbuf, hipStream_t stream) 
 
 template <typename T>
 int dispatch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, hipStream_t stream) {
-    // Vector row loads need 16-byte aligned rows: aligned bases, and a state
-    // batch stride that keeps them aligned.
-    const bool vec = a.initial_batch_stride % 8 == 0;
     if constexpr (std::is_same<T, bf16_t>::value) {
         if (chunk_path(a) && chunk_enabled()) return launch_chunked(a, zbuf, stream);
     }
-    if (a.bank_size <= 8) {
-        if (lazy_path(a)) return launch_forward<T, 8, 4, true>(a, zbuf, pb, stream);
-        if (vec && a.head_width % 8 == 0) return launch_forward<T, 8, 8>(a, zbuf, pb, stream);
-        return launch_forward<T, 8, 1>(a, zbuf, pb, stream);
+    if (lazy_path(a)) return launch_forward<T, 4>(a, zbuf, pb, stream);
+    // column pairs of BF16 where a head fills more than one wave of single columns: loads of 4 bytes need an even width
+    const bool pairs = sizeof(T) == 2 && a.head_width % 2 == 0 && a.head_width > kWave;
+    if constexpr (sizeof(T) == 2) {
+        if (pairs && a.bank_size <= 4) return launch_staged_forward<T, 4, 1, 2>(a, zbuf, pb, stream);
+        if (pairs && a.bank_size <= 8) return launch_staged_forward<T, 8, 1, 2>(a, zbuf, pb, stream);
     }
-    if (a.bank_size <= 16) {
-        if (vec && a.head_width % 4 == 0) return launch_forward<T, 16, 4>(a, zbuf, pb, stream);
-        return launch_forward<T, 16, 1>(a, zbuf, pb, stream);
-    }
-    if (vec && a.head_width % 2 == 0) return launch_forward<T, 32, 2>(a, zbuf, pb, stream);
-    return launch_forward<T, 32, 1>(a, zbuf, pb, stream);
+    if (a.bank_size <= 4) return launch_staged_forward<T, 4, 1, 1>(a, zbuf, pb, stream);
+    if (a.bank_size <= 8) return launch_staged_forward<T, 8, 1, 1>(a, zbuf, pb, stream);
+    if (a.bank_size <= 16) return launch_staged_forward<T, 16, 2, 1>(a, zbuf, pb, stream);
+    return launch_staged_forward<T, 32, 4, 1>(a, zbuf, pb, stream);
 }
 
 size_t elem_size(int dtype) { return dtype == BDM_BF16 ? 2 : 4; }

@@ -90,6 +90,29 @@ __device__ __forceinline__ void order_item(int64_t k, int range, int groups, int
     group = round * gpr + w % in_round;
 }
 
+// The (segment, head, column tile) of this block.  In order: segments
+// remapped so each XCD takes a contiguous range, head = y, tile = z.  With
+// p.seg_order: blocks reach the XCDs round-robin in dispatch order (x
+// fastest), and the k-th block of XCD x runs item k of its range
+// (order_item): rounds of (head, tile) groups, segments longest first.
+template <typename P>
+__device__ __forceinline__ void block_item(const P &p, int &seg, int &head, int &tile) {
+    const int nseg = gridDim.x;
+    if (p.seg_order) {
+        const int64_t linear = (int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        const int range = nseg / 8;
+        int rank, group;
+        order_item(linear / 8, range, int(gridDim.y * gridDim.z), p.order_gpr, rank, group);
+        seg = p.seg_order[int(linear % 8) * range + rank];
+        head = group / int(gridDim.z);
+        tile = group % int(gridDim.z);
+    } else {
+        seg = p.xcd_remap ? int((blockIdx.x % 8) * (nseg / 8) + blockIdx.x / 8) : int(blockIdx.x);
+        head = blockIdx.y;
+        tile = blockIdx.z;
+    }
+}
+
 // Blocks of `kernel` (block_threads each) that one XCD holds at once: its
 // CUs times the resident blocks per CU.  The occupancy query costs ~10 us of
 // host time, on the path between two launches, so each (kernel, threads,

@@ -206,6 +206,45 @@ def test_forward_matches_oracle(device, case):
     assert rel_err(final, ref_final) < TOL, rel_err(final, ref_final)
 
 
+# The staged kernel: padded rows (3 of 4, 5 of 8, 12 of 16, 20 of 32), one and two columns per lane, column tiles with
+# a remainder, odd widths, KW other than KR, segments of less than a stage, of several and empty ones.
+STAGED_CASES = [
+    # batch, time, heads, S, v, J, KW, KR
+    (1, 60, 1, 4, 128, 6, 2, 3), (2, 17, 2, 3, 33, 16, 4, 4), (1, 40, 1, 4, 130, 4, 4, 4), (2, 21, 1, 5, 66, 12, 3, 1),
+    (1, 50, 2, 8, 65, 4, 2, 2), (1, 45, 2, 16, 33, 6, 2, 4), (2, 9, 1, 12, 100, 16, 4, 4), (1, 30, 1, 32, 17, 4, 4, 4),
+    (1, 1, 1, 20, 1, 6, 1, 1),
+]
+
+
+@pytest.mark.parametrize('case', STAGED_CASES, ids=[str(i) for i in range(len(STAGED_CASES))])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
+def test_staged_forward_matches_oracle(device, case, dtype):
+    """FP32 within 2e-5 of the oracle (sums over at most 32 rows and 100 events, in another order); BF16 with the
+    state rounded every 5 events (no divisor of the kernel's 16-event stages) within the bound of the other cases."""
+    from bdm_amd import ops
+    batch, time, heads, s, v, j, kw, kr = case
+    gen = torch.Generator().manual_seed(700 + s + v)
+    wi, ri = (torch.stack([torch.randperm(j, generator=gen)[:k] for _ in range(batch * time)]).reshape(batch, time, k)
+              for k in (kw, kr))
+    ww, rw = (torch.rand(batch, time, k, generator=gen).to(dtype) for k in (kw, kr))
+    q, k, v_, g, b, w = controllers(batch, time, heads, s, v, gen, dtype)
+    state = initial_state(j, heads, s, v, gen)
+    interval = 5 if dtype == torch.bfloat16 else 0
+    dev = [t.to(device) for t in (q, k, v_, g, b, w, wi, ww, ri, rw, state)]
+    announce('staged forward', case, dtype)
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    final = torch.empty(batch, j, heads, s, v, device=device, dtype=torch.float32)
+    y = ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
+                           round_interval=interval, final_state=final)
+    torch.cuda.synchronize()
+    state_dtype = torch.bfloat16 if interval else torch.float32
+    ref, ref_final = oracle_reads(q, k, v_, g, b, w, wi, ww, ri, rw, state, j, routed_decay=True,
+                                  state_dtype=state_dtype, interval=interval or 16, return_final=True)
+    tol = TOL if dtype == torch.bfloat16 else 2e-5
+    assert rel_err(y, ref) < tol, rel_err(y, ref)
+    assert rel_err(final, ref_final) < tol, rel_err(final, ref_final)
+
+
 @pytest.mark.parametrize('state_dtype', [torch.bfloat16, torch.float32])
 def test_forward_long_read_runs_match_oracle(device, state_dtype):
     """Segments whose events are runs of more than one 16-event stage of reads
