@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
     constexpr int NR = (C * S + kLanes - 1) / kLanes;  // (event, row) operands per lane
     constexpr int kKey = 0, kDecay = S, kErase = 2 * S, kStride = 3 * S + 4;
     struct Staged {
-        RawCols<T, CPL> a[C], b[C];  // write: v, w; read: dy, dy
+        LaneCols<T, CPL> a[C], b[C];  // write: v, w; read: dy, dy
         T x[NR], bb[NR];             // write: k, b; read: q
         float g[NR];
         uint32_t m0[R][CPL];  // start state (BF16 or FP32 bits)

@@ -26,6 +26,7 @@
 #include <mutex>
 #include <cstring>
 #include <type_traits>
+#include <utility>
 
 #include "bdm_common.h"
 #include "recurrence_ops.h"
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64) void staged_forward_kernel(ForwardParams<T> p) 
         float weight;
     };
     struct Staged {
-        RawCols<T, CPL> a[E], b[E];  // v and w of a write
+        LaneCols<T, CPL> a[E], b[E];  // v and w of a write
         T x[NR], bb[NR];             // write: k, b; read: q
         float g[NR];
     };
@@ -678,7 +679,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
         }
         group += p.group_base;
         // the stage path runs the long segments (the whole workgroup leaves together)
-        if (p.skip_long && p.cu[seg + 1] - p.cu[seg] > kPieceEvents) return;
+        if (p.skip_long && p.cu[seg + 1] - p.cu[seg] > p.skip_long) return;
     } else if constexpr (MODE == 3) {
         is_piece = true;  // every piece of every long segment, one per block
     } else if constexpr (MODE == 1) {
@@ -1243,6 +1244,382 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
     }
 }
 
+// ----------------------------------------------------------------------------
+// Long segments under MODE 0's policy: a chain of thousands of events whose
+// length no other wave can share, so it is the time per event of one wave that
+// counts, not the instructions.  Waves of a workgroup divide a segment's work
+// on one virtual head by kind, a stage of 16 events apart, a barrier per stage:
+//  * a consumer holds the state of 64 columns, one per lane, and does nothing
+//    but the events, without branches: a read is a write with u = 0 (its z is
+//    the write's row sum), so both are the same 8 + 8 FMAs (chain_event);
+//  * one producer forms the row operands, as lazy_forward_kernel's prep does;
+//  * a producer per 64 columns loads v, w a stage further ahead, two events per
+//    load (lanes 0..31 the column pairs of event 2i, lanes 32..63 of 2i + 1),
+//    leaves x = bf(w p) v in LDS and stores the z of the stage before.
+// The arithmetic is lazy_forward_kernel's, in its order, apart from the rounding
+// of x + sum.  Bound: the consumer's issue and one barrier, ~75 ns per event
+// (lazy_forward_kernel: 211).  Measured on the way there (1,000-stage chain, one
+// launch alone): row operands read from LDS at each event 2,780 us (each event
+// waits for LDS), by row_newbcast 2,240; the preparation moved to producers
+// 1,718, their event values by DPP instead of bpermute 1,364, and the row
+// operands' producer apart 1,214.
+template <int NC>
+struct ChainLds {  // [stage parity]
+    float rows[2][kLazyStage][20];  // per event: 8 coefficients, 8 betas, pad
+    float decay[2][kLazyStage][8];  // eager stages
+    float fold[2][8];
+    float x[2][NC][kLazyStage][kWave];
+    float z[2][NC][kLazyStage][kWave];
+    uint32_t writes[2];  // bit e: event e writes
+    int eager[2];
+};
+
+// Event E of a stage on one column's state: z = coef^T h, then for a write
+// (mask all ones) u = z + x, h += beta u; a read's mask is 0, so that its u is 0
+// also where the state holds infinities.  Lane 16 q + e of coef, beta and
+// decay holds event e's row operand (in every row q), which row_newbcast:E
+// hands to the lanes of its row: no LDS read or scalar register per operand.
+// One asm block: the compiler does not fold a DPP source into an FMA.  The
+// s_nop gives the 2 wait states that a DPP read of a VGPR needs should the
+// compiler have moved an operand just before; inside the block no DPP source
+// is written.
+#define BDM_BCAST " row_newbcast:%c[e] row_mask:0xf bank_mask:0xf\n\t"
+template <int E, bool EAGER>
+__device__ __forceinline__ void chain_event(float (&h)[8], const float (&coef)[8], const float (&beta)[8],
+                                            const float (&decay)[8], float x, uint32_t mask, float &z) {
+    if constexpr (EAGER) {
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %[h0], %[d0], %[h0]" BDM_BCAST "v_mul_f32_dpp %[h1], %[d1], %[h1]" BDM_BCAST
+            "v_mul_f32_dpp %[h2], %[d2], %[h2]" BDM_BCAST "v_mul_f32_dpp %[h3], %[d3], %[h3]" BDM_BCAST
+            "v_mul_f32_dpp %[h4], %[d4], %[h4]" BDM_BCAST "v_mul_f32_dpp %[h5], %[d5], %[h5]" BDM_BCAST
+            "v_mul_f32_dpp %[h6], %[d6], %[h6]" BDM_BCAST "v_mul_f32_dpp %[h7], %[d7], %[h7]" BDM_BCAST
+            : [h0] "+v"(h[0]), [h1] "+v"(h[1]), [h2] "+v"(h[2]), [h3] "+v"(h[3]), [h4] "+v"(h[4]), [h5] "+v"(h[5]),
+              [h6] "+v"(h[6]), [h7] "+v"(h[7])
+            : [d0] "v"(decay[0]), [d1] "v"(decay[1]), [d2] "v"(decay[2]), [d3] "v"(decay[3]), [d4] "v"(decay[4]),
+              [d5] "v"(decay[5]), [d6] "v"(decay[6]), [d7] "v"(decay[7]), [e] "i"(E));
+    }
+    float u;
+    asm("s_nop 1\n\t"
+        "v_mul_f32_dpp %[z], %[c0], %[h0]" BDM_BCAST "v_fmac_f32_dpp %[z], %[c1], %[h1]" BDM_BCAST
+        "v_fmac_f32_dpp %[z], %[c2], %[h2]" BDM_BCAST "v_fmac_f32_dpp %[z], %[c3], %[h3]" BDM_BCAST
+        "v_fmac_f32_dpp %[z], %[c4], %[h4]" BDM_BCAST "v_fmac_f32_dpp %[z], %[c5], %[h5]" BDM_BCAST
+        "v_fmac_f32_dpp %[z], %[c6], %[h6]" BDM_BCAST "v_fmac_f32_dpp %[z], %[c7], %[h7]" BDM_BCAST
+        "v_add_f32 %[u], %[z], %[x]\n\t"
+        "v_and_b32 %[u], %[m], %[u]\n\t"
+        "v_fmac_f32_dpp %[h0], %[b0], %[u]" BDM_BCAST "v_fmac_f32_dpp %[h1], %[b1], %[u]" BDM_BCAST
+        "v_fmac_f32_dpp %[h2], %[b2], %[u]" BDM_BCAST "v_fmac_f32_dpp %[h3], %[b3], %[u]" BDM_BCAST
+        "v_fmac_f32_dpp %[h4], %[b4], %[u]" BDM_BCAST "v_fmac_f32_dpp %[h5], %[b5], %[u]" BDM_BCAST
+        "v_fmac_f32_dpp %[h6], %[b6], %[u]" BDM_BCAST "v_fmac_f32_dpp %[h7], %[b7], %[u]" BDM_BCAST
+        : [z] "=&v"(z), [u] "=&v"(u), [h0] "+v"(h[0]), [h1] "+v"(h[1]), [h2] "+v"(h[2]), [h3] "+v"(h[3]),
+          [h4] "+v"(h[4]), [h5] "+v"(h[5]), [h6] "+v"(h[6]), [h7] "+v"(h[7])
+        : [c0] "v"(coef[0]), [c1] "v"(coef[1]), [c2] "v"(coef[2]), [c3] "v"(coef[3]), [c4] "v"(coef[4]),
+          [c5] "v"(coef[5]), [c6] "v"(coef[6]), [c7] "v"(coef[7]), [b0] "v"(beta[0]), [b1] "v"(beta[1]),
+          [b2] "v"(beta[2]), [b3] "v"(beta[3]), [b4] "v"(beta[4]), [b5] "v"(beta[5]), [b6] "v"(beta[6]),
+          [b7] "v"(beta[7]), [x] "v"(x), [m] "v"(mask), [e] "i"(E));
+}
+#undef BDM_BCAST
+
+// Events FIRST .. FIRST + 7 of a stage, x read from and z written to the lane's column of LDS.
+template <int FIRST, bool EAGER, int... E>
+__device__ __forceinline__ void chain_half(std::integer_sequence<int, E...>, float (&h)[8], const float (&coef)[8],
+                                           const float (&beta)[8], const float (&decay)[8], const float (*x)[kWave],
+                                           uint32_t writes, float (*z)[kWave], int lane) {
+    const float xs[] = {x[FIRST + E][lane]...};
+    float zs[sizeof...(E)];
+    (chain_event<FIRST + E, EAGER>(h, coef, beta, decay, xs[E], 0u - ((writes >> (FIRST + E)) & 1u), zs[E]), ...);
+    ((z[FIRST + E][lane] = zs[E]), ...);
+}
+
+template <bool EAGER>
+__device__ __forceinline__ void chain_stage(float (&h)[8], const float (&coef)[8], const float (&beta)[8],
+                                            const float (&decay)[8], const float (*x)[kWave], uint32_t writes,
+                                            float (*z)[kWave], int lane) {
+    constexpr auto half = std::make_integer_sequence<int, kLazyStage / 2>{};
+    chain_half<0, EAGER>(half, h, coef, beta, decay, x, writes, z, lane);
+    chain_half<kLazyStage / 2, EAGER>(half, h, coef, beta, decay, x, writes, z, lane);
+}
+
+// Lane 16 q + e of x holds event e's value: event 2 I in lanes 0..31, event 2 I + 1 in lanes 32..63.
+template <int I>
+__device__ __forceinline__ int event_pair(int x) {
+    const int even = __builtin_amdgcn_update_dpp(0, x, 0x150 + 2 * I, 0xF, 0xF, true);
+    return __builtin_amdgcn_update_dpp(even, x, 0x151 + 2 * I, 0xC, 0xF, false);
+}
+
+template <int... I, typename F>
+__device__ __forceinline__ void for_each_index(std::integer_sequence<int, I...>, F f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// What a producer wave knows of a stage: lane 16 q + e of event e.
+struct ChainEvent {
+    uint32_t route;
+    int token;
+    bool write, read;
+};
+
+template <typename T>
+__device__ __forceinline__ int64_t chain_order(const ForwardParams<T> &p, int64_t start, int64_t end, int stage) {
+    const int64_t at = start + int64_t(stage) * kLazyStage + (threadIdx.x & (kLazyStage - 1));
+    return at < end ? p.order[at] : int64_t(-1);
+}
+
+template <typename T>
+__device__ __forceinline__ ChainEvent chain_decode(const ForwardParams<T> &p, int64_t o) {
+    ChainEvent m;
+    const int64_t write_events = p.nt * p.kw, events = p.nt * (int64_t(p.kw) + p.kr);
+    const bool live = o >= 0;
+    o = o < 0 ? 0 : (o >= events ? events - 1 : o);
+    const bool rd = o >= write_events;
+    m.route = uint32_t(rd ? o - write_events : o);
+    m.token = int(p.k_shift >= 0 ? m.route >> p.k_shift : m.route / uint32_t(rd ? p.kr : p.kw));
+    m.write = live && !rd;
+    m.read = live && rd;
+    return m;
+}
+
+__device__ __forceinline__ int chain_stages(int64_t start, int64_t end) {
+    return int((end - start + kLazyStage - 1) / kLazyStage);
+}
+
+// The producer of a virtual head's row operands.
+template <typename T, int NC>
+__device__ __forceinline__ void chain_rows(const ForwardParams<T> &p, int seg, int vhead, ChainLds<NC> &lds) {
+    constexpr int S = 8, NE = kLazyStage;
+    using Raw = typename Pair<T>::raw;
+    const int lane = int(threadIdx.x) & (kWave - 1);
+    const int64_t start = p.cu[seg], end = p.cu[seg + 1];
+    const int nstages = chain_stages(start, end);
+    const int ev = lane & (NE - 1), quarter = lane >> 4;  // event, rows 2*quarter, 2*quarter + 1
+    Raw lkey{}, lerase{};  // k (a write), b (q for a read)
+    float2 lgate{};
+    float weight = 0.f;
+    ChainEvent m{};
+    auto issue = [&](const ChainEvent &next) {
+        m = next;
+        const int64_t row = (int64_t(m.token) * p.s_heads + vhead / p.split) * S + 2 * quarter;
+        weight = to_f32((m.read ? p.rw : p.ww)[m.route]);
+        lkey = Pair<T>::load(p.k + row);
+        lerase = Pair<T>::load((m.read ? p.q : p.b) + row);
+        lgate = *reinterpret_cast<const float2 *>(p.g + row);
+    };
+    // as the lazy kernel's stage prep; an event past the segment's end or a read has beta = 0
+    auto finish = [&](int buf) {
+        float d[2], prod[2], sc[2];
+        const float key[2] = {Pair<T>::lo(lkey), Pair<T>::hi(lkey)}, gate[2] = {lgate.x, lgate.y};
+        const float erase[2] = {Pair<T>::lo(lerase), Pair<T>::hi(lerase)};
+        bool low = false;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            prod[r] = round_to<T>(erase[r] * weight) * (m.read ? p.scale : -key[r]);
+            d[r] = m.write ? __expf(p.routed_decay ? gate[r] * weight : gate[r]) : 1.f;
+            sc[r] = row_prefix_product(d[r]);
+            low |= !(sc[r] >= kScaleFloor);
+        }
+        const bool eager = __ballot(low) != 0;
+        float coef[2], beta[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            coef[r] = !(m.write | m.read) ? 0.f : (eager ? prod[r] : prod[r] * sc[r]);
+            beta[r] = !m.write ? 0.f : (eager ? key[r] : key[r] * __builtin_amdgcn_rcpf(sc[r]));
+        }
+        *reinterpret_cast<float2 *>(&lds.rows[buf][ev][2 * quarter]) = make_float2(coef[0], coef[1]);
+        *reinterpret_cast<float2 *>(&lds.rows[buf][ev][S + 2 * quarter]) = make_float2(beta[0], beta[1]);
+        *reinterpret_cast<float2 *>(&lds.decay[buf][ev][2 * quarter]) = make_float2(d[0], d[1]);
+        if (ev == NE - 1)
+            *reinterpret_cast<float2 *>(&lds.fold[buf][2 * quarter]) =
+                eager ? make_float2(1.f, 1.f) : make_float2(sc[0], sc[1]);
+        const uint32_t writes = uint32_t(__ballot(m.write)) & 0xffffu;
+        if (lane == 0) lds.writes[buf] = writes, lds.eager[buf] = eager;
+    };
+    // order of stage s + 3, loads of s + 2 and operands of s + 1 while the consumers run stage s
+    issue(chain_decode(p, chain_order(p, start, end, 0)));
+    int64_t near = chain_order(p, start, end, 1), far = chain_order(p, start, end, 2);
+    finish(0);
+    issue(chain_decode(p, near));
+    __syncthreads();
+    for (int s = 0; s < nstages; ++s) {
+        near = far;
+        far = chain_order(p, start, end, s + 3);
+        finish((s + 1) & 1);
+        issue(chain_decode(p, near));
+        __syncthreads();
+    }
+    __syncthreads();
+}
+
+// The producer of a 64-column tile: x of every stage and the stores of its reads' z.
+template <typename T, int NC>
+__device__ __forceinline__ void chain_columns(const ForwardParams<T> &p, int seg, int vhead, int tile, int which,
+                                              ChainLds<NC> &lds) {
+    constexpr int NE = kLazyStage, NP = NE / 2;
+    constexpr auto pairs = std::make_integer_sequence<int, NP>{};
+    using Raw = typename Pair<T>::raw;
+    constexpr uint32_t kNone = 0xffffffffu;  // (no row starts at an odd byte)
+    const int lane = int(threadIdx.x) & (kWave - 1);
+    const int64_t start = p.cu[seg], end = p.cu[seg + 1];
+    const int nstages = chain_stages(start, end);
+    const int side = lane >> 5, pair = (lane & 31) * 2;  // event parity, first column
+    // rows of v, w and z by 32-bit byte offsets (chain_path)
+    const uint32_t row_bytes = uint32_t(p.heads) * uint32_t(p.width) * uint32_t(sizeof(T));
+    const uint32_t lane_bytes = uint32_t(vhead * p.width + tile * kWave + pair) * uint32_t(sizeof(T));
+    const char *v = reinterpret_cast<const char *>(p.v), *w = reinterpret_cast<const char *>(p.w);
+    char *z = reinterpret_cast<char *>(p.zbuf);
+    Raw lv[NP], lw[NP];
+    float weight = 0.f;
+    uint32_t z_row = kNone, z_next = kNone;  // z rows of the stage that the consumers run, and of the one after
+    auto issue = [&](const ChainEvent &m) {
+        // a read's v, w are not used: the last write's before it, whose lines are on their way
+        const uint32_t before = uint32_t(__ballot(m.write)) & 0xffffu & ((2u << (lane & (NE - 1))) - 1u);
+        const uint32_t row = uint32_t(__shfl(m.token, before ? 31 - __clz(before) : 0)) * row_bytes;
+        for_each_index(pairs, [&](auto i) {
+            const uint32_t at = uint32_t(event_pair<i>(int(row))) + lane_bytes;
+            lv[i] = Pair<T>::load(reinterpret_cast<const T *>(v + at));
+            lw[i] = Pair<T>::load(reinterpret_cast<const T *>(w + at));
+        });
+        weight = to_f32((m.read ? p.rw : p.ww)[m.route]);
+        z_next = m.read ? m.route * row_bytes : kNone;
+    };
+    auto finish = [&](int buf) {
+        for_each_index(pairs, [&](auto i) {
+            const float pw = __int_as_float(event_pair<i>(__float_as_int(weight)));
+            *reinterpret_cast<float2 *>(&lds.x[buf][which][2 * i + side][pair]) =
+                make_float2(round_to<T>(Pair<T>::lo(lw[i]) * pw) * Pair<T>::lo(lv[i]),
+                            round_to<T>(Pair<T>::hi(lw[i]) * pw) * Pair<T>::hi(lv[i]));
+        });
+    };
+    auto store_z = [&](uint32_t rows, int buf) {
+        for_each_index(pairs, [&](auto i) {
+            const float2 z2 = *reinterpret_cast<const float2 *>(&lds.z[buf][which][2 * i + side][pair]);
+            const float pairs2[2] = {z2.x, z2.y};
+            const uint32_t row = uint32_t(event_pair<i>(int(rows)));
+            if (row != kNone) store_cols(reinterpret_cast<T *>(z + (row + lane_bytes)), pairs2);
+        });
+    };
+    // as chain_rows; also the z of stage s - 1
+    issue(chain_decode(p, chain_order(p, start, end, 0)));
+    int64_t near = chain_order(p, start, end, 1), far = chain_order(p, start, end, 2);
+    finish(0);
+    z_row = z_next;
+    issue(chain_decode(p, near));
+    __syncthreads();
+    for (int s = 0; s < nstages; ++s) {
+        const uint32_t done = z_row;
+        near = far;
+        far = chain_order(p, start, end, s + 3);
+        finish((s + 1) & 1);
+        z_row = z_next;
+        issue(chain_decode(p, near));
+        __syncthreads();
+        store_z(done, s & 1);
+    }
+    __syncthreads();
+}
+
+// The consumer of a 64-column tile: the state of one column per lane.
+template <typename T, int NC>
+__device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg, int vhead, int tile, int which,
+                                              ChainLds<NC> &lds) {
+    constexpr int S = 8, NE = kLazyStage;
+    const int lane = int(threadIdx.x) & (kWave - 1);
+    const int bank = seg % p.banks;
+    const int64_t bidx = seg / p.banks;
+    const int64_t start = p.cu[seg], end = p.cu[seg + 1];
+    const int nstages = int((end - start + NE - 1) / NE);
+    const bool rounding = p.round_interval > 0;
+    const int64_t head_cols = int64_t(vhead / p.split) * S * p.row_stride + int64_t(vhead % p.split) * p.width +
+                              tile * kWave + lane;
+    const int64_t state_offset = int64_t(bank) * p.s_heads * S * p.row_stride + head_cols;
+    float h[S];
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        const int64_t at = bidx * p.init_bstride + state_offset + int64_t(r) * p.row_stride;
+        const float x = p.init_dtype == BDM_BF16 ? to_f32(static_cast<const bf16_t *>(p.initial)[at])
+                                                 : static_cast<const float *>(p.initial)[at];
+        h[r] = rounding ? round_bf16(x) : x;
+    }
+    auto store_h = [&](void *base, int dtype, int64_t offset) {
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const int64_t at = offset + int64_t(r) * p.row_stride;
+            if (dtype == BDM_BF16) static_cast<bf16_t *>(base)[at] = from_f32<bf16_t>(h[r]);
+            else static_cast<float *>(base)[at] = h[r];
+        }
+    };
+    auto load8 = [&](const float *row, float (&x)[S]) {
+        const float4 lo = reinterpret_cast<const float4 *>(row)[0], hi = reinterpret_cast<const float4 *>(row)[1];
+        x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w, x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
+    };
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s < nstages; ++s) {
+        const int buf = s & 1;
+        float coef[S], beta[S];
+        load8(lds.rows[buf][lane & (NE - 1)], coef);
+        load8(lds.rows[buf][lane & (NE - 1)] + S, beta);
+        const uint32_t writes = __builtin_amdgcn_readfirstlane(lds.writes[buf]);
+        const int eager = __builtin_amdgcn_readfirstlane(lds.eager[buf]);
+        if (s > 0) {
+            if (rounding) {
+#pragma unroll
+                for (int r = 0; r < S; ++r) h[r] = round_bf16(h[r]);
+            }
+            // snapshot of the state before event 16 s of the segment (see staged_forward_kernel)
+            if (p.snap)
+                store_h(p.snap, p.snap_dtype, (start / NE + s - 1) * p.s_heads * S * p.row_stride + head_cols);
+        }
+        if (!eager) {
+            chain_stage<false>(h, coef, beta, coef, lds.x[buf][which], writes, lds.z[buf][which], lane);
+        } else {
+            float decay[S];
+            load8(lds.decay[buf][lane & (NE - 1)], decay);
+            chain_stage<true>(h, coef, beta, decay, lds.x[buf][which], writes, lds.z[buf][which], lane);
+        }
+        float fold[S];
+        load8(lds.fold[buf], fold);
+#pragma unroll
+        for (int r = 0; r < S; ++r) h[r] *= fold[r];
+        __syncthreads();
+    }
+    if (p.final_state)
+        store_h(p.final_state, p.final_dtype, bidx * (int64_t(p.banks) * p.s_heads * S * p.row_stride) + state_offset);
+    __syncthreads();
+}
+
+// One workgroup of 2 NC + 1 waves per (long segment, virtual head, 64 NC
+// columns): waves 0 .. NC-1 consume, the others produce.  Items of an XCD: its
+// segments longest first; a workgroup stops at the first segment that is not
+// long.
+template <typename T, int NC>
+__global__ __launch_bounds__(kWave *(2 * NC + 1)) __attribute__((amdgpu_waves_per_eu(5, 8))) void chain_forward_kernel(
+    ForwardParams<T> p) {
+    __shared__ __align__(16) ChainLds<NC> lds;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    auto each_item = [&](auto run) {  // (a loop per role: no role's loop invariants live through another's)
+        const int range = p.nseg / 8, parts = p.width / (NC * kWave), per_seg = p.heads * parts;
+#pragma unroll 1
+        for (int64_t item = blockIdx.x / 8;; item += gridDim.x / 8) {
+            const int64_t rank = item / per_seg;
+            if (rank >= range) return;
+            const int seg = p.seg_order[int(blockIdx.x % 8) * range + int(rank)];
+            if (p.cu[seg + 1] - p.cu[seg] <= p.skip_long) return;
+            // the longest segments ahead of the others on a SIMD, which have time
+            if (rank < 2) __builtin_amdgcn_s_setprio(3);
+            else if (rank < 6) __builtin_amdgcn_s_setprio(2);
+            else __builtin_amdgcn_s_setprio(1);
+            run(seg, int(item % per_seg) / parts, int(item % parts) * NC);
+        }
+    };
+    if (wave < NC)
+        each_item([&](int seg, int vhead, int tile) { chain_consume<T, NC>(p, seg, vhead, tile + wave, wave, lds); });
+    else if (wave == NC)
+        each_item([&](int seg, int vhead, int) { chain_rows<T, NC>(p, seg, vhead, lds); });
+    else
+        each_item([&](int seg, int vhead, int tile) {
+            chain_columns<T, NC>(p, seg, vhead, tile + wave - NC - 1, wave - NC - 1, lds);
+        });
+}
+
 // Exclusive prefix of x over the 1024 threads of the workgroup, and the
 // total in *total: within each wave by shuffles, then over the 16 wave totals
 // by the first wave.  lds: 1024 / kWave + 1 ints.
@@ -1750,6 +2127,8 @@ struct PieceBuffers {
     int *st_count = nullptr, *st_segs = nullptr;
     float *st_r = nullptr, *st_p = nullptr, *st_z0 = nullptr, *st_c = nullptr;
     int *st_tgt = nullptr;
+    // Segments longer than this run on chain_forward_kernel (0: none do).
+    int chain_events = 0;
 };
 
 // Profiling events of bdm_forward (phase_events): 0 before the recurrence,
@@ -1999,11 +2378,30 @@ int launch_stage_path(const ForwardParams<T> &p0, const PieceBuffers &pb, int th
 // its chain's latency, beside the sequential kernel over the other segments
 // (on an auxiliary stream, after the pieces), then the reads and the
 // combine over every column.
+// chain_forward_kernel over the segments longer than p.skip_long: on each XCD
+// at most 128 workgroups (4 per CU, what its LDS holds), fewer where its range
+// cannot hold that many long segments.
+template <typename T>
+int launch_chains(const bdm_forward_args &a, const ForwardParams<T> &p, hipStream_t st) {
+    const int64_t range = p.nseg / 8, sequences = (range + a.bank_count - 1) / a.bank_count + 1;
+    const int64_t events = std::min(a.batch, sequences) * a.time * (int64_t(a.write_banks) + a.read_banks);
+    const int64_t segments = std::min(range, events / (p.skip_long + 1));
+    const int nc = p.width % (2 * kWave) == 0 ? 2 : 1;
+    const int64_t items = segments * p.heads * (p.width / (nc * kWave));
+    const unsigned blocks = 8 * unsigned(std::min<int64_t>(128, items));
+    if (!blocks) return BDM_OK;
+    if (nc == 2)
+        chain_forward_kernel<T, 2><<<blocks, 5 * kWave, 0, st>>>(p);
+    else
+        chain_forward_kernel<T, 1><<<blocks, 3 * kWave, 0, st>>>(p);
+    return check_launch("chain_forward_kernel");
+}
+
 template <typename T, int CPL>
 int launch_overlapped_stage(const bdm_forward_args &a, ForwardParams<T> p, const void *kernel, unsigned nseg,
                             int groups, int threads, const T *zbuf, const OverlapAux &ax, const PieceBuffers &pb,
                             hipStream_t stream) {
-    p.skip_long = 1;  // the sequential kernel leaves the long segments to the stage path
+    p.skip_long = kPieceEvents;  // the sequential kernel leaves the long segments to the stage path
     if (int rc = launch_stage_path<T, CPL>(p, pb, threads, groups, stream, ax.fork)) return rc;
     hipStream_t side = ax.stream[0];
     if (hipStreamWaitEvent(side, ax.fork, 0) != hipSuccess)
@@ -2022,17 +2420,32 @@ int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void 
     if (pb.stage_pieces > 0)
         return launch_overlapped_stage<T, CPL>(a, p, kernel, nseg, groups, threads, zbuf, ax, pb, stream);
     const int gpr = p.order_gpr;
-    const int parts = overlap_parts((groups + gpr - 1) / gpr, groups);
+    const bool chain = pb.chain_events > 0;
+    int parts = groups > gpr ? overlap_parts((groups + gpr - 1) / gpr, groups) : 1;
+    if (chain) parts = min(parts, kOverlapAux - 1);
+    hipEvent_t chains_done = ax.join[kOverlapAux - 1];
+    // part i's stream: the caller's and the auxiliary ones, or behind the chains the auxiliary ones
+    auto stream_of = [&](int i) { return chain ? ax.stream[i] : (i ? ax.stream[i - 1] : stream); };
     if (hipEventRecord(ax.fork, stream) != hipSuccess)
         return fail(BDM_ERR_LAUNCH, "forward: forking the combine streams");
-    for (int i = 1; i < parts; ++i) {
-        if (hipStreamWaitEvent(ax.stream[i - 1], ax.fork, 0) != hipSuccess)
+    if (chain) {
+        // The long segments first, on the caller's stream: the parts wait for
+        // the fork on theirs, a few microseconds, in which the chains' blocks
+        // reach their slots (behind one-wave blocks, which take every slot as
+        // it frees, a workgroup of five waves would wait for the last of them).
+        p.skip_long = pb.chain_events;
+        if (int rc = launch_chains<T>(a, p, stream)) return rc;
+        if (hipEventRecord(chains_done, stream) != hipSuccess)
+            return fail(BDM_ERR_LAUNCH, "forward: recording the chains' end");
+    }
+    for (int i = chain ? 0 : 1; i < parts; ++i) {
+        if (hipStreamWaitEvent(stream_of(i), ax.fork, 0) != hipSuccess)
             return fail(BDM_ERR_LAUNCH, "forward: forking the combine streams");
-        for (int gate = 0; gate < i; ++gate) overlap_gate_kernel<<<1, 1, 0, ax.stream[i - 1]>>>();
+        for (int gate = 0; gate < i; ++gate) overlap_gate_kernel<<<1, 1, 0, stream_of(i)>>>();
         if (int rc = check_launch("overlap_gate_kernel")) return rc;
     }
     for (int i = 0; i < parts; ++i) {
-        hipStream_t st = i ? ax.stream[i - 1] : stream;
+        hipStream_t st = stream_of(i);
         // the larger parts first: the last part's combine is the one left
         // exposed after the recurrence
         const int g0 = groups - int(int64_t(groups) * (parts - i) / parts);
@@ -2043,13 +2456,15 @@ int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void 
         if (int rc = launch_mode0<T>(kernel, dim3(nseg, unsigned(g1 - g0)), threads, pr, st)) return rc;
         if (i == parts - 1)
             if (int rc = record_phase(a, 1, st)) return rc;
+        if (chain && hipStreamWaitEvent(st, chains_done, 0) != hipSuccess)
+            return fail(BDM_ERR_LAUNCH, "forward: joining the chains");
         const int h0 = g0 * p.heads_per_block;
         const int h1 = min(g1 * p.heads_per_block, p.heads);
         if (int rc = launch_combine_kernels<T>(a, zbuf, st, h0 * p.width, (h1 - h0) * p.width)) return rc;
     }
-    for (int i = 1; i < parts; ++i)
-        if (hipEventRecord(ax.join[i - 1], ax.stream[i - 1]) != hipSuccess ||
-            hipStreamWaitEvent(stream, ax.join[i - 1], 0) != hipSuccess)
+    for (int i = 0; i < (chain ? parts : parts - 1); ++i)
+        if (hipEventRecord(ax.join[i], ax.stream[i]) != hipSuccess ||
+            hipStreamWaitEvent(stream, ax.join[i], 0) != hipSuccess)
             return fail(BDM_ERR_LAUNCH, "forward: joining the combine streams");
     return record_phase(a, 2, stream);
 }
@@ -2193,7 +2608,9 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
                 // rounds whose heads' columns split y in whole 16-byte groups
                 const bool aligned_rounds = (int64_t(p.heads_per_block) * p.width * sizeof(T)) % 16 == 0 &&
                                             (int64_t(a.heads) * a.head_width * sizeof(T)) % 16 == 0;
-                if (a.read_banks > 0 && int(grid.y) > p.order_gpr && aligned_rounds && overlap_enabled()) {
+                const bool rounds = int(grid.y) > p.order_gpr && aligned_rounds;
+                if (a.read_banks > 0 && (rounds || pb.chain_events) && overlap_enabled()) {
+                    if (!rounds) p.order_gpr = int(grid.y);
                     if (const OverlapAux *ax = overlap_aux(stream)) {
                         // the shared events are recorded and waited for by one call at a time
                         std::lock_guard<std::mutex> lock(overlap_launch_mutex());
@@ -2205,7 +2622,7 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             // the stage path after the sequential kernel, on the same stream
             if (pb.stage_pieces > 0) {
                 ForwardParams<T> ps = p;
-                ps.skip_long = 1;
+                ps.skip_long = kPieceEvents;
                 if (int rc = launch_mode0<T>(kernel, grid, lthreads, ps, stream)) return rc;
                 if (int rc = launch_stage_path<T, CPL>(p, pb, lthreads, int(grid.y), stream)) return rc;
                 return launch_combine<T>(a, zbuf, stream);
@@ -2264,6 +2681,31 @@ int64_t stage_pieces(const bdm_forward_args &a) {
 int64_t stage_slots(const bdm_forward_args &a) {
     const int64_t events = a.batch * a.time * (int64_t(a.write_banks) + a.read_banks);
     return events / kLazyStage + a.batch * a.bank_count + 1;
+}
+
+// The length above which a segment runs on chain_forward_kernel beside the
+// others (0: the path is off).  MODE 0 takes ~0.21 us per event of a lone
+// segment, 2T events at most, and ~0.63 ns per event and 1,024 columns over the
+// whole chip, (KW + KR) B T events: where batch * columns is small the longest
+// segment of a skewed routing outlasts everything else.  At 65,536 columns times
+// route slots (B = 4, 1,024 columns, 8 + 8 banks, T = 8,192, 2,048 banks, Zipf
+// 1.1: 15,000 of 524,288 events in one segment) the whole forward went from 3.53
+// to 1.21 ms; at twice that a fork costs 3 us of a uniform routing's 424, and
+// the path is left out.  Long is 2,048 events, a third of the time of everything
+// else there (1,024: 1.28 ms, 3,072: 1.22), or 4 times the mean.  Without
+// snapshots only: a training step's backward walks the same chain at its own
+// pace.
+bool order_path(const bdm_forward_args &a);
+int chain_events(const bdm_forward_args &a) {
+    const int64_t columns = int64_t(a.heads) * a.head_width, slots = int64_t(a.write_banks) + a.read_banks;
+    const int64_t nt = a.batch * a.time, row = columns * (a.ctrl_dtype == BDM_BF16 ? 2 : 4);
+    const int width = a.head_width / std::max(1, lazy_split(a));
+    if (!lazy_path(a) || a.round_interval <= 0 || a.snapshots || !order_path(a) || stage_enabled() || width % kWave != 0 ||
+        a.time < 2048 || a.batch * columns * slots > 98304 || nt * row > int64_t(UINT32_MAX) ||
+        nt * a.read_banks * row > int64_t(UINT32_MAX) || nt * slots > int64_t(INT32_MAX))
+        return 0;
+    const int64_t mean = a.time * slots / a.bank_count, length = std::max<int64_t>(2048, 4 * mean);
+    return a.time >= length ? int(length) : 0;
 }
 
 // Whether the recurrence takes each XCD range's segments longest first
@@ -2462,6 +2904,7 @@ extern "C" int bdm_forward(const bdm_forward_args *a, void *workspace, size_t wo
         pb.order_given = a->segment_order != nullptr;
         if (pb.order_given) pb.seg_order = const_cast<int *>(a->segment_order);
     }
+    if (pb.seg_order) pb.chain_events = chain_events(*a);
     pb.stage_pieces = stage_pieces(*a);
     if (pb.stage_pieces > INT32_MAX / 2) return fail(BDM_ERR_UNSUPPORTED, "forward: too many pieces");
     if (pb.stage_pieces) {

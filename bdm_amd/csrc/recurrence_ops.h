@@ -103,13 +103,13 @@ struct Pair<float> {
 
 // Columns of T as loaded: a pair (CPL = 2, one load) or one.
 template <typename T, int CPL>
-struct RawCols {
+struct LaneCols {
     T x;
     __device__ __forceinline__ void load(const T *at) { x = *at; }
     __device__ __forceinline__ float get(int) const { return to_f32(x); }
 };
 template <typename T>
-struct RawCols<T, 2> {
+struct LaneCols<T, 2> {
     typename Pair<T>::raw x;
     __device__ __forceinline__ void load(const T *at) { x = Pair<T>::load(at); }
     __device__ __forceinline__ float get(int c) const { return c ? Pair<T>::hi(x) : Pair<T>::lo(x); }

@@ -354,6 +354,47 @@ def test_forward_decay_extremes_match_oracle(device, decay, state_dtype):
     assert rel_err(final, ref_final) < TOL, rel_err(final, ref_final)
 
 
+@pytest.mark.parametrize('heads,v,dtype,decay', [
+    (2, 128, torch.bfloat16, 'mild'), (1, 64, torch.bfloat16, 'mild'), (1, 384, torch.bfloat16, 'mixed'),
+    (1, 128, torch.float32, 'mild'), (1, 128, torch.bfloat16, 'strong')],
+    ids=['h2v128', 'h1v64', 'h1v384', 'f32', 'eager'])
+def test_forward_long_chains_match_oracle(device, heads, v, dtype, decay, monkeypatch):
+    """Rounding policy: segments of 3,000 and 4,500 events (no multiple of the 16-event stages) among short and empty
+    ones take the producer/consumer kernel; reads and final states against the oracle and against the same forward
+    without it, which differs in the rounding of one sum per write and in the state roundings that flips."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(37)
+    batch, time, s, j = 2, 2304, 8, 8
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.03, torch.randint(1, 6, (batch, time, 1), generator=gen), 0)
+              for _ in range(2))
+    ri[1, 700:] = 6  # sequence 1: reads mostly elsewhere, a run of writes only
+    ww, rw = (torch.rand(batch, time, 1, generator=gen).to(dtype) for _ in range(2))
+    q, k, v_, g, b, w = controllers(batch, time, heads, s, v, gen, dtype)
+    if decay == 'strong':  # every stage's scale underflows
+        g = g * 200.0
+    elif decay == 'mixed':
+        g = g * torch.where(torch.rand(batch, time, 1, 1, generator=gen) < 0.02, 200.0, 1.0)
+    state = initial_state(j, heads, s, v, gen)
+    dev = [t.to(device) for t in (q, k, v_, g, b, w, wi, ww, ri, rw, state)]
+    announce('forward long chains', heads, v, dtype, decay)
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    lengths = sorted((meta.cu_seqlens[1:] - meta.cu_seqlens[:-1]).tolist())
+    assert lengths[-1] > 4000 and 2304 < lengths[-2] < 4000 and lengths[0] == 0
+    results = []
+    for overlap in ('1', '0'):
+        monkeypatch.setenv('BDM_COMBINE_OVERLAP', overlap)  # 0: one launch over whole segments
+        final = torch.empty(batch, j, heads, s, v, device=device, dtype=torch.float32)
+        y = ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
+                               round_interval=16, final_state=final)
+        torch.cuda.synchronize()
+        results.append((y, final))
+    ref = oracle_reads(q, k, v_, g, b, w, wi, ww, ri, rw, state, j, routed_decay=True, state_dtype=torch.bfloat16,
+                       interval=16, return_final=True)
+    for ours, whole, theirs in zip(*results, ref):
+        assert rel_err(ours, theirs) < TOL, rel_err(ours, theirs)
+        assert rel_err(ours, whole) < TOL, rel_err(ours, whole)
+
+
 def test_forward_per_head_layout_and_determinism(device):
     from bdm_amd import bank_training
     gen = torch.Generator().manual_seed(11)
