@@ -59,6 +59,7 @@ struct BackwardParams {
     float *dinit;   // [batch, J, H, S, v]
     int64_t init_bstride, nt;
     int heads, s_real, width, banks, kw, kr, tiles;
+    int k_shift;  // log2 of KW and KR when both are that power of two, else -1 (route -> token by shift)
     int init_dtype, snap_dtype, routed_decay, rounding;
     int xcd_remap;
     float scale;
@@ -136,10 +137,9 @@ __device__ __forceinline__ float reduce_scatter(const float (&x)[N], int lane) {
     return out;
 }
 
-// One entry per event of the packed order: token, route slot (PER_TOKEN: the
-// route's index within its token), is_read and the route weight (FP32 bits),
-// shared by every head.
-template <typename T, bool PER_TOKEN>
+// One entry per event of the packed order: token, route slot, is_read and
+// the route weight (FP32 bits), shared by every head.
+template <typename T>
 __global__ __launch_bounds__(256) void event_meta_kernel(const int64_t *order, int64_t events, int64_t write_events,
                                                          int kw, int kr, const T *ww, const T *rw, int4 *meta) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void event_meta_kernel(const int64_t *order, i
     const int64_t route = rd ? o - write_events : o;
     const int64_t token = rd ? route / kr : route / kw;
     const float weight = to_f32(rd ? rw[route] : ww[route]);
-    meta[e] = make_int4(int(token), int(PER_TOKEN ? route - token * (rd ? kr : kw) : route), rd ? 1 : 0, __float_as_int(weight));
+    meta[e] = make_int4(int(token), int(route), rd ? 1 : 0, __float_as_int(weight));
 }
 
 template <typename T, typename SNAP>
@@ -632,9 +632,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
     const int lane_col = head * p.width + colc;
 
     auto chunk_len = [&](int c) { return int(min(int64_t(C), end - (start + int64_t(c) * C))); };
+    // Event lane % C of chunk c: token, route index within the token, is_read, route weight.
     auto load_meta = [&](int c) {
+        const int64_t write_events = p.nt * p.kw, events = p.nt * (int64_t(p.kw) + p.kr);
         const int len = chunk_len(c);
-        return p.meta[start + int64_t(c) * C + (lane < len ? lane : len - 1)];
+        int64_t o = p.order[start + int64_t(c) * C + (lane < len ? lane : len - 1)];
+        o = o < 0 ? 0 : (o >= events ? events - 1 : o);
+        const bool rd = o >= write_events;
+        const int64_t route = rd ? o - write_events : o;
+        const int k = rd ? p.kr : p.kw;
+        const int64_t token = p.k_shift >= 0 ? route >> p.k_shift
+                                             : (events <= int64_t(UINT32_MAX) ? int64_t(uint32_t(route) / uint32_t(k)) : route / k);
+        return make_int4(int(token), int(route - token * k), rd ? 1 : 0, __float_as_int(to_f32(rd ? p.rw[route] : p.ww[route])));
     };
     auto store_meta = [&](int c, const int4 &m) {
         if (lane < C) s_meta[c & 1][lane] = m;
@@ -1176,7 +1185,7 @@ __global__ __launch_bounds__(256) void token_vjp_kernel(VjpParams<T> p) {
 
 struct Workspace {
     float *du, *wpart, *rpart;
-    int4 *meta;      // per-event meta
+    int4 *meta;      // per-event meta of the S = 8 chunk kernel (null otherwise)
     int *seg_order;  // longest-first segment order (null: bank order)
     size_t bytes;
 };
@@ -1232,7 +1241,7 @@ Workspace carve(const bdm_backward_args &a, void *base) {
     const size_t du = align256(nt * a.write_banks * a.heads * size_t(a.head_width) * sizeof(float));
     const size_t wp = align256(tiles * 3 * nt * a.write_banks * hs * sizeof(float));
     const size_t rp = align256(tiles * nt * a.read_banks * hs * sizeof(float));
-    const size_t mt = align256(nt * size_t(a.write_banks + a.read_banks) * sizeof(int4));
+    const size_t mt = chunk_path(a) ? align256(nt * size_t(a.write_banks + a.read_banks) * sizeof(int4)) : 0;
     const int64_t nseg = int64_t(a.batch) * a.bank_count;
     const size_t so = order_geometry(nseg) ? align256(size_t(nseg) * sizeof(int)) : 0;
     char *c = static_cast<char *>(base);
@@ -1240,7 +1249,7 @@ Workspace carve(const bdm_backward_args &a, void *base) {
     w.du = reinterpret_cast<float *>(c);
     w.wpart = reinterpret_cast<float *>(c ? c + du : nullptr);
     w.rpart = reinterpret_cast<float *>(c ? c + du + wp : nullptr);
-    w.meta = reinterpret_cast<int4 *>(c ? c + du + wp + rp : nullptr);
+    w.meta = reinterpret_cast<int4 *>(c && mt ? c + du + wp + rp : nullptr);
     w.seg_order = reinterpret_cast<int *>(c && so && order_enabled() ? c + du + wp + rp + mt : nullptr);
     w.bytes = du + wp + rp + mt + so;
     return w;
@@ -1276,6 +1285,9 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
     p.kw = a.write_banks;
     p.kr = a.read_banks;
     p.tiles = column_tiles(a);
+    p.k_shift = -1;
+    for (int sh = 0; sh < 8; ++sh)
+        if (a.write_banks == (1 << sh) && a.read_banks == (1 << sh)) p.k_shift = sh;
     p.init_dtype = a.initial_dtype;
     p.snap_dtype = a.snapshot_dtype;
     p.routed_decay = a.routed_decay;
@@ -1284,12 +1296,13 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
     const int64_t nseg = a.batch * a.bank_count;
     p.xcd_remap = (nseg % 8 == 0) ? 1 : 0;
     const dim3 grid(unsigned(nseg), unsigned(a.heads), unsigned(p.tiles));
-    const int64_t events = p.nt * (p.kw + p.kr);
-    if ((events + 255) / 256 > int64_t(UINT32_MAX)) return fail(BDM_ERR_UNSUPPORTED, "backward: too many events");
-    event_meta_kernel<T, !CHUNK><<<unsigned((events + 255) / 256), 256, 0, stream>>>(p.order, events, p.nt * p.kw, p.kw,
-                                                                                    p.kr, p.ww, p.rw, ws.meta);
-    if (int rc = check_launch("event_meta_kernel")) return rc;
-    p.meta = ws.meta;
+    if constexpr (CHUNK) {
+        const int64_t events = p.nt * (p.kw + p.kr);
+        const unsigned blocks = unsigned((events + 255) / 256);
+        event_meta_kernel<T><<<blocks, 256, 0, stream>>>(p.order, events, p.nt * p.kw, p.kw, p.kr, p.ww, p.rw, ws.meta);
+        if (int rc = check_launch("event_meta_kernel")) return rc;
+        p.meta = ws.meta;
+    }
     if (ws.seg_order) {
         launch_segment_order(p.cu, nseg, ws.seg_order, stream);
         if (int rc = check_launch("segment_order_kernel")) return rc;
