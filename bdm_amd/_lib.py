@@ -38,6 +38,10 @@ EXPORTED_SYMBOLS = (
     'bdm_router_select_pair',
     'bdm_route_dispatch_workspace_size',
     'bdm_route_dispatch',
+    'bdm_controller_backward',
+    'bdm_output_backward_partials',
+    'bdm_output_backward',
+    'bdm_router_backward',
 )
 
 _i32, _i64, _f32, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
@@ -132,6 +136,31 @@ class OutputArgs(ctypes.Structure):
     """Mirror of ``bdm_output_args``."""
     _fields_ = [
         ('raw', _vp), ('gate', _vp), ('norm_weight', _vp), ('norm_bias', _vp), ('out', _vp),
+        ('tokens', _i64), ('gate_stride', _i64),
+        ('width', _i32), ('ctrl_dtype', _i32), ('param_dtype', _i32), ('norm_kind', _i32), ('eps', _f32),
+    ]
+
+
+class ControllerGradArgs(ctypes.Structure):
+    """Mirror of ``bdm_controller_grad_args``."""
+    _fields_ = [
+        ('proj', _vp), ('f', _vp), ('a_log', _vp), ('dt_bias', _vp),
+        ('grad_q', _vp), ('grad_k', _vp), ('grad_v', _vp), ('grad_b', _vp), ('grad_w', _vp), ('grad_g', _vp),
+        ('grad_read', _vp), ('grad_write', _vp), ('grad_gate', _vp),
+        ('grad_proj', _vp), ('grad_f', _vp), ('grad_terms', _vp),
+        ('tokens', _i64), ('proj_stride', _i64), ('f_stride', _i64),
+        ('q_col', _i32), ('k_col', _i32), ('v_col', _i32), ('b_col', _i32), ('w_col', _i32),
+        ('read_col', _i32), ('write_col', _i32), ('gate_col', _i32),
+        ('heads', _i32), ('bank_size', _i32), ('head_width', _i32), ('route_width', _i32),
+        ('ctrl_dtype', _i32), ('param_dtype', _i32), ('qk_norm', _i32),
+    ]
+
+
+class OutputGradArgs(ctypes.Structure):
+    """Mirror of ``bdm_output_grad_args``."""
+    _fields_ = [
+        ('raw', _vp), ('gate', _vp), ('grad_out', _vp), ('norm_weight', _vp), ('norm_bias', _vp),
+        ('grad_raw', _vp), ('grad_gate', _vp), ('partials', _vp),
         ('tokens', _i64), ('gate_stride', _i64),
         ('width', _i32), ('ctrl_dtype', _i32), ('param_dtype', _i32), ('norm_kind', _i32), ('eps', _f32),
     ]
@@ -238,6 +267,14 @@ def library() -> ctypes.CDLL:
     lib.bdm_route_dispatch_workspace_size.restype = _size_t
     lib.bdm_route_dispatch.argtypes = [ctypes.POINTER(RouteDispatchArgs), _vp, _size_t, _vp]
     lib.bdm_route_dispatch.restype = _i32
+    lib.bdm_controller_backward.argtypes = [ctypes.POINTER(ControllerGradArgs), _vp]
+    lib.bdm_controller_backward.restype = _i32
+    lib.bdm_output_backward_partials.argtypes = [_i64]
+    lib.bdm_output_backward_partials.restype = _i64
+    lib.bdm_output_backward.argtypes = [ctypes.POINTER(OutputGradArgs), _vp]
+    lib.bdm_output_backward.restype = _i32
+    lib.bdm_router_backward.argtypes = [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp]
+    lib.bdm_router_backward.restype = _i32
     return lib
 
 

@@ -28,6 +28,57 @@ from .routing import SharedResidualRouter, product_key_route
 Tensor = torch.Tensor
 
 
+class _LayerInputs(torch.autograd.Function):
+    """The controllers, route scores and output-gate projection of a layer from
+    one projection [N, P] of its input: f_proj's second factor and the controller
+    epilogue forward; backward, every column of the projection's gradient in one
+    kernel around the two products of that factor."""
+
+    @staticmethod
+    def forward(ctx, proj, f_weight, a_log, dt_bias, columns, geometry):
+        hv, rw = geometry['head_width'], geometry['route_width']
+        total = geometry['heads'] * hv
+        f = F.linear(proj[:, columns['f']:columns['f'] + hv], f_weight)
+        controllers = ops.controller_epilogue(proj, f, columns, a_log, dt_bias, heads=geometry['heads'],
+                                              bank_size=geometry['bank_size'], head_width=hv,
+                                              qk_norm=geometry['qk_norm'])
+        ctx.save_for_backward(proj, f, f_weight, a_log, dt_bias)
+        ctx.columns, ctx.geometry = columns, geometry
+        # copies, not views: an output that shares an input's storage could not be saved or changed in place apart
+        read, write, gate = (proj[:, columns[n]:columns[n] + width].contiguous()
+                             for n, width in (('read', rw), ('write', rw), ('gate', total)))
+        return (*controllers, read, write, gate)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *grads):
+        proj, f, f_weight, a_log, dt_bias = ctx.saved_tensors
+        columns, geometry = ctx.columns, ctx.geometry
+        grad_proj, grad_f, terms = ops.controller_backward(proj, f, columns, a_log, dt_bias, grads, **geometry)
+        at = slice(columns['f'], columns['f'] + geometry['head_width'])
+        torch.mm(grad_f, f_weight, out=grad_proj[:, at])
+        grad_weight = grad_f.t() @ proj[:, at]
+        grad_dt, rate = terms.sum(0)
+        grad_a = rate.view(geometry['heads'], geometry['bank_size']).sum(-1)
+        return grad_proj, grad_weight, grad_a.to(a_log.dtype), grad_dt.to(dt_bias.dtype), None, None
+
+
+class _OutputInterface(torch.autograd.Function):
+    """norm(raw) * sigmoid(gate) before o_proj (_parameters.py:222-232)."""
+
+    @staticmethod
+    def forward(ctx, raw, gate, weight, bias, eps, kind):
+        ctx.save_for_backward(raw, gate, weight, bias)
+        ctx.eps, ctx.kind = eps, kind
+        return ops.output_epilogue(raw, gate, weight, bias, eps=eps, kind=kind)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_out):
+        raw, gate, weight, bias = ctx.saved_tensors
+        return (*ops.output_backward(raw, gate, weight, bias, grad_out, eps=ctx.eps, kind=ctx.kind), None, None)
+
+
 class BankedDeltaMemory(nn.Module):
     """Shared-residual product routing around dense GDN2 memory banks."""
 
@@ -329,7 +380,64 @@ class BankedDeltaMemory(nn.Module):
             raise ValueError('the hip backend requires ROCm tensors; the CPU oracle lives in oracle/')
         if not torch.is_grad_enabled() and self._fused_supported(hidden):
             return self._forward_inference(hidden)
+        if torch.is_grad_enabled() and self._fused_training_supported(hidden):
+            return self._forward_training(hidden)
         return self._project_bank_output(hidden, self.bank_reads(hidden))
+
+    def _fused_training_supported(self, hidden: Tensor) -> bool:
+        """Whether the autograd forward may project once and run the fused
+        controller and output kernels: BF16 throughout (FP32 keeps torch's exact
+        exponentials and divisions), 16-byte column groups, and plain projections
+        whose own forward and hooks the one product stands for."""
+        linears = (self.q_proj, self.k_proj, self.v_proj, self.f_proj[0], self.f_proj[1], self.b_proj, self.w_proj,
+                   self.shared_router.base, self.shared_router.read_residual, self.shared_router.write_residual,
+                   self.output_gate)
+        plain = all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                                                  or m._backward_pre_hooks) for m in linears)
+        containers = (self.f_proj, self.shared_router)
+        return (plain and hidden.dtype == torch.bfloat16 and not torch.is_autocast_enabled('cuda')
+                and type(self.f_proj) is nn.Sequential and len(self.f_proj) == 2
+                and type(self.shared_router) is SharedResidualRouter
+                and not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                            for m in containers)
+                and all(t.dtype == torch.bfloat16 and t.device == hidden.device for t in self.parameters())
+                and all(m.bias is None for m in linears[:7])
+                and self._fused_supported(hidden) and self.head_value_width % 8 == 0
+                and self.factor_route_width % 8 == 0)
+
+    def _forward_training(self, hidden: Tensor) -> Tensor:
+        """forward under autograd: one projection of the input by the
+        concatenated weights (so that its gradients are one product each), the
+        controllers and the output interface as one kernel each way."""
+        router, lead = self.shared_router, hidden.shape[:-1]
+        parts = [self.q_proj.weight, self.k_proj.weight, self.v_proj.weight, self.f_proj[0].weight,
+                 self.b_proj.weight, self.w_proj.weight, router.base.weight + router.read_residual.weight,
+                 router.base.weight + router.write_residual.weight, self.output_gate.weight]
+        names = ('q', 'k', 'v', 'f', 'b', 'w', 'read', 'write', 'gate')
+        columns, at = {}, 0
+        for name, part in zip(names, parts):
+            columns[name], at = at, at + part.shape[0]
+        bias = torch.cat([router.base.bias.new_zeros(columns['read']), router.base.bias + router.read_residual.bias,
+                          router.base.bias + router.write_residual.bias, self.output_gate.bias])
+        proj = F.linear(hidden.reshape(-1, self.hidden_size), torch.cat(parts), bias)
+        hv, rw, heads = self.head_value_width, self.factor_route_width, (*lead, self.num_heads)
+        geometry = dict(heads=self.num_heads, bank_size=self.bank_size, head_width=hv, route_width=rw,
+                        qk_norm=self.config.qk_normalization)
+        q, k, v, g, b, w, read, write, gate = _LayerInputs.apply(proj, self.f_proj[1].weight, self.A_log, self.dt_bias,
+                                                                columns, geometry)
+        (ww, wi), (rw_, ri) = self._route_both(write.view(*lead, rw), read.view(*lead, rw))
+        state = self._state_heads(self.materialize_initial_state())
+        operator = bank_training if self.config.routed_decay else role_bank_training
+        raw = operator(q.view(*heads, self.bank_size), k.view(*heads, self.bank_size), v.view(*heads, hv),
+                       g.view(*heads, self.bank_size), b.view(*heads, self.bank_size), w.view(*heads, hv),
+                       wi, ww, ri, rw_, state, self.bank_count, self.bank_size ** -0.5,
+                       compact_replay=self.compact_replay,
+                       state_dtype=getattr(torch, self.config.training_state_dtype))
+        layer = self.config.output_normalization == 'layer'
+        normalized = _OutputInterface.apply(raw.reshape(-1, self.value_width), gate, self.output_norm_weight,
+                                            self.output_norm_bias if layer else None, self.norm_eps,
+                                            'layer' if layer else 'rms')
+        return self.o_proj(normalized.view(*lead, self.value_width))
 
     def _forward_inference(self, hidden: Tensor) -> Tensor:
         """forward without autograd: the projections through one GEMM and the

@@ -672,6 +672,79 @@ def output_epilogue(raw: Tensor, gate: Tensor, weight: Tensor, bias: Tensor | No
     return out
 
 
+def controller_backward(proj: Tensor, f: Tensor, columns: dict, a_log: Tensor, dt_bias: Tensor, grads, *, heads: int,
+                        bank_size: int, head_width: int, route_width: int, qk_norm: str):
+    """Gradients of ``controller_epilogue`` and of the route-score and gate
+    slices of ``proj`` beside it.  ``grads``: those of (q, k, v, g, b, w, read
+    scores, write scores, gate).  Returns (grad_proj, whose f columns are left
+    unset, grad_f [N, H*S] in f's dtype, the FP32 terms [N, 2, H*S] of the
+    gradients of dt_bias and A_log)."""
+    _require_gpu(proj, f, a_log, dt_bias, *grads)
+    n, hs = proj.shape[0], heads * bank_size
+    gq, gk, gv, gg, gb, gw, gread, gwrite, ggate = (_aligned(t) for t in grads)
+    a_log, dt_bias = a_log.contiguous(), _aligned(dt_bias)
+    grad_proj = torch.empty_like(proj)
+    grad_f = torch.empty(n, hs, device=proj.device, dtype=proj.dtype)
+    terms = torch.empty(n, 2, hs, device=proj.device, dtype=torch.float32)
+    args = _lib.ControllerGradArgs()
+    args.proj, args.f, args.a_log, args.dt_bias = (t.data_ptr() for t in (proj, f, a_log, dt_bias))
+    args.grad_q, args.grad_k, args.grad_v, args.grad_b, args.grad_w, args.grad_g = (
+        t.data_ptr() for t in (gq, gk, gv, gb, gw, gg))
+    args.grad_read, args.grad_write, args.grad_gate = (t.data_ptr() for t in (gread, gwrite, ggate))
+    args.grad_proj, args.grad_f, args.grad_terms = grad_proj.data_ptr(), grad_f.data_ptr(), terms.data_ptr()
+    args.tokens, args.proj_stride, args.f_stride = n, proj.stride(0), f.stride(0)
+    args.q_col, args.k_col, args.v_col = columns['q'], columns['k'], columns['v']
+    args.b_col, args.w_col = columns['b'], columns['w']
+    args.read_col, args.write_col, args.gate_col = columns['read'], columns['write'], columns['gate']
+    args.heads, args.bank_size, args.head_width, args.route_width = heads, bank_size, head_width, route_width
+    args.ctrl_dtype, args.param_dtype = _dtype_code(proj.dtype), _dtype_code(a_log.dtype)
+    args.qk_norm = 1 if qk_norm == 'nvidia' else 0
+    _lib.check(_lib.library().bdm_controller_backward(ctypes.byref(args), _stream(proj.device)),
+               'bdm_controller_backward')
+    return grad_proj, grad_f, terms
+
+
+def output_backward(raw: Tensor, gate: Tensor, weight: Tensor, bias: Tensor | None, grad_out: Tensor, *, eps: float,
+                    kind: str):
+    """Gradients (raw, gate, weight, bias or None) of ``output_epilogue`` for
+    BF16 rows; the parameters' in FP32 sums over the tokens, rounded once."""
+    _require_gpu(raw, gate, weight, bias, grad_out)
+    raw, grad_out, weight = _aligned(raw), _aligned(grad_out), _aligned(weight)
+    bias = None if bias is None else _aligned(bias)
+    tokens, width = raw.shape
+    lib = _lib.library()
+    grad_raw, grad_gate = torch.empty_like(raw), torch.empty_like(raw)
+    partials = torch.empty(int(lib.bdm_output_backward_partials(tokens)), 2, width, device=raw.device,
+                           dtype=torch.float32)
+    args = _lib.OutputGradArgs()
+    args.raw, args.gate, args.grad_out = raw.data_ptr(), gate.data_ptr(), grad_out.data_ptr()
+    args.norm_weight, args.norm_bias = weight.data_ptr(), _addr(bias)
+    args.grad_raw, args.grad_gate, args.partials = grad_raw.data_ptr(), grad_gate.data_ptr(), partials.data_ptr()
+    args.tokens, args.gate_stride, args.width = tokens, gate.stride(0), width
+    args.ctrl_dtype, args.param_dtype = _dtype_code(raw.dtype), _dtype_code(weight.dtype)
+    args.norm_kind = 1 if kind == 'layer' else 0
+    args.eps = float(eps)
+    _lib.check(lib.bdm_output_backward(ctypes.byref(args), _stream(raw.device)), 'bdm_output_backward')
+    if bias is None:
+        return grad_raw, grad_gate, partials[:, 0].sum(0).to(weight.dtype), None
+    grad_weight, grad_bias = partials.sum(0).to(weight.dtype)
+    return grad_raw, grad_gate, grad_weight, grad_bias
+
+
+def router_backward(weights: Tensor, indices: Tensor, grad_weights: Tensor, factors: tuple[int, int]) -> Tensor:
+    """Gradient of ``router_select``'s weights with respect to its scores."""
+    _require_gpu(weights, indices, grad_weights)
+    j1, j2 = factors
+    k = weights.shape[-1]
+    grad_weights = grad_weights.to(weights.dtype).contiguous()
+    grad = torch.empty((*weights.shape[:-1], j1 + j2), device=weights.device, dtype=weights.dtype)
+    rows = weights.numel() // k
+    _lib.check(_lib.library().bdm_router_backward(
+        _ptr(weights), _ptr(indices), _ptr(grad_weights), _ptr(grad), rows, j1, j2, k, _dtype_code(weights.dtype),
+        _stream(weights.device)), 'bdm_router_backward')
+    return grad
+
+
 # ---------------------------------------------------------------------------
 # skinny linear maps (decode)
 

@@ -3,8 +3,8 @@
 ``SharedResidualRouter`` keeps the reference module's structure and parameter
 names (implementation/bdm/routing.py:11-68).  ``product_key_route`` keeps the
 signature and outputs of gdn2_banks.py:74-114; the selection runs in the HIP
-router kernel and its backward is the softmax/gather adjoint of the reference's
-autograd graph, written in torch ops on the device.
+router kernel, and its backward, the softmax/gather adjoint of the reference's
+autograd graph, in one kernel.
 """
 
 from __future__ import annotations
@@ -68,15 +68,7 @@ class _ProductKeyRoute(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_weights, grad_indices):
         weights, indices = ctx.saved_tensors
-        j1, j2 = ctx.factors
-        w = weights.float()
-        dw = grad_weights.float()
-        # softmax adjoint, then each selected pair sum feeds one entry of each factor
-        dvals = (w * (dw - (w * dw).sum(-1, keepdim=True))).to(weights.dtype).float()
-        grad = torch.zeros((*weights.shape[:-1], j1 + j2), device=weights.device, dtype=torch.float32)
-        grad[..., :j1].scatter_add_(-1, torch.div(indices, j2, rounding_mode='floor'), dvals)
-        grad[..., j1:].scatter_add_(-1, indices.remainder(j2), dvals)
-        return grad.to(weights.dtype), None, None
+        return ops.router_backward(weights, indices, grad_weights, ctx.factors), None, None
 
 
 def product_key_route(projected: torch.Tensor, *, bank_count: int, selected_banks: int,

@@ -392,6 +392,63 @@ typedef struct bdm_output_args {
 int bdm_output_epilogue(const bdm_output_args *args, void *stream);
 
 /*
+ * Gradients of bdm_controller_epilogue and of the slices beside its columns:
+ * from the forward's proj [tokens, proj_stride] and f [tokens, f_stride] and the
+ * gradients of q, k, b [tokens, H, S], g [tokens, H, S] FP32, v, w [tokens, H,
+ * v], the route scores [tokens, route_width] and the output gate's projection
+ * [tokens, H*v] (all contiguous, 16-byte aligned, BF16),
+ *   grad_proj [tokens, proj_stride]: every column of q, k, v, b, w, read, write
+ *     and gate (the other columns are left alone),
+ *   grad_f [tokens, H*S] BF16, grad_terms [tokens, 2, H*S] FP32: each token's
+ *     d dt_bias and, summing to d A_log over tokens and rows, dg * g.
+ * Columns, strides, H*v and route_width are multiples of 8, bank_size 8, 16 or
+ * 32 (autograd of heads.py:11-22, _parameters.py:189-220).
+ */
+typedef struct bdm_controller_grad_args {
+    const void *proj, *f, *a_log, *dt_bias;
+    const void *grad_q, *grad_k, *grad_v, *grad_b, *grad_w;
+    const float *grad_g;
+    const void *grad_read, *grad_write, *grad_gate;
+    void *grad_proj, *grad_f;
+    float *grad_terms;
+    int64_t tokens, proj_stride, f_stride;
+    int32_t q_col, k_col, v_col, b_col, w_col, read_col, write_col, gate_col;
+    int32_t heads, bank_size, head_width, route_width;
+    int32_t ctrl_dtype, param_dtype, qk_norm;
+} bdm_controller_grad_args;
+
+int bdm_controller_backward(const bdm_controller_grad_args *args, void *stream);
+
+/*
+ * Gradients of bdm_output_epilogue (BF16 rows; _parameters.py:222-232): grad_raw
+ * and grad_gate [tokens, width], and in partials (FP32,
+ * bdm_output_backward_partials(tokens) rows of 2 * width) the partial sums of d
+ * norm_weight, then, for the layer norm, of d norm_bias.  Tensors 16-byte
+ * aligned, gate_stride a multiple of 8, width at most 4096.
+ */
+typedef struct bdm_output_grad_args {
+    const void *raw, *gate, *grad_out;
+    const void *norm_weight, *norm_bias;
+    void *grad_raw, *grad_gate;
+    float *partials;
+    int64_t tokens, gate_stride;
+    int32_t width, ctrl_dtype, param_dtype, norm_kind;
+    float eps;
+} bdm_output_grad_args;
+
+int64_t bdm_output_backward_partials(int64_t tokens);
+int bdm_output_backward(const bdm_output_grad_args *args, void *stream);
+
+/*
+ * Gradient of bdm_router_select's weights with respect to its scores (autograd
+ * of gdn2_banks.py:104-114): weights, indices, grad_weights [rows, selected],
+ * grad_scores [rows, J1 + J2], contiguous.
+ */
+int bdm_router_backward(const void *weights, const int64_t *indices, const void *grad_weights, void *grad_scores,
+                        int64_t rows, int32_t factor_first, int32_t factor_second, int32_t selected, int32_t dtype,
+                        void *stream);
+
+/*
  * Bank occupancy of a write-route table: the Elastic-SDM final-union
  * regularizer applied to banks (reproduction/experiments/
  * elastic_bank_regularizer.py:10-25), reduced over the (sequence, bank)
