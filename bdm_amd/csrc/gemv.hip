@@ -110,16 +110,6 @@ __device__ __forceinline__ void prologue_row(const GemvParams<T> &p, int m, int 
         for (int i = 0; i < NCH; ++i)
 #pragma unroll
             for (int j = 0; j < 8; ++j) xr[i][j] = round_to<T>(xr[i][j] * scale * wt[i][j]);
-    } else if constexpr (PRO == kSwiglu) {
-        const T *row = p.x + int64_t(m) * 2 * p.k;
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            float a[8], b[8];
-            load8<T, true>(row + gs[i] * 8, a);
-            load8<T, true>(row + p.k + gs[i] * 8, b);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xr[i][j] = swiglu_value<T>(a[j], b[j]);
-        }
     } else {
         float gt[NCH][8];
         const T *x = p.x + int64_t(m) * p.k;
@@ -173,13 +163,22 @@ __device__ __forceinline__ void prologue_row(const GemvParams<T> &p, int m, int 
 
 // The GEMV with a prologue: one pass over a row of at most NCH * 512
 // elements.  Every weight load of the wave's R rows is issued first; the
-// input rows are formed in registers while they are in flight.
+// input rows are formed in registers while they are in flight.  SwiGLU, whose
+// exponential and division cost 40 instructions an element, is formed once per
+// workgroup, by its 8 waves together, and read back from LDS: formed by every
+// wave it was longer than the weight's stream (2048 x 5632, one row: 17.5 -> 7.8
+// us); the norms are a few instructions an element and a sum that every wave
+// repeats in the standalone kernel's order.
+template <int PRO>
+constexpr int kGemvWaves = PRO == kSwiglu ? 8 : 4;
+
 template <typename T, int M, int R, int NCH, int PRO>
-__global__ __launch_bounds__(256) void gemv_prologue_kernel(GemvParams<T> p) {
+__global__ __launch_bounds__(kGemvWaves<PRO> *kWave) void gemv_prologue_kernel(GemvParams<T> p) {
+    constexpr bool kShared = PRO == kSwiglu;
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
-    const int64_t row0 = (int64_t(blockIdx.x) * (blockDim.x / kWave) + wave) * R;
-    if (row0 >= p.n) return;
+    const int64_t row0 = (int64_t(blockIdx.x) * kGemvWaves<PRO> + wave) * R;
+    if (!kShared && row0 >= p.n) return;
     const int groups = p.k / 8;
     float wv[NCH][R][8];
 #pragma unroll
@@ -195,7 +194,24 @@ __global__ __launch_bounds__(256) void gemv_prologue_kernel(GemvParams<T> p) {
 #pragma unroll 1
     for (int m = 0; m < M; ++m) {
         float xr[NCH][8];
-        prologue_row<T, NCH, PRO>(p, m, lane, store_sum, xr);
+        if constexpr (kShared) {
+            __shared__ __align__(16) T xs[NCH * kWave * 8];
+            const T *row = p.x + int64_t(m) * 2 * p.k;
+            if (m) __syncthreads();
+            for (int g = threadIdx.x; g < groups; g += kGemvWaves<PRO> * kWave) {
+                float a[8], b[8], x[8];
+                load8<T, true>(row + g * 8, a);
+                load8<T, true>(row + p.k + g * 8, b);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = swiglu_value<T>(a[j], b[j]);
+                store_row<8>(xs + g * 8, x);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < NCH; ++i) load8<T, true>(xs + min(lane + i * kWave, groups - 1) * 8, xr[i]);
+        } else {
+            prologue_row<T, NCH, PRO>(p, m, lane, store_sum, xr);
+        }
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.f;
@@ -319,7 +335,8 @@ int launch_prologue(const GemvParams<T> &p, hipStream_t s) {
     auto go = [&](auto nch_tag, auto r_tag) {
         constexpr int NCH = decltype(nch_tag)::value, R = decltype(r_tag)::value;
         const int64_t waves = (p.n + R - 1) / R;
-        gemv_prologue_kernel<T, M, R, NCH, PRO><<<unsigned((waves + 3) / 4), 256, 0, s>>>(p);
+        constexpr int W = kGemvWaves<PRO>;
+        gemv_prologue_kernel<T, M, R, NCH, PRO><<<unsigned((waves + W - 1) / W), W * kWave, 0, s>>>(p);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;

@@ -158,3 +158,17 @@ def test_lm_fused_decode_equals_unfused(device):
             for a, b in zip(fused, plain):
                 assert torch.equal(a, b), t
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32], ids=['bf16', 'f32'])
+@pytest.mark.parametrize('rows,n,k', [(1, 1, 8), (2, 7, 520), (4, 2050, 2048), (1, 2048, 5632), (3, 13, 6144), (1, 8200, 504)])
+def test_gemv_swiglu_shared_in_lds(device, dtype, rows, n, k):
+    """The SwiGLU row formed once per workgroup: output rows that leave waves of the last workgroup idle, K of one group
+    to the largest; bit for bit the separate kernel's row through the plain GEMV's sums."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(rows * 7 + n)
+    gu = torch.randn(rows, 2 * k, generator=gen).to(dtype).to(device)
+    w = (torch.randn(n, k, generator=gen) * k ** -0.5).to(dtype).to(device)
+    print('CASE gemv swiglu', dtype, rows, n, k, flush=True)
+    y = ops.gemv_fused(gu, w, None, prologue='swiglu')
+    assert torch.equal(y, ops.gemv(ops.swiglu(gu, k), w))
