@@ -2888,6 +2888,11 @@ extern "C" int bdm_forward(const bdm_forward_args *a, void *workspace, size_t wo
     PieceBuffers pb;
     pb.max_pieces = max_pieces(*a);
     if (pb.max_pieces > INT32_MAX / 2) return fail(BDM_ERR_UNSUPPORTED, "forward: too many pieces");
+    // A token writes and reads a bank at most once, so a segment holds at most
+    // 2T events: up to two pieces' worth it runs whole, in one launch instead of
+    // four (two pieces cost two passes over theirs: 512 tokens, H4 v64, 27 + 4.5
+    // + 4 + 4 us), and the combine may run beside it.
+    if (2 * a->time <= 2 * kPieceEvents) pb.max_pieces = 0;
     if (pb.max_pieces) {
         char *at = ws + forward_zbuf_bytes(a);
         const size_t n = size_t(pb.max_pieces);

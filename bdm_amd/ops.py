@@ -30,7 +30,8 @@ def _dtype_code(dtype: torch.dtype) -> int:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle of the current stream, without a Stream object per launch
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_gpu(*tensors: Tensor) -> torch.device:
@@ -55,11 +56,9 @@ def _aligned(t: Tensor) -> Tensor:
     return t
 
 
-def _ptr(t: Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
 def _addr(t: Tensor | None):
+    """A pointer argument: a plain integer (a ctypes object per pointer costs
+    as much as the check around it, and the collector has to visit it)."""
     return None if t is None else t.data_ptr()
 
 
@@ -88,8 +87,8 @@ def router_select(projected: Tensor, *, bank_count: int, selected_banks: int) ->
     weights = torch.empty((*scores.shape[:-1], count), device=scores.device, dtype=scores.dtype)
     indices = torch.empty((*scores.shape[:-1], count), device=scores.device, dtype=torch.int64)
     _lib.check(_lib.library().bdm_router_select(
-        _ptr(scores), _dtype_code(scores.dtype), rows, row_stride, j1, j2, selected_banks,
-        _ptr(weights), _ptr(indices), _stream(scores.device)), 'bdm_router_select')
+        _addr(scores), _dtype_code(scores.dtype), rows, row_stride, j1, j2, selected_banks,
+        _addr(weights), _addr(indices), _stream(scores.device)), 'bdm_router_select')
     return weights, indices
 
 
@@ -121,8 +120,8 @@ def router_select_pair(first: Tensor, second: Tensor, *, bank_count: int,
     outs = [(torch.empty((*lead, count), device=device, dtype=first.dtype),
              torch.empty((*lead, count), device=device, dtype=torch.int64)) for _ in range(2)]
     _lib.check(_lib.library().bdm_router_select_pair(
-        _ptr(views[0][0]), views[0][1], _ptr(views[1][0]), views[1][1], _dtype_code(first.dtype), rows, j1, j2,
-        selected_banks, _ptr(outs[0][0]), _ptr(outs[0][1]), _ptr(outs[1][0]), _ptr(outs[1][1]),
+        _addr(views[0][0]), views[0][1], _addr(views[1][0]), views[1][1], _dtype_code(first.dtype), rows, j1, j2,
+        selected_banks, _addr(outs[0][0]), _addr(outs[0][1]), _addr(outs[1][0]), _addr(outs[1][1]),
         _stream(device)), 'bdm_router_select_pair')
     return outs[0], outs[1]
 
@@ -207,8 +206,8 @@ def dispatch_build(write_indices: Tensor, read_indices: Tensor, bank_count: int)
     ws_bytes = lib.bdm_dispatch_workspace_size_ex(batch, time, bank_count, kw, kr)
     workspace = torch.empty(max(int(ws_bytes), 1), device=device, dtype=torch.uint8)
     _lib.check(lib.bdm_dispatch_build(
-        _ptr(wi), _ptr(ri), batch, time, kw, kr, bank_count, _ptr(order), _ptr(inverse), _ptr(tokens), _ptr(cu),
-        _ptr(status), _ptr(workspace), ws_bytes, _stream(device)), 'bdm_dispatch_build')
+        _addr(wi), _addr(ri), batch, time, kw, kr, bank_count, _addr(order), _addr(inverse), _addr(tokens), _addr(cu),
+        _addr(status), _addr(workspace), ws_bytes, _stream(device)), 'bdm_dispatch_build')
     meta = Dispatch(order, inverse, tokens, cu, status)
     if _validate_routes:
         meta.check_routes()
@@ -250,21 +249,21 @@ def route_dispatch(write_scores: Tensor, read_scores: Tensor, *, bank_count: int
     status = torch.empty(1, device=device, dtype=torch.int32)
     seg_order = torch.empty(batch * bank_count, device=device, dtype=torch.int32)
     args = _lib.RouteDispatchArgs()
-    args.write_scores, args.write_stride = _ptr(views[0][0]), views[0][1]
-    args.read_scores, args.read_stride = _ptr(views[1][0]), views[1][1]
+    args.write_scores, args.write_stride = _addr(views[0][0]), views[0][1]
+    args.read_scores, args.read_stride = _addr(views[1][0]), views[1][1]
     args.score_dtype = _dtype_code(write_scores.dtype)
     args.batch, args.time = batch, time
     args.factor_first, args.factor_second, args.selected = j1, j2, k
-    args.write_weights, args.write_indices = _ptr(ww), _ptr(wi)
-    args.read_weights, args.read_indices = _ptr(rw), _ptr(ri)
-    args.order, args.cu_seqlens, args.status = _ptr(order), _ptr(cu), _ptr(status)
-    args.inverse = _ptr(inverse) if maps else None
-    args.tokens = _ptr(tokens) if maps else None
-    args.segment_order = _ptr(seg_order)
+    args.write_weights, args.write_indices = _addr(ww), _addr(wi)
+    args.read_weights, args.read_indices = _addr(rw), _addr(ri)
+    args.order, args.cu_seqlens, args.status = _addr(order), _addr(cu), _addr(status)
+    args.inverse = _addr(inverse) if maps else None
+    args.tokens = _addr(tokens) if maps else None
+    args.segment_order = _addr(seg_order)
     lib = _lib.library()
     ws_bytes = lib.bdm_route_dispatch_workspace_size(ctypes.byref(args))
     workspace = torch.empty(max(int(ws_bytes), 1), device=device, dtype=torch.uint8)
-    _lib.check(lib.bdm_route_dispatch(ctypes.byref(args), _ptr(workspace), ws_bytes, _stream(device)),
+    _lib.check(lib.bdm_route_dispatch(ctypes.byref(args), _addr(workspace), ws_bytes, _stream(device)),
                'bdm_route_dispatch')
     meta = Dispatch(order, inverse, tokens, cu, status, seg_order)
     if _validate_routes:
@@ -423,7 +422,7 @@ def routed_forward(q, k, v, g, b, w, wi, ww, ri, rw, initial: Tensor, meta: Disp
     elif workspace.dtype != torch.uint8 or workspace.device != x.device or workspace.numel() < ws_bytes \
             or not workspace.is_contiguous():
         raise ValueError(f'workspace must be a contiguous uint8 tensor of at least {ws_bytes} bytes on {x.device}')
-    _lib.check(lib.bdm_forward(ctypes.byref(args), _ptr(workspace), ws_bytes, _stream(x.device)), 'bdm_forward')
+    _lib.check(lib.bdm_forward(ctypes.byref(args), _addr(workspace), ws_bytes, _stream(x.device)), 'bdm_forward')
     return output
 
 
@@ -475,7 +474,7 @@ def routed_backward(x: RoutedInputs, meta: Dispatch, grad_output: Tensor, snapsh
     lib = _lib.library()
     ws_bytes = lib.bdm_backward_workspace_size(ctypes.byref(args))
     workspace = torch.empty(max(int(ws_bytes), 1), device=x.device, dtype=torch.uint8)
-    _lib.check(lib.bdm_backward(ctypes.byref(args), _ptr(workspace), ws_bytes, _stream(x.device)), 'bdm_backward')
+    _lib.check(lib.bdm_backward(ctypes.byref(args), _addr(workspace), ws_bytes, _stream(x.device)), 'bdm_backward')
     return out
 
 
@@ -740,7 +739,7 @@ def router_backward(weights: Tensor, indices: Tensor, grad_weights: Tensor, fact
     grad = torch.empty((*weights.shape[:-1], j1 + j2), device=weights.device, dtype=weights.dtype)
     rows = weights.numel() // k
     _lib.check(_lib.library().bdm_router_backward(
-        _ptr(weights), _ptr(indices), _ptr(grad_weights), _ptr(grad), rows, j1, j2, k, _dtype_code(weights.dtype),
+        _addr(weights), _addr(indices), _addr(grad_weights), _addr(grad), rows, j1, j2, k, _dtype_code(weights.dtype),
         _stream(weights.device)), 'bdm_router_backward')
     return grad
 
@@ -778,7 +777,7 @@ def gemv(x: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     x2 = _aligned(x.reshape(rows, k))
     b = None if bias is None else bias.contiguous()
     y = torch.empty(rows, n, device=x.device, dtype=x.dtype)
-    _lib.check(_lib.library().bdm_gemv(_ptr(x2), _ptr(weight), _ptr(b), _ptr(y), rows, n, k,
+    _lib.check(_lib.library().bdm_gemv(_addr(x2), _addr(weight), _addr(b), _addr(y), rows, n, k,
                                        _dtype_code(x.dtype), _stream(x.device)), 'bdm_gemv')
     return y.view(*lead, n)
 
@@ -865,7 +864,7 @@ def rms_norm(x: Tensor, weight: Tensor, eps: float, residual: Tensor | None = No
     total = None if res is None else torch.empty_like(x)
     width = x.shape[-1]
     _lib.check(_lib.library().bdm_rms_norm(
-        _ptr(x), _ptr(res), _ptr(weight), _ptr(total), _ptr(out), x.numel() // width, width, _dtype_code(x.dtype),
+        _addr(x), _addr(res), _addr(weight), _addr(total), _addr(out), x.numel() // width, width, _dtype_code(x.dtype),
         _dtype_code(weight.dtype), float(eps), _stream(x.device)), 'bdm_rms_norm')
     return out if res is None else (total, out)
 
@@ -888,7 +887,7 @@ def rms_norm_backward(x: Tensor, grad_out: Tensor, weight: Tensor, eps: float):
     grad_x = torch.empty_like(x)
     grad_weight = torch.empty_like(weight)
     _lib.check(lib.bdm_rms_norm_backward(
-        _ptr(x), _ptr(grad_out), _ptr(weight), _ptr(grad_x), _ptr(grad_weight), _ptr(partials), rows, width,
+        _addr(x), _addr(grad_out), _addr(weight), _addr(grad_x), _addr(grad_weight), _addr(partials), rows, width,
         _dtype_code(x.dtype), _dtype_code(weight.dtype), float(eps), _stream(x.device)), 'bdm_rms_norm_backward')
     return grad_x, grad_weight
 
@@ -901,7 +900,7 @@ def swiglu_pair(a: Tensor, b: Tensor) -> Tensor:
         raise ValueError('swiglu_pair takes two BF16/FP32 tensors of one shape')
     a, b = a.contiguous(), b.contiguous()
     out = torch.empty_like(a)
-    _lib.check(_lib.library().bdm_swiglu_pair(_ptr(a), _ptr(b), _ptr(out), a.numel(), _dtype_code(a.dtype),
+    _lib.check(_lib.library().bdm_swiglu_pair(_addr(a), _addr(b), _addr(out), a.numel(), _dtype_code(a.dtype),
                                                _stream(a.device)), 'bdm_swiglu_pair')
     return out
 
@@ -914,7 +913,7 @@ def swiglu_backward(a: Tensor, b: Tensor, grad_out: Tensor):
         raise ValueError('swiglu_backward takes three tensors of one shape and dtype')
     a, b, grad_out = a.contiguous(), b.contiguous(), grad_out.contiguous()
     grad_a, grad_b = torch.empty_like(a), torch.empty_like(b)
-    _lib.check(_lib.library().bdm_swiglu_backward(_ptr(a), _ptr(b), _ptr(grad_out), _ptr(grad_a), _ptr(grad_b),
+    _lib.check(_lib.library().bdm_swiglu_backward(_addr(a), _addr(b), _addr(grad_out), _addr(grad_a), _addr(grad_b),
                                                    a.numel(), _dtype_code(a.dtype), _stream(a.device)),
                'bdm_swiglu_backward')
     return grad_a, grad_b
@@ -928,7 +927,7 @@ def swiglu(gate_up: Tensor, hidden: int) -> Tensor:
         raise ValueError('gate_up must be [..., 2*hidden] with hidden a multiple of 8')
     gate_up = _aligned(gate_up)
     out = torch.empty(*gate_up.shape[:-1], hidden, device=gate_up.device, dtype=gate_up.dtype)
-    _lib.check(_lib.library().bdm_swiglu(_ptr(gate_up), _ptr(out), gate_up.numel() // (2 * hidden), hidden,
+    _lib.check(_lib.library().bdm_swiglu(_addr(gate_up), _addr(out), gate_up.numel() // (2 * hidden), hidden,
                                          _dtype_code(gate_up.dtype), _stream(gate_up.device)), 'bdm_swiglu')
     return out
 
@@ -956,8 +955,8 @@ def bank_occupancy_totals(weights: Tensor, indices: Tensor, bank_count: int, val
     counts = torch.empty(batch, bank_count, device=device, dtype=torch.int32)
     first = torch.empty(batch, bank_count, device=device, dtype=torch.int32) if first_write else None
     _lib.check(_lib.library().bdm_bank_occupancy(
-        _ptr(w), _lib.BDM_BF16 if w is None else _dtype_code(w.dtype), _ptr(mask), _ptr(meta.order), _ptr(meta.cu_seqlens), batch, time, k,
-        bank_count, _ptr(totals), _ptr(counts), _ptr(first), _stream(device)), 'bdm_bank_occupancy')
+        _addr(w), _lib.BDM_BF16 if w is None else _dtype_code(w.dtype), _addr(mask), _addr(meta.order), _addr(meta.cu_seqlens), batch, time, k,
+        bank_count, _addr(totals), _addr(counts), _addr(first), _stream(device)), 'bdm_bank_occupancy')
     if first_write:
         return totals, counts, first
     return totals, counts
@@ -978,6 +977,6 @@ def written_bank_curve(first_write: Tensor, prefixes) -> Tensor:
     first = first_write.contiguous()
     written = torch.empty(batch, ends.numel(), device=device, dtype=torch.int32)
     _lib.check(_lib.library().bdm_written_bank_curve(
-        _ptr(first), batch, banks, _ptr(ends), ends.numel(), _ptr(written), _stream(device)),
+        _addr(first), batch, banks, _addr(ends), ends.numel(), _addr(written), _stream(device)),
         'bdm_written_bank_curve')
     return written
