@@ -33,6 +33,8 @@
 // reference's rounding (role_bank_dispatch.py:99-131); route-weight
 // gradients add the heads' contributions in head order in FP32.
 // token_vjp_kernel: the same for shapes outside that kernel's limits.
+#include <type_traits>
+
 #include "bdm_common.h"
 #include "recurrence_ops.h"
 #include "segment_order.h"
@@ -926,11 +928,15 @@ __device__ __forceinline__ float stride8_sum(float x) {
 }
 
 // One workgroup per token, one wave per head (heads <= 16); S <= 8, KW, KR
-// <= 8 and width <= 64 * CPL.  Lane (j, r) = (lane / 8, lane % 8) holds the
+// <= 8 and width <= 64 * CPL * wph.  Bound: HBM, the FP32 du of a token's
+// writes (537 MB at 8,192 tokens, 8 writes, 2,048 columns).  One load per
+// slot and lane for its adjacent columns, and WAVES: a wide head's waves each
+// load the tiles of their own columns for the S side instead of all of them:
+// 311 -> 180 us there, 113 -> 86 at 8,192 tokens, H8 v128.  Lane (j, r) = (lane / 8, lane % 8) holds the
 // S-side gradients of route slot j, row r; lane l owns value columns
 // l*CPL .. l*CPL + CPL - 1.  The rounding points follow
 // role_bank_dispatch.py:99-131; sums over slots and rows are in FP32.
-template <typename T, int CPL>
+template <typename T, int CPL, bool VEC, bool WAVES>
 __global__ __launch_bounds__(1024) void token_grad_kernel(VjpParams<T> p) {
     constexpr int MAXH = 16, MAXK = 8, MAXW = 16;
     __shared__ float s_route[MAXH][2 * MAXK];  // per head: d(ww) of each write slot, then d(rw)
@@ -955,64 +961,113 @@ __global__ __launch_bounds__(1024) void token_grad_kernel(VjpParams<T> p) {
     const float b0 = to_f32(p.b[row * p.s_real + rr]);
     const float g0 = p.g[row * p.s_real + rr];
     const float pw = to_f32(p.ww[wslot]), pr = to_f32(p.rw[rslot]);
-    const float *wp0 = p.wpart + (wslot * p.heads + head) * 3 * p.s_real + rr;
-    float su = wp0[0], sx = wp0[p.s_real], sp = wp0[2 * p.s_real];
-    float sq = p.rpart[(rslot * p.heads + head) * p.s_real + rr];
+    // a wave's column tile of U, X, P and dq (a head of one wave sums its tiles itself)
+    const auto tile_part = [&](int t, float (&x)[4]) {
+        const float *wp = p.wpart + ((int64_t(t) * wslots + wslot) * p.heads + head) * 3 * p.s_real + rr;
+        x[0] = wp[0], x[1] = wp[p.s_real], x[2] = wp[2 * p.s_real];
+        x[3] = p.rpart[((int64_t(t) * rslots + rslot) * p.heads + head) * p.s_real + rr];
+    };
+    constexpr int kTilesPerWave = 2;  // of 128 columns, of a wave's 256 (WAVES)
+    float part[kTilesPerWave][4];
+    tile_part(WAVES ? min(hw * kTilesPerWave, p.tiles - 1) : 0, part[0]);
+    if constexpr (WAVES) tile_part(min(hw * kTilesPerWave + 1, p.tiles - 1), part[1]);
     const int c0 = (hw * kLanes + lane) * CPL;
     bool live[CPL];
     float v0[CPL], w0[CPL], vwsum[CPL], wsum[CPL], wv[MAXK];
+    // every slot's du and weight requested up front (slots >= KW re-read slot
+    // KW-1: straight-line loads, all in flight together).  VEC: the width is a
+    // multiple of CPL, so a lane's columns are one load and live together.
+    float dus[MAXK][CPL], pws[MAXK];
+    if constexpr (VEC) {
+        const int cc = c0 < p.width ? c0 : p.width - CPL;  // lanes past the width re-read the last columns and drop them
+        load_row<CPL>(p.v + row * p.width + cc, v0);
+        load_row<CPL>(p.w + row * p.width + cc, w0);
+#pragma unroll
+        for (int jj = 0; jj < MAXK; ++jj) {
+            const int64_t slot = token * p.kw + (jj < p.kw ? jj : p.kw - 1);
+            pws[jj] = to_f32(p.ww[slot]);
+            const float *du = p.du + (slot * p.heads + head) * p.width + cc;
+            if constexpr (CPL == 2) {
+                const float2 x = *reinterpret_cast<const float2 *>(du);
+                dus[jj][0] = x.x, dus[jj][1] = x.y;
+            } else {
+                load_row<CPL>(du, dus[jj]);
+            }
+        }
+    } else {
+        int cols[CPL];  // clamped columns
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            cols[c] = min(c0 + c, p.width - 1);
+            v0[c] = to_f32(p.v[row * p.width + cols[c]]);
+            w0[c] = to_f32(p.w[row * p.width + cols[c]]);
+        }
+#pragma unroll
+        for (int jj = 0; jj < MAXK; ++jj) {
+            const int64_t slot = token * p.kw + (jj < p.kw ? jj : p.kw - 1);
+            pws[jj] = to_f32(p.ww[slot]);
+            const float *du = p.du + (slot * p.heads + head) * p.width;
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) dus[jj][c] = du[cols[c]];
+        }
+    }
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
         live[c] = c0 + c < p.width;
-        const int cc = min(c0 + c, p.width - 1);
-        const float vx = to_f32(p.v[row * p.width + cc]), wx = to_f32(p.w[row * p.width + cc]);
-        v0[c] = live[c] ? vx : 0.f;
-        w0[c] = live[c] ? wx : 0.f;
+        v0[c] = live[c] ? v0[c] : 0.f;
+        w0[c] = live[c] ? w0[c] : 0.f;
         vwsum[c] = wsum[c] = 0.f;
     }
-    // every slot's du and weight requested up front (slots >= KW re-read slot
-    // KW-1: straight-line loads, all in flight together)
-    float dus[MAXK][CPL], pws[MAXK];
-    int cols[CPL];  // clamped columns: lanes past the width re-read the last one and drop it
+    float su = part[0][0], sx = part[0][1], sp = part[0][2], sq = part[0][3];
+    if constexpr (WAVES) {
+        // each wave of a head loads its own tiles; the first adds them, in tile order
+        __shared__ float s_part[MAXW * kTilesPerWave][4][kLanes];
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) cols[c] = min(c0 + c, p.width - 1);
+        for (int n = 0; n < kTilesPerWave; ++n)
 #pragma unroll
-    for (int jj = 0; jj < MAXK; ++jj) {
-        const int64_t slot = token * p.kw + (jj < p.kw ? jj : p.kw - 1);
-        pws[jj] = to_f32(p.ww[slot]);
-        const float *du = p.du + (slot * p.heads + head) * p.width;
-#pragma unroll
-        for (int c = 0; c < CPL; ++c) dus[jj][c] = du[cols[c]];
+            for (int x = 0; x < 4; ++x) s_part[wave * kTilesPerWave + n][x][lane] = part[n][x];
+        __syncthreads();
+        if (hw == 0)
+            for (int t = 1; t < p.tiles; ++t) {
+                su += s_part[wave * kTilesPerWave + t][0][lane];
+                sx += s_part[wave * kTilesPerWave + t][1][lane];
+                sp += s_part[wave * kTilesPerWave + t][2][lane];
+                sq += s_part[wave * kTilesPerWave + t][3][lane];
+            }
+    } else {
+        for (int t = 1; t < p.tiles; ++t) {  // column tiles past the first
+            tile_part(t, part[1]);
+            su += part[1][0];
+            sx += part[1][1];
+            sp += part[1][2];
+            sq += part[1][3];
+        }
     }
-    for (int t = 1; t < p.tiles; ++t) {  // column tiles past the first
-        const float *wp = p.wpart + ((int64_t(t) * wslots + wslot) * p.heads + head) * 3 * p.s_real + rr;
-        su += wp[0];
-        sx += wp[p.s_real];
-        sp += wp[2 * p.s_real];
-        sq += p.rpart[((int64_t(t) * rslots + rslot) * p.heads + head) * p.s_real + rr];
-    }
-    // dk = U - eb X ; db = -k X ; dg = P - a X (role_bank_kernel.py:128-135)
-    const float eb = round_to<T>(b0 * pw);
-    const float dk = round_to<T>(su - eb * sx);
-    const float db = round_to<T>(-k0 * sx);
-    const float dg = sp - eb * k0 * sx;
-    // routed decay: the packed gate was g*p (routed_update.py:43-47)
-    const float k_term = wl ? dk : 0.f;
-    const float g_term = wl ? (p.routed_decay ? dg * pw : dg) : 0.f;
-    const float b_term = wl ? round_to<T>(db * pw) : 0.f;
-    const float wb = round_to<T>(group8_sum(wl ? round_to<T>(db * b0) : 0.f));
-    const float dec = group8_sum(wl ? dg * g0 : 0.f);
-    const float dq = round_to<T>(sq);
-    const float q_term = rl ? round_to<T>(dq * pr) : 0.f;
-    const float wr = round_to<T>(group8_sum(rl ? round_to<T>(dq * q0) : 0.f));
-    const float kwsum = stride8_sum(k_term), gsum = stride8_sum(g_term), bsum = stride8_sum(b_term);
-    const float qsum = stride8_sum(q_term);
-    if (hw == 0 && j == 0 && srow) {
-        const int64_t at = row * p.s_real + r;
-        p.dq[at] = from_f32<T>(qsum);
-        p.dk[at] = from_f32<T>(kwsum);
-        p.dg[at] = gsum;
-        p.db[at] = from_f32<T>(bsum);
+    float wb = 0.f, wr = 0.f, dec = 0.f;
+    if (!WAVES || hw == 0) {
+        // dk = U - eb X ; db = -k X ; dg = P - a X (role_bank_kernel.py:128-135)
+        const float eb = round_to<T>(b0 * pw);
+        const float dk = round_to<T>(su - eb * sx);
+        const float db = round_to<T>(-k0 * sx);
+        const float dg = sp - eb * k0 * sx;
+        // routed decay: the packed gate was g*p (routed_update.py:43-47)
+        const float k_term = wl ? dk : 0.f;
+        const float g_term = wl ? (p.routed_decay ? dg * pw : dg) : 0.f;
+        const float b_term = wl ? round_to<T>(db * pw) : 0.f;
+        wb = round_to<T>(group8_sum(wl ? round_to<T>(db * b0) : 0.f));
+        dec = group8_sum(wl ? dg * g0 : 0.f);
+        const float dq = round_to<T>(sq);
+        const float q_term = rl ? round_to<T>(dq * pr) : 0.f;
+        wr = round_to<T>(group8_sum(rl ? round_to<T>(dq * q0) : 0.f));
+        const float kwsum = stride8_sum(k_term), gsum = stride8_sum(g_term), bsum = stride8_sum(b_term);
+        const float qsum = stride8_sum(q_term);
+        if (j == 0 && srow) {
+            const int64_t at = row * p.s_real + r;
+            p.dq[at] = from_f32<T>(qsum);
+            p.dk[at] = from_f32<T>(kwsum);
+            p.dg[at] = gsum;
+            p.db[at] = from_f32<T>(bsum);
+        }
     }
 
     // ---- value columns: the token's write events in route order
@@ -1033,11 +1088,23 @@ __global__ __launch_bounds__(1024) void token_grad_kernel(VjpParams<T> p) {
             }
         }
     }
+    if constexpr (VEC) {
+        if (live[0]) {
+            if constexpr (CPL == 2) {
+                store_cols(p.dv + row * p.width + c0, vwsum);
+                store_cols(p.dw + row * p.width + c0, wsum);
+            } else {
+                store_row<CPL>(p.dv + row * p.width + c0, vwsum);
+                store_row<CPL>(p.dw + row * p.width + c0, wsum);
+            }
+        }
+    } else {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        if (live[c]) {
-            p.dv[row * p.width + c0 + c] = from_f32<T>(vwsum[c]);
-            p.dw[row * p.width + c0 + c] = from_f32<T>(wsum[c]);
+        for (int c = 0; c < CPL; ++c) {
+            if (live[c]) {
+                p.dv[row * p.width + c0 + c] = from_f32<T>(vwsum[c]);
+                p.dw[row * p.width + c0 + c] = from_f32<T>(wsum[c]);
+            }
         }
     }
     const float wv_total = reduce_scatter<MAXK>(wv, lane);
@@ -1345,14 +1412,25 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
     const unsigned blocks = unsigned(p.nt);
     if (token_grad_path(a)) {
         const unsigned threads = unsigned(a.heads * v.wph) * kLanes;
-        if (v.wph > 1)
-            token_grad_kernel<T, 4><<<blocks, threads, 0, stream>>>(v);
-        else if (a.head_width <= kLanes)
-            token_grad_kernel<T, 1><<<blocks, threads, 0, stream>>>(v);
-        else if (a.head_width <= 2 * kLanes)
-            token_grad_kernel<T, 2><<<blocks, threads, 0, stream>>>(v);
+        auto launch = [&](auto cpl, auto waves) {
+            constexpr int CPL = decltype(cpl)::value;
+            constexpr bool WAVES = decltype(waves)::value;
+            // (one column a lane is one load either way)
+            if (CPL > 1 && a.head_width % CPL == 0)
+                token_grad_kernel<T, CPL, (CPL > 1), WAVES><<<blocks, threads, 0, stream>>>(v);
+            else
+                token_grad_kernel<T, CPL, false, WAVES><<<blocks, threads, 0, stream>>>(v);
+        };
+        constexpr std::integral_constant<int, 4> four{};
+        // the head's waves share its tiles of 128 columns (the tiles of the kernels of pairs, up to 8 rows)
+        if (v.wph > 1 && p.tiles <= 2 * v.wph)
+            launch(four, std::true_type{});
+        else if (v.wph > 1 || a.head_width > 2 * kLanes)
+            launch(four, std::false_type{});
+        else if (a.head_width > kLanes)
+            launch(std::integral_constant<int, 2>{}, std::false_type{});
         else
-            token_grad_kernel<T, 4><<<blocks, threads, 0, stream>>>(v);
+            launch(std::integral_constant<int, 1>{}, std::false_type{});
         return check_launch("token_grad_kernel");
     }
     const size_t lds = size_t(a.heads) * size_t(a.write_banks + a.read_banks) * sizeof(float);
