@@ -139,6 +139,65 @@ __device__ __forceinline__ float reduce_scatter(const float (&x)[N], int lane) {
     return out;
 }
 
+// Sums of N values over the lane's 32-lane half partners and row partners: the
+// first two steps of reduce_scatter.  z[i] of row j (lane / 16) is a 16-lane
+// partial of value (N / 4) j + i.
+template <int N>
+__device__ __forceinline__ void sum_rows(const float (&x)[N], float (&z)[N / 4]) {
+    float y[N / 2];
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) y[i] = half_pair_sum(x[i], x[i + N / 2]);
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) z[i] = row_pair_sum(y[i], y[i + N / 4]);
+}
+
+// Totals over 16-lane rows of six values in 13 additions where each value's own
+// row_total takes 4 (24): a DPP addition that writes only some of a row's four
+// banks (of 4 lanes) leaves room in the others for the next value.  A lane at
+// position t of its row returns, for t % 8 = 0, 4 and 1, the total of
+// a[0], a[1] and a[2] (t < 8) or of b[0], b[1] and b[2].  chunk_backward_kernel:
+// 566 -> 546 us at 8,192 tokens, H8 v128, 1,058 -> 1,040 with one head of 2,048
+// columns.  The order of the
+// instructions and the s_nop give the 2 wait states a DPP read of a VGPR needs
+// after a VALU write of it.
+__device__ __forceinline__ float row_totals6(float (&a)[3], const float (&b)[3], int lane) {
+    asm volatile("s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+                 "v_add_f32_dpp %0, %3, %3 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %1, %1, %1 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+                 "v_add_f32_dpp %1, %4, %4 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %2, %2, %2 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+                 "v_add_f32_dpp %2, %5, %5 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+                 "v_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+                 "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 0\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 0\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                 "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2])
+                 : "v"(b[0]), "v"(b[1]), "v"(b[2]));
+    return (lane & 3) == 0 ? a[0] : a[2];
+}
+
+// The same of two values: lanes 0..7 of a row return a's total, 8..15 b's.
+__device__ __forceinline__ float row_totals2(float a, float b) {
+    asm volatile("s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+                 "v_add_f32_dpp %0, %1, %1 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a)
+                 : "v"(b));
+    return a;
+}
+
 // One entry per event of the packed order: token, route slot, is_read and
 // the route weight (FP32 bits), shared by every head.
 template <typename T>
@@ -388,6 +447,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
 #pragma unroll
         for (int c = 0; c < CPL; ++c) dm[r][c] = 0.f;
 
+    // The output of the lane in row_totals6's layout (value 3 j + i of U, X, P by
+    // rows 4 g .. 4 g + 3: j the 16-lane row, i = 0, 1, 2 at positions 0, 4, 1 of
+    // its half g) and in row_totals2's (rows 2 j and 2 j + 1 of dq).
+    const int w_pos = lane & 7, w_out = 3 * (lane >> 4) + (w_pos == 0 ? 0 : (w_pos == 4 ? 1 : 2));
+    const int w_at = (w_out >> 2) * S + 4 * ((lane >> 3) & 1) + (w_out & 3);
+    const bool w_mine = w_pos == 0 || w_pos == 4 || w_pos == 1;
+    const int r_at = 2 * (lane >> 4) + ((lane >> 3) & 1);
+
     // Adjoint of write e, pre-event state st = diag(s) Mh, dm = diag(sigma) dMh:
     //   du = dMh^T (k sigma); u = x - Mh^T (a decay s)
     //   U = sigma (dMh u); X = decay s (Mh du); P = decay s sigma rowsum(dMh o Mh)
@@ -415,6 +482,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
         if (live) *reinterpret_cast<float2 *>(du_lane + uint64_t(slot) * hw) = make_float2(du[0], du[1]);
         float *wp = wp_tile + uint64_t(slot) * uint32_t(p.heads * 3 * S);
         // rows 0..3, then 4..7: red = U[4], X[4], P[4] of the group
+        float z[2][3];
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             float red[12];
@@ -431,13 +499,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
                     dm[r][c] = fmaf(-au[r], du[c], dm[r][c]);
                 }
             }
-            const int pos = lane & 15;
-            const int at = 3 * (lane >> 4) + (pos < 3 ? pos : 0);  // kind = at / 4, row 4g + at % 4
-            const int kind = at >> 2, r = 4 * g + (at & 3);
-            const float o =
-                reduce_scatter<12>(red, lane) * reinterpret_cast<const float *>(&s_rows[e][0])[kScale + kind * S + r];
-            if (pos < 3) wp[kind * S + r] = o;
+            sum_rows<12>(red, z[g]);
         }
+        const float o = row_totals6(z[0], z[1], lane) * reinterpret_cast<const float *>(&s_rows[e][0])[kScale + w_at];
+        if (w_mine) wp[w_at] = o;
     };
     // Adjoint of read e with state st = diag(s) Mh: dq = scale s (Mh dy); dMh += (eq scale / sigma) dy^T.
     auto read_back = [&](int e, int buf, const float (&st)[S][CPL]) {
@@ -457,10 +522,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
 #pragma unroll
             for (int c = 0; c < CPL; ++c) dm[r][c] = fmaf(eq[r], dy[c], dm[r][c]);
         const uint32_t slot = uint32_t(__builtin_amdgcn_readfirstlane(s_meta[buf][e].y));
-        const int pos = lane & 15;
-        const int at = (S / 4) * (lane >> 4) + (pos < S / 4 ? pos : 0);
-        const float o = reduce_scatter<S>(red, lane) * reinterpret_cast<const float *>(&s_rows[e][0])[kScale + at];
-        if (pos < S / 4) rp_tile[uint64_t(slot) * uint32_t(p.heads * S) + at] = o;
+        float z[S / 4];
+        sum_rows<S>(red, z);
+        const float o = row_totals2(z[0], z[1]) * reinterpret_cast<const float *>(&s_rows[e][0])[kScale + r_at];
+        if ((lane & 7) == 0) rp_tile[uint64_t(slot) * uint32_t(p.heads * S) + r_at] = o;
     };
 
     if (count > 0) {
