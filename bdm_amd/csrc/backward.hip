@@ -214,6 +214,12 @@ __global__ __launch_bounds__(256) void event_meta_kernel(const int64_t *order, i
     meta[e] = make_int4(int(token), int(route), rd ? 1 : 0, __float_as_int(weight));
 }
 
+// Lane e's address, uniform over the wave.
+__device__ __forceinline__ const char *lane_ptr(uint64_t x, int e) {
+    const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(x), e), hi = __builtin_amdgcn_readlane(uint32_t(x >> 32), e);
+    return reinterpret_cast<const char *>(uint64_t(hi) << 32 | lo);
+}
+
 template <typename T, typename SNAP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void chunk_backward_kernel(
     BackwardParams<T> p) {
@@ -266,21 +272,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
     auto store_meta = [&](int c, const int4 &m) {
         if (lane < C) s_meta[c & 1][lane] = m;
     };
-    // Loads of chunk c's operands and start state (its meta is in LDS).
+    // Loads of chunk c's operands and start state (its meta is in LDS).  Lane e
+    // (mod C) forms the row addresses of event e, each event takes them with
+    // v_readlane as its loads' scalar base, where each event waited for its LDS
+    // read and formed both addresses in scalar instructions (546 -> 510 us at
+    // 8,192 tokens, H8 v128, 1,040 -> 974 with one head of 2,048 columns).
     auto issue_stage = [&](int c, Staged &sg) {
         const int len = chunk_len(c);
-        const int4 *mt = s_meta[c & 1];
+        const int ev = lane & (C - 1);
+        const int4 m = s_meta[c & 1][ev < len ? ev : len - 1];
+        const uint64_t row = uint64_t(uint32_t(m.x)) * hw;
+        const uint64_t ra = reinterpret_cast<uint64_t>((m.z ? p.dy : p.v) + row);
+        const uint64_t rb = reinterpret_cast<uint64_t>((m.z ? p.dy : p.w) + row);
+        const uint32_t byte = uint32_t(lane_col) * uint32_t(sizeof(T));
 #pragma unroll
         for (int e = 0; e < C; ++e) {
-            const int4 m = mt[e < len ? e : len - 1];
-            const uint64_t row = uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(m.x))) * hw;
-            const bool rd = __builtin_amdgcn_readfirstlane(m.z) != 0;
-            sg.a[e] = P2::load((rd ? p.dy : p.v) + row + lane_col);
-            sg.b[e] = P2::load((rd ? p.dy : p.w) + row + lane_col);
+            sg.a[e] = P2::load(reinterpret_cast<const T *>(lane_ptr(ra, e) + byte));
+            sg.b[e] = P2::load(reinterpret_cast<const T *>(lane_ptr(rb, e) + byte));
         }
         {
-            const int e = lane & (C - 1), rp = (lane >> 4) * 2;
-            const int4 m = mt[e < len ? e : len - 1];
+            const int rp = (lane >> 4) * 2;
             const int64_t at = (int64_t(m.x) * p.heads + head) * S + rp;
             sg.kq = P2::load((m.z ? p.q : p.k) + at);
             sg.bb = P2::load(p.b + at);
@@ -296,22 +307,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
     // Operand rows, columns and the start state of chunk c into LDS.
     auto finish_stage = [&](int c, const Staged &sg) {
         const int len = chunk_len(c);
-        const int4 *mt = s_meta[c & 1];
+        // lane = 16 j + e holds rows 2j, 2j+1 of event e: the scans over a
+        // chunk's events run inside 16-lane rows (DPP row shifts)
+        const int e = lane & (C - 1), rp = (lane >> 4) * 2;
+        const int4 m = s_meta[c & 1][e < len ? e : len - 1];
 #pragma unroll
-        for (int e = 0; e < C; ++e) {
-            const int4 m = mt[e < len ? e : len - 1];
-            const bool rd = __builtin_amdgcn_readfirstlane(m.z) != 0;
-            const float pw = __int_as_float(__builtin_amdgcn_readfirstlane(m.w));
-            ColSlot cs;
-            cs.a = live ? sg.a[e] : P2::zero();
-            cs.b = (live && !rd) ? P2::scaled(sg.b[e], pw) : P2::zero();
-            s_cols[e][lane] = cs;
+        for (int i = 0; i < C; ++i) {
+            ColSlot cs;  // a read's b is not used
+            cs.a = live ? sg.a[i] : P2::zero();
+            cs.b = live ? P2::scaled(sg.b[i], __int_as_float(__builtin_amdgcn_readlane(m.w, i))) : P2::zero();
+            s_cols[i][lane] = cs;
         }
         {
-            // lane = 16 j + e holds rows 2j, 2j+1 of event e: the scans over a
-            // chunk's events run inside 16-lane rows (DPP row shifts)
-            const int e = lane & (C - 1), rp = (lane >> 4) * 2;
-            const int4 m = mt[e < len ? e : len - 1];
             const bool valid = e < len;
             const bool wr = valid && m.z == 0;
             const float pw = __int_as_float(m.w);
@@ -459,7 +466,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
     //   du = dMh^T (k sigma); u = x - Mh^T (a decay s)
     //   U = sigma (dMh u); X = decay s (Mh du); P = decay s sigma rowsum(dMh o Mh)
     //   dMh -= (a / sigma) du^T                      (role_bank_kernel.py:128-138)
-    auto write_back = [&](int e, int buf, const float (&st)[S][CPL]) {
+    auto write_back = [&](int e, int slots, const float (&st)[S][CPL]) {
         float kk[S], ce[S], au[S];
         rows8(e, kKey, kk);
         rows8(e, kErase, ce);
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
             u[c] = fmaf(ew[c], v[c], -erase);
             du[c] = acc;
         }
-        const uint32_t slot = uint32_t(__builtin_amdgcn_readfirstlane(s_meta[buf][e].y));
+        const uint32_t slot = uint32_t(__builtin_amdgcn_readlane(slots, e));
         if (live) *reinterpret_cast<float2 *>(du_lane + uint64_t(slot) * hw) = make_float2(du[0], du[1]);
         float *wp = wp_tile + uint64_t(slot) * uint32_t(p.heads * 3 * S);
         // rows 0..3, then 4..7: red = U[4], X[4], P[4] of the group
@@ -505,7 +512,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
         if (w_mine) wp[w_at] = o;
     };
     // Adjoint of read e with state st = diag(s) Mh: dq = scale s (Mh dy); dMh += (eq scale / sigma) dy^T.
-    auto read_back = [&](int e, int buf, const float (&st)[S][CPL]) {
+    auto read_back = [&](int e, int slots, const float (&st)[S][CPL]) {
         float eq[S];
         rows8(e, kKey, eq);
         const ColSlot cs = s_cols[e][lane];
@@ -521,7 +528,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
         for (int r = 0; r < S; ++r)
 #pragma unroll
             for (int c = 0; c < CPL; ++c) dm[r][c] = fmaf(eq[r], dy[c], dm[r][c]);
-        const uint32_t slot = uint32_t(__builtin_amdgcn_readfirstlane(s_meta[buf][e].y));
+        const uint32_t slot = uint32_t(__builtin_amdgcn_readlane(slots, e));
         float z[S / 4];
         sum_rows<S>(red, z);
         const float o = row_totals2(z[0], z[1]) * reinterpret_cast<const float *>(&s_rows[e][0])[kScale + r_at];
@@ -543,9 +550,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
 #pragma unroll 1
     for (int c = count - 1; c >= 0; --c) {
         __syncthreads();
-        const int buf = c & 1;
         const int len = chunk_len(c);
-        const int4 mine = s_meta[buf][lane & (C - 1)];
+        const int4 mine = s_meta[c & 1][lane & (C - 1)];
         const uint32_t wmask = uint32_t(__ballot(lane < len && mine.z == 0)) & 0xffffu;
         const uint32_t rmask = uint32_t(__ballot(lane < len && mine.z != 0)) & 0xffffu;
         const uint32_t fmask = __builtin_amdgcn_readfirstlane(s_eager) ? wmask : 0u;
@@ -570,8 +576,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
                 for (int cc = 0; cc < CPL; ++cc) st[HALF - 1][r][cc] = m[r][cc];
 #pragma unroll
             for (int e = C - 1; e >= HALF; --e) {
-                if (wmask & (1u << e)) write_back(e, buf, st[e - HALF]);
-                else if (rmask & (1u << e)) read_back(e, buf, st[e - HALF]);
+                if (wmask & (1u << e)) write_back(e, mine.y, st[e - HALF]);
+                else if (rmask & (1u << e)) read_back(e, mine.y, st[e - HALF]);
                 if (fmask & (1u << e)) fold(e, dm);
             }
         }
@@ -597,8 +603,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ch
         if (c >= 1) issue_stage(c - 1, sg);
 #pragma unroll
         for (int e = HALF - 1; e >= 0; --e) {
-            if (wmask & (1u << e)) write_back(e, buf, st[e]);
-            else if (rmask & (1u << e)) read_back(e, buf, st[e]);
+            if (wmask & (1u << e)) write_back(e, mine.y, st[e]);
+            else if (rmask & (1u << e)) read_back(e, mine.y, st[e]);
             if (fmask & (1u << e)) fold(e, dm);
         }
         // the adjoint leaves the chunk in eager form: dm = diag(sigma) dMh
