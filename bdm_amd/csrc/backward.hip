@@ -669,9 +669,10 @@ __device__ __forceinline__ float reduce_columns(const float (&x)[N], int lane, i
 //    are formed once per event, spread over the lanes, not by every lane.
 //  * The sums over columns (U, X, P, dq) are permlane swaps and DPP adds.
 // Bound: instruction issue of the event loop.  Before it, one kernel loaded
-// every operand at its event and reduced by shuffles: 813 -> 115 us at 16,384
-// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 1,934 -> 239
-// us at 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events).  Two
+// every operand at its event and reduced by shuffles: 813 -> 103 us at 16,384
+// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 1,934 -> 229
+// us at 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events); of
+// these, addresses and route slots by readlane took 115 -> 103 and 239 -> 229.  Two
 // row groups at S = 16 (32 columns per wave) double the waves, which the
 // second size needs to fill the chip, and halve a lane's states.
 template <typename T, int S, int RG, int CPL, int C>
@@ -721,17 +722,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
     auto store_meta = [&](int c, const int4 &m) {
         if (lane < C) s_meta[c & 1][lane] = m;
     };
-    // Loads of chunk c's operands and start state (its meta is in LDS).
+    // Loads of chunk c's operands and start state (its meta is in LDS); the
+    // column addresses as in chunk_backward_kernel.
     auto issue_stage = [&](int c, Staged &sg) {
         const int len = chunk_len(c);
         const int4 *mt = s_meta[c & 1];
+        const int ev = lane & (C - 1);
+        const int4 me = mt[ev < len ? ev : len - 1];
+        const int64_t row = int64_t(me.x) * hw;
+        const uint64_t ra = reinterpret_cast<uint64_t>((me.z ? p.dy : p.v) + row);
+        const uint64_t rb = reinterpret_cast<uint64_t>((me.z ? p.dy : p.w) + row);
+        const uint32_t byte = uint32_t(lane_col) * uint32_t(sizeof(T));
 #pragma unroll
         for (int e = 0; e < C; ++e) {
-            const int4 m = mt[e < len ? e : len - 1];
-            const int64_t row = int64_t(__builtin_amdgcn_readfirstlane(m.x)) * hw;
-            const bool rd = __builtin_amdgcn_readfirstlane(m.z) != 0;
-            sg.a[e].load((rd ? p.dy : p.v) + row + lane_col);
-            sg.b[e].load((rd ? p.dy : p.w) + row + lane_col);
+            sg.a[e].load(reinterpret_cast<const T *>(lane_ptr(ra, e) + byte));
+            sg.b[e].load(reinterpret_cast<const T *>(lane_ptr(rb, e) + byte));
         }
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
@@ -760,9 +765,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
     auto finish_stage = [&](int c, const Staged &sg, float (&m0)[R][CPL]) {
         const int len = chunk_len(c);
         const int4 *mt = s_meta[c & 1];
+        const int weight = mt[(lane & (C - 1)) < len ? lane & (C - 1) : len - 1].w;  // lane e: event e's
 #pragma unroll
         for (int e = 0; e < C; ++e) {
-            const float pw = __int_as_float(mt[e < len ? e : len - 1].w);
+            const float pw = __int_as_float(__builtin_amdgcn_readlane(weight, e));
 #pragma unroll
             for (int cc = 0; cc < CPL; ++cc) {  // (the row groups of a column store the same values)
                 s_cols[e][cc][col] = live ? sg.a[e].get(cc) : 0.f;
@@ -827,12 +833,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc) dm[r][cc] = 0.f;
 
-    auto slot_of = [&](int e, int buf, int per_token) {
-        const int4 m = s_meta[buf][e];
-        return int64_t(__builtin_amdgcn_readfirstlane(m.x)) * per_token + __builtin_amdgcn_readfirstlane(m.y);
+    // Route slot of event e from the chunk's metadata, lane e holding event e's.
+    auto slot_of = [&](int e, const int4 &meta, int per_token) {
+        return int64_t(__builtin_amdgcn_readlane(meta.x, e)) * per_token + __builtin_amdgcn_readlane(meta.y, e);
     };
     // Adjoint of write e with the state st before it.
-    auto write_back = [&](int e, int buf, float (&st)[R][CPL]) {
+    auto write_back = [&](int e, const int4 &meta, float (&st)[R][CPL]) {
         float kk[R], dd[R], a[R];
         rows_of(e, kKey, kk);
         rows_of(e, kDecay, dd);
@@ -850,7 +856,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
             u[cc] = fmaf(s_cols[e][CPL + cc][col], s_cols[e][cc][col], -sum_row_groups<RG>(erase));
             du[cc] = sum_row_groups<RG>(acc);
         }
-        const int64_t slot = slot_of(e, buf, p.kw);
+        const int64_t slot = slot_of(e, meta, p.kw);
         if (live && row0 == 0) {
             float *du_row = p.du + slot * hw + head * p.width + col0;
             if constexpr (CPL == 2) *reinterpret_cast<float2 *>(du_row) = make_float2(du[0], du[1]);
@@ -882,12 +888,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         }
     };
     // Adjoint of read e with the state st it read: dq = scale st dy, dm += scale eq dy^T.
-    auto read_back = [&](int e, int buf, const float (&st)[R][CPL]) {
+    auto read_back = [&](int e, const int4 &meta, const float (&st)[R][CPL]) {
         float eq[R], dy[CPL], red[R];
         rows_of(e, kKey, eq);
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc) dy[cc] = s_cols[e][cc][col];
-        float *rp = p.rpart + ((int64_t(tile) * p.nt * p.kr + slot_of(e, buf, p.kr)) * p.heads + head) * p.s_real;
+        float *rp = p.rpart + ((int64_t(tile) * p.nt * p.kr + slot_of(e, meta, p.kr)) * p.heads + head) * p.s_real;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             red[r] = 0.f;
@@ -918,9 +924,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
 #pragma unroll 1
     for (int c = count - 1; c >= 0; --c) {
         __syncthreads();
-        const int buf = c & 1;
         const int len = chunk_len(c);
-        const int4 mine = s_meta[buf][lane & (C - 1)];
+        const int4 mine = s_meta[c & 1][lane & (C - 1)];
         const uint32_t wmask = uint32_t(__ballot(lane < len && mine.z == 0)) & ((1u << C) - 1);
         const uint32_t rmask = uint32_t(__ballot(lane < len && mine.z != 0)) & ((1u << C) - 1);
         float st[C][R][CPL];
@@ -934,8 +939,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         }
 #pragma unroll
         for (int e = C - 1; e >= C / 2; --e) {
-            if (wmask & (1u << e)) write_back(e, buf, st[e]);
-            else if (rmask & (1u << e)) read_back(e, buf, st[e]);
+            if (wmask & (1u << e)) write_back(e, mine, st[e]);
+            else if (rmask & (1u << e)) read_back(e, mine, st[e]);
         }
         // the next chunk's loads, in flight while the first half is differentiated
         int4 meta2 = make_int4(0, 0, 0, 0);
@@ -944,8 +949,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         if (c >= 1) issue_stage(c - 1, sg);
 #pragma unroll
         for (int e = C / 2 - 1; e >= 0; --e) {
-            if (wmask & (1u << e)) write_back(e, buf, st[e]);
-            else if (rmask & (1u << e)) read_back(e, buf, st[e]);
+            if (wmask & (1u << e)) write_back(e, mine, st[e]);
+            else if (rmask & (1u << e)) read_back(e, mine, st[e]);
         }
         __syncthreads();
         if (c >= 2) store_meta(c - 2, meta2);
