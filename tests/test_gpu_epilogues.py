@@ -86,6 +86,30 @@ def test_controller_epilogue_matches_torch_ops(device, qk, bank_size):
         assert rel_err(rr.reshape(ref_rr.shape), ref_rr) < 1e-2 and rel_err(wr.reshape(ref_wr.shape), ref_wr) < 1e-2
 
 
+@pytest.mark.parametrize('bank_size', [8, 16])
+@pytest.mark.parametrize('tokens', [4096, 4097, 4098, 4099])
+def test_controller_epilogue_token_groups_equal_single_tokens(device, tokens, bank_size):
+    """From 4,096 rows a workgroup takes four tokens, and the last one has 4, 1, 2 or 3: each row's arithmetic
+    is the one-token workgroup's, which shorter calls over the same rows run, so every bit is equal."""
+    from bdm_amd import ops
+    layer = _layer(device, torch.bfloat16, 'nvidia', 'layer', bank_size=bank_size)
+    announce('controller epilogue groups', tokens, bank_size)
+    gen = torch.Generator().manual_seed(tokens)
+    with torch.no_grad():
+        cols = layer._fused_weights()[2]
+        width = layer._fused_weights()[0].shape[0]
+        proj = torch.randn(tokens, width, generator=gen).to(torch.bfloat16).to(device)
+        f = torch.randn(tokens, layer.num_heads * bank_size, generator=gen).to(torch.bfloat16).to(device)
+        run = lambda lo, hi: ops.controller_epilogue(  # noqa: E731
+            proj[lo:hi], f[lo:hi], cols, layer.A_log, layer.dt_bias, heads=layer.num_heads, bank_size=bank_size,
+            head_width=layer.head_value_width, qk_norm='nvidia')
+        whole = run(0, tokens)
+        parts = [torch.cat(t) for t in zip(run(0, 2048), run(2048, 4095), run(4095, tokens))]
+        torch.cuda.synchronize()
+    for name, a, b in zip('qkvgbw', whole, parts):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize('qk', ['nvidia', 'original'])
 def test_controller_epilogue_matches_oracle_controllers(device, qk):
     """The fused projection + controller epilogue against the CPU oracle's own
