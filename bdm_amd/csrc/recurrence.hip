@@ -1011,7 +1011,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
 #pragma unroll
                     for (int c = 0; c < CPL; c += 2) round_pair<bf16_t>(h[r][c], h[r][c + 1]);
             }
-            // snapshot of the state before event `base` (see routed_forward_kernel)
+            // snapshot of the state before event `base`
             if (void *snap = lds_ptr(P_SNAP)) {
                 // stage starts are the multiples of snap_interval = kLazyStage
                 const int64_t sslot = (start / NE) + st - 1;
@@ -2372,12 +2372,6 @@ int launch_stage_path(const ForwardParams<T> &p0, const PieceBuffers &pb, int th
     return check_launch("stage_reads_kernel");
 }
 
-// With the stage path (long segments under the rounding policy) its chain of
-// kernels is the critical path, and all of it runs on the caller's stream:
-// the pieces (MODE 3) alone on the device, then the scan, which is bound by
-// its chain's latency, beside the sequential kernel over the other segments
-// (on an auxiliary stream, after the pieces), then the reads and the
-// combine over every column.
 // chain_forward_kernel over the segments longer than p.skip_long: on each XCD
 // at most 128 workgroups (4 per CU, what its LDS holds), fewer where its range
 // cannot hold that many long segments.
@@ -2397,6 +2391,12 @@ int launch_chains(const bdm_forward_args &a, const ForwardParams<T> &p, hipStrea
     return check_launch("chain_forward_kernel");
 }
 
+// With the stage path (long segments under the rounding policy) its chain of
+// kernels is the critical path, and all of it runs on the caller's stream:
+// the pieces (MODE 3) alone on the device, then the scan, which is bound by
+// its chain's latency, beside the sequential kernel over the other segments
+// (on an auxiliary stream, after the pieces), then the reads and the
+// combine over every column.
 template <typename T, int CPL>
 int launch_overlapped_stage(const bdm_forward_args &a, ForwardParams<T> p, const void *kernel, unsigned nseg,
                             int groups, int threads, const T *zbuf, const OverlapAux &ax, const PieceBuffers &pb,
@@ -2626,6 +2626,13 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
                 if (int rc = launch_mode0<T>(kernel, grid, lthreads, ps, stream)) return rc;
                 if (int rc = launch_stage_path<T, CPL>(p, pb, lthreads, int(grid.y), stream)) return rc;
                 return launch_combine<T>(a, zbuf, stream);
+            }
+            // without the auxiliary streams (switched off, or a capture that comes before
+            // they exist) the long segments' chains still run, ahead of the others: the
+            // same results whichever way a call goes
+            if (pb.seg_order && pb.chain_events > 0 && a.read_banks > 0) {
+                p.skip_long = pb.chain_events;
+                if (int rc = launch_chains<T>(a, p, stream)) return rc;
             }
             if (int rc = launch_mode0<T>(kernel, grid, lthreads, p, stream)) return rc;
         }

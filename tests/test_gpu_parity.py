@@ -381,8 +381,9 @@ def test_forward_long_chains_match_oracle(device, heads, v, dtype, decay, monkey
     lengths = sorted((meta.cu_seqlens[1:] - meta.cu_seqlens[:-1]).tolist())
     assert lengths[-1] > 4000 and 2304 < lengths[-2] < 4000 and lengths[0] == 0
     results = []
-    for overlap in ('1', '0'):
-        monkeypatch.setenv('BDM_COMBINE_OVERLAP', overlap)  # 0: one launch over whole segments
+    for order, overlap in (('1', '1'), ('0', '1'), ('1', '0')):  # order 0: one kernel over whole segments
+        monkeypatch.setenv('BDM_SEGMENT_ORDER', order)
+        monkeypatch.setenv('BDM_COMBINE_OVERLAP', overlap)
         final = torch.empty(batch, j, heads, s, v, device=device, dtype=torch.float32)
         y = ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
                                round_interval=16, final_state=final)
@@ -390,7 +391,8 @@ def test_forward_long_chains_match_oracle(device, heads, v, dtype, decay, monkey
         results.append((y, final))
     ref = oracle_reads(q, k, v_, g, b, w, wi, ww, ri, rw, state, j, routed_decay=True, state_dtype=torch.bfloat16,
                        interval=16, return_final=True)
-    for ours, whole, theirs in zip(*results, ref):
+    for ours, whole, serial, theirs in zip(*results, ref):
+        assert torch.equal(ours, serial)
         assert rel_err(ours, theirs) < TOL, rel_err(ours, theirs)
         assert rel_err(ours, whole) < TOL, rel_err(ours, whole)
 
