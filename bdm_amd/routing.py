@@ -4,7 +4,7 @@
 names (implementation/bdm/routing.py:11-68).  ``product_key_route`` keeps the
 signature and outputs of gdn2_banks.py:74-114; the selection runs in the HIP
 router kernel, and its backward, the softmax/gather adjoint of the reference's
-autograd graph, in one kernel.
+autograd graph, in one kernel (in torch ops where it is differentiated again).
 """
 
 from __future__ import annotations
@@ -68,7 +68,21 @@ class _ProductKeyRoute(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_weights, grad_indices):
         weights, indices = ctx.saved_tensors
-        return ops.router_backward(weights, indices, grad_weights, ctx.factors), None, None
+        # under create_graph the kernel's result would end the graph without an error
+        adjoint = _router_adjoint if torch.is_grad_enabled() else ops.router_backward
+        return adjoint(weights, indices, grad_weights, ctx.factors), None, None
+
+
+def _router_adjoint(weights, indices, grad_weights, factors):
+    """ops.router_backward in differentiable torch ops: the softmax adjoint, rounded
+    as the values were, then each selected pair sum feeds one entry of each factor."""
+    j1, j2 = factors
+    w, dw = weights.float(), grad_weights.float()
+    values = (w * (dw - (w * dw).sum(-1, keepdim=True))).to(weights.dtype).float()
+    grad = torch.zeros((*weights.shape[:-1], j1 + j2), device=weights.device, dtype=torch.float32)
+    grad[..., :j1].scatter_add_(-1, torch.div(indices, j2, rounding_mode='floor'), values)
+    grad[..., j1:].scatter_add_(-1, indices.remainder(j2), values)
+    return grad.to(weights.dtype)
 
 
 def product_key_route(projected: torch.Tensor, *, bank_count: int, selected_banks: int,
