@@ -365,9 +365,11 @@ extern "C" int bdm_router_backward(const void *weights, const int64_t *indices, 
                                    int64_t rows, int32_t factor_first, int32_t factor_second, int32_t selected,
                                    int32_t dtype, void *stream) {
     using namespace bdm;
-    if (!weights || !indices || !grad_weights || !grad_scores || rows <= 0 || factor_first <= 0 || factor_second <= 0 ||
-        selected <= 0)
-        return fail(BDM_ERR_INVALID, "router backward: null pointer or bad geometry");
+    if (rows < 0 || factor_first <= 0 || factor_second <= 0 || selected <= 0)
+        return fail(BDM_ERR_INVALID, "router backward: bad geometry");
+    if (rows == 0) return BDM_OK;
+    if (!weights || !indices || !grad_weights || !grad_scores)
+        return fail(BDM_ERR_INVALID, "router backward: null pointer");
     const int64_t blocks = (rows * (int64_t(factor_first) + factor_second) + 255) / 256;
     if (blocks > INT32_MAX) return fail(BDM_ERR_UNSUPPORTED, "router backward: too many rows");
     hipStream_t s = as_stream(stream);

@@ -206,3 +206,11 @@ def test_epilogues_reject_bad_arguments(lib):
     assert lib.bdm_output_epilogue(ctypes.byref(out), None) == -1
     out.width, out.gate_stride, out.norm_kind = 128, 128, 2
     assert lib.bdm_output_epilogue(ctypes.byref(out), None) == -1
+
+
+def test_router_backward_without_rows(lib):
+    """As the forward: no rows are no work (null pointers with them), a negative count is an error."""
+    assert lib.bdm_router_select(None, 0, 0, 16, 8, 8, 4, None, None, None) == 0
+    assert lib.bdm_router_backward(None, None, None, None, 0, 8, 8, 4, 0, None) == 0
+    assert lib.bdm_router_backward(None, None, None, None, -1, 8, 8, 4, 0, None) != 0
+    assert lib.bdm_router_backward(None, None, None, None, 1, 8, 8, 4, 0, None) != 0
