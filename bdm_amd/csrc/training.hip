@@ -48,7 +48,8 @@ __global__ __launch_bounds__(256) void controller_backward_kernel(ControllerGrad
     const T *row = p.proj + token * p.proj_stride;
     T *drow = p.dproj + token * p.proj_stride;
     const int total = p.heads * p.hv, vc = total / 8, rc = p.route_width / 8;
-    const int items = 4 * p.heads + 3 * vc + 2 * rc;
+    const int wide = (p.dgate ? 3 : 2) * vc;  // v, w and, where the projection has it, the gate
+    const int items = 4 * p.heads + wide + 2 * rc;
     const int64_t hs = int64_t(p.heads) * S;
     for (int it = threadIdx.x; it < items; it += int(blockDim.x)) {
         if (it < 4 * p.heads) {
@@ -115,8 +116,8 @@ __global__ __launch_bounds__(256) void controller_backward_kernel(ControllerGrad
             continue;
         }
         const int c = it - 4 * p.heads;
-        const int kind = c < 3 * vc ? c / vc : 3 + (c - 3 * vc) / rc;  // v, w, gate, read, write
-        const int col = (c < 3 * vc ? c % vc : (c - 3 * vc) % rc) * 8;
+        const int kind = c < wide ? c / vc : 3 + (c - wide) / rc;  // v, w, gate, read, write
+        const int col = (c < wide ? c % vc : (c - wide) % rc) * 8;
         if (kind >= 2) {
             const T *src = kind == 2 ? p.dgate + token * total : (kind == 3 ? p.dread : p.dwrite) + token * p.route_width;
             T *dst = drow + (kind == 2 ? p.gate_col : (kind == 3 ? p.read_col : p.write_col));
@@ -290,9 +291,10 @@ extern "C" int bdm_controller_backward(const bdm_controller_grad_args *a, void *
     if (a->tokens <= 0 || a->tokens > INT32_MAX || a->heads <= 0 || a->head_width <= 0 || a->route_width <= 0)
         return fail(BDM_ERR_INVALID, "controller backward: bad geometry");
     const void *ptrs[] = {a->proj, a->f, a->dt_bias, a->grad_q, a->grad_k, a->grad_v, a->grad_b, a->grad_w, a->grad_g,
-                          a->grad_read, a->grad_write, a->grad_gate, a->grad_proj, a->grad_f, a->grad_terms};
+                          a->grad_read, a->grad_write, a->grad_proj, a->grad_f, a->grad_terms};
     for (const void *ptr : ptrs)
         if (!ptr || !aligned(ptr, 16)) return fail(BDM_ERR_INVALID, "controller backward: null or unaligned tensor");
+    if (!aligned(a->grad_gate, 16)) return fail(BDM_ERR_INVALID, "controller backward: unaligned gate gradient");
     const int64_t cols[] = {a->q_col, a->k_col, a->v_col, a->b_col, a->w_col, a->read_col, a->write_col, a->gate_col,
                             a->proj_stride, a->f_stride, int64_t(a->heads) * a->head_width, a->route_width};
     for (int64_t c : cols)

@@ -13,6 +13,7 @@ keep working, ``'role'`` (the reference's GPU backend name).
 
 from __future__ import annotations
 
+import functools
 import hashlib
 import math
 
@@ -28,16 +29,68 @@ from .routing import SharedResidualRouter, product_key_route
 Tensor = torch.Tensor
 
 
+def _unit_rows(value: Tensor, kind: str) -> Tensor:
+    """l2 normalization of q and k: 'nvidia': x * rsqrt(sum x^2 + 1e-6) in FP32
+    (the in-file formula of _parameters.py:219; the reference calls FLA's l2norm
+    on GPU, which is not available here); 'original': F.normalize (:220)."""
+    if kind == 'nvidia':
+        xf = value.float()
+        return (xf * torch.rsqrt(xf.square().sum(-1, keepdim=True) + 1e-6)).to(value.dtype)
+    return F.normalize(value.float(), dim=-1).to(value.dtype)
+
+
+def _controller_ops(q, k, v, f, b, w, a_log, dt_bias, normalize, *, heads, bank_size, head_width):
+    """The controllers (heads.py:11-22) in torch ops of their projections
+    [..., width]: q, k, g, b [..., H, S]; v, w [..., H, v]."""
+    shape = (*q.shape[:-1], heads)
+    q = normalize(F.silu(q).reshape(*shape, bank_size))
+    k = normalize(F.silu(k).reshape(*shape, bank_size))
+    v = F.silu(v).reshape(*shape, head_width)
+    g = -a_log.float().exp()[:, None] * F.softplus((f.float() + dt_bias.float()).reshape(*shape, bank_size))
+    b = b.sigmoid().reshape(*shape, bank_size)
+    w = w.sigmoid().reshape(*shape, head_width)
+    return q, k, v, g, b, w
+
+
+def _output_ops(raw, gate, weight, bias, eps, kind):
+    """norm(raw) * sigmoid(gate), the input of o_proj (_parameters.py:222-232), in torch ops."""
+    if kind == 'layer':
+        normalized = F.layer_norm(raw, (raw.shape[-1],), weight, bias, eps)
+    else:
+        variance = raw.float().square().mean(dim=-1, keepdim=True)
+        normalized = raw * torch.rsqrt(variance + eps).to(raw.dtype)
+        normalized = normalized * weight.to(raw.dtype)
+    return normalized * torch.sigmoid(gate).to(raw.dtype)
+
+
+def _differentiable(grads) -> bool:
+    """Whether a backward has to run in torch ops: its result is differentiated
+    again (create_graph; a kernel's would end the graph), or the gradients are
+    batched (is_grads_batched)."""
+    wrapped = torch._C._functorch
+    return torch.is_grad_enabled() or any(wrapped.is_legacy_batchedtensor(t) or wrapped.is_functorch_wrapped_tensor(t)
+                                          for t in grads)
+
+
+def _torch_gradients(form, inputs, grads):
+    """Gradients of ``form(*inputs)`` by autograd; None for an input that takes none."""
+    create = torch.is_grad_enabled()
+    with torch.enable_grad():
+        outputs = form(*inputs)
+        wanted = [t for t in inputs if t is not None and t.requires_grad]
+        found = iter(torch.autograd.grad(outputs, wanted, grads, create_graph=create))
+    return tuple(next(found) if t is not None and t.requires_grad else None for t in inputs)
+
+
 class _LayerInputs(torch.autograd.Function):
-    """The controllers, route scores and output-gate projection of a layer from
-    one projection [N, P] of its input: f_proj's second factor and the controller
-    epilogue forward; backward, every column of the projection's gradient in one
-    kernel around the two products of that factor."""
+    """The controllers and route scores of a layer from one projection [N, P] of
+    its input: f_proj's second factor and the controller epilogue forward;
+    backward, every column of the projection's gradient in one kernel around the
+    two products of that factor."""
 
     @staticmethod
     def forward(ctx, proj, f_weight, a_log, dt_bias, columns, geometry):
         hv, rw = geometry['head_width'], geometry['route_width']
-        total = geometry['heads'] * hv
         f = F.linear(proj[:, columns['f']:columns['f'] + hv], f_weight)
         controllers = ops.controller_epilogue(proj, f, columns, a_log, dt_bias, heads=geometry['heads'],
                                               bank_size=geometry['bank_size'], head_width=hv,
@@ -45,22 +98,34 @@ class _LayerInputs(torch.autograd.Function):
         ctx.save_for_backward(proj, f, f_weight, a_log, dt_bias)
         ctx.columns, ctx.geometry = columns, geometry
         # copies, not views: an output that shares an input's storage could not be saved or changed in place apart
-        read, write, gate = (proj[:, columns[n]:columns[n] + width].contiguous()
-                             for n, width in (('read', rw), ('write', rw), ('gate', total)))
-        return (*controllers, read, write, gate)
+        scores = (proj[:, columns[n]:columns[n] + rw].contiguous() for n in ('read', 'write'))
+        return (*controllers, *scores)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, *grads):
         proj, f, f_weight, a_log, dt_bias = ctx.saved_tensors
         columns, geometry = ctx.columns, ctx.geometry
-        grad_proj, grad_f, terms = ops.controller_backward(proj, f, columns, a_log, dt_bias, grads, **geometry)
+        if _differentiable(grads):
+            form = functools.partial(_layer_inputs_ops, columns=columns, **geometry)
+            return (*_torch_gradients(form, (proj, f_weight, a_log, dt_bias), grads), None, None)
+        grad_proj, grad_f, terms = ops.controller_backward(proj, f, columns, a_log, dt_bias, (*grads, None), **geometry)
         at = slice(columns['f'], columns['f'] + geometry['head_width'])
         torch.mm(grad_f, f_weight, out=grad_proj[:, at])
         grad_weight = grad_f.t() @ proj[:, at]
         grad_dt, rate = terms.sum(0)
         grad_a = rate.view(geometry['heads'], geometry['bank_size']).sum(-1)
         return grad_proj, grad_weight, grad_a.to(a_log.dtype), grad_dt.to(dt_bias.dtype), None, None
+
+
+def _layer_inputs_ops(proj, f_weight, a_log, dt_bias, *, columns, heads, bank_size, head_width, route_width, qk_norm):
+    """_LayerInputs' forward in torch ops."""
+    keys, total = heads * bank_size, heads * head_width
+    widths = dict(q=keys, k=keys, v=total, f=head_width, b=keys, w=total, read=route_width, write=route_width)
+    part = {n: proj[:, columns[n]:columns[n] + width] for n, width in widths.items()}
+    controllers = _controller_ops(part['q'], part['k'], part['v'], F.linear(part['f'], f_weight), part['b'], part['w'],
+                                  a_log, dt_bias, lambda x: _unit_rows(x, qk_norm), heads=heads, bank_size=bank_size,
+                                  head_width=head_width)
+    return (*controllers, part['read'], part['write'])
 
 
 class _OutputInterface(torch.autograd.Function):
@@ -73,9 +138,11 @@ class _OutputInterface(torch.autograd.Function):
         return ops.output_epilogue(raw, gate, weight, bias, eps=eps, kind=kind)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, grad_out):
         raw, gate, weight, bias = ctx.saved_tensors
+        if _differentiable([grad_out]):
+            form = functools.partial(_output_ops, eps=ctx.eps, kind=ctx.kind)
+            return (*_torch_gradients(form, (raw, gate, weight, bias), grad_out), None, None)
         return (*ops.output_backward(raw, gate, weight, bias, grad_out, eps=ctx.eps, kind=ctx.kind), None, None)
 
 
@@ -248,25 +315,13 @@ class BankedDeltaMemory(nn.Module):
         return (ww, wi), (rw, ri), ops.dispatch_build(wi, ri, self.bank_count)
 
     def _normalize_qk(self, value: Tensor) -> Tensor:
-        """'nvidia': x * rsqrt(sum x^2 + 1e-6) in FP32 (the in-file formula of
-        _parameters.py:219; the reference calls FLA's l2norm on GPU, which is not
-        available here); 'original': F.normalize (:220)."""
-        if self.config.qk_normalization == 'nvidia':
-            xf = value.float()
-            return (xf * torch.rsqrt(xf.square().sum(-1, keepdim=True) + 1e-6)).to(value.dtype)
-        return F.normalize(value.float(), dim=-1).to(value.dtype)
+        return _unit_rows(value, self.config.qk_normalization)
 
     def _controllers(self, hidden: Tensor):
         """Per-head controllers (heads.py:11-22): q,k,g,b [B,T,H,S]; v,w [B,T,H,v]."""
-        shape = (*hidden.shape[:-1], self.num_heads)
-        q = self._normalize_qk(F.silu(self.q_proj(hidden)).reshape(*shape, self.bank_size))
-        k = self._normalize_qk(F.silu(self.k_proj(hidden)).reshape(*shape, self.bank_size))
-        v = F.silu(self.v_proj(hidden)).reshape(*shape, self.head_value_width)
-        g = -self.A_log.float().exp()[:, None] * F.softplus(
-            (self.f_proj(hidden).float() + self.dt_bias.float()).reshape(*shape, self.bank_size))
-        b = self.b_proj(hidden).sigmoid().reshape(*shape, self.bank_size)
-        w = self.w_proj(hidden).sigmoid().reshape(*shape, self.head_value_width)
-        return q, k, v, g, b, w
+        return _controller_ops(self.q_proj(hidden), self.k_proj(hidden), self.v_proj(hidden), self.f_proj(hidden),
+                               self.b_proj(hidden), self.w_proj(hidden), self.A_log, self.dt_bias, self._normalize_qk,
+                               heads=self.num_heads, bank_size=self.bank_size, head_width=self.head_value_width)
 
     # -- fused inference path -----------------------------------------------------------
     def _fused_weights(self):
@@ -347,16 +402,15 @@ class BankedDeltaMemory(nn.Module):
                                          kind='layer' if layer else 'rms')
         return ops.linear(normalized, self.o_proj.weight, self.o_proj.bias).view(*raw.shape[:-1], -1)
 
+    def _output_norm(self):
+        """The output normalization's weight, bias (None for RMS), eps and kind."""
+        layer = self.config.output_normalization == 'layer'
+        return (self.output_norm_weight, self.output_norm_bias if layer else None, self.norm_eps,
+                'layer' if layer else 'rms')
+
     def _project_bank_output(self, hidden: Tensor, raw: Tensor) -> Tensor:
         """LN (or RMS) x sigmoid gate -> o_proj (_parameters.py:222-232)."""
-        if self.config.output_normalization == 'layer':
-            normalized = F.layer_norm(raw, (self.value_width,), self.output_norm_weight,
-                                      self.output_norm_bias, self.norm_eps)
-            return self.o_proj(normalized * torch.sigmoid(self.output_gate(hidden)).to(raw.dtype))
-        variance = raw.float().square().mean(dim=-1, keepdim=True)
-        normalized = raw * torch.rsqrt(variance + self.norm_eps).to(raw.dtype)
-        normalized = normalized * self.output_norm_weight.to(raw.dtype)
-        return self.o_proj(normalized * torch.sigmoid(self.output_gate(hidden)).to(raw.dtype))
+        return self.o_proj(_output_ops(raw, self.output_gate(hidden), *self._output_norm()))
 
     def _state_heads(self, state: Tensor) -> Tensor:
         return state.reshape(self.bank_count, self.num_heads, self.bank_size, self.head_value_width)
@@ -390,8 +444,7 @@ class BankedDeltaMemory(nn.Module):
         exponentials and divisions), 16-byte column groups, and plain projections
         whose own forward and hooks the one product stands for."""
         linears = (self.q_proj, self.k_proj, self.v_proj, self.f_proj[0], self.f_proj[1], self.b_proj, self.w_proj,
-                   self.shared_router.base, self.shared_router.read_residual, self.shared_router.write_residual,
-                   self.output_gate)
+                   self.shared_router.base, self.shared_router.read_residual, self.shared_router.write_residual)
         plain = all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                                                   or m._backward_pre_hooks) for m in linears)
         containers = (self.f_proj, self.shared_router)
@@ -406,25 +459,26 @@ class BankedDeltaMemory(nn.Module):
                 and self.factor_route_width % 8 == 0)
 
     def _forward_training(self, hidden: Tensor) -> Tensor:
-        """forward under autograd: one projection of the input by the
-        concatenated weights (so that its gradients are one product each), the
-        controllers and the output interface as one kernel each way."""
+        """forward under autograd: the projections that the operator reads as one,
+        by the concatenated weights (so that their gradients are one product
+        each), the controllers and the output interface as one kernel each way.
+        The output gate stays a call of its own: its gradients then do not
+        depend on the operator's, as those of o_proj and the norm."""
         router, lead = self.shared_router, hidden.shape[:-1]
         parts = [self.q_proj.weight, self.k_proj.weight, self.v_proj.weight, self.f_proj[0].weight,
                  self.b_proj.weight, self.w_proj.weight, router.base.weight + router.read_residual.weight,
-                 router.base.weight + router.write_residual.weight, self.output_gate.weight]
-        names = ('q', 'k', 'v', 'f', 'b', 'w', 'read', 'write', 'gate')
+                 router.base.weight + router.write_residual.weight]
         columns, at = {}, 0
-        for name, part in zip(names, parts):
+        for name, part in zip(('q', 'k', 'v', 'f', 'b', 'w', 'read', 'write'), parts):
             columns[name], at = at, at + part.shape[0]
         bias = torch.cat([router.base.bias.new_zeros(columns['read']), router.base.bias + router.read_residual.bias,
-                          router.base.bias + router.write_residual.bias, self.output_gate.bias])
+                          router.base.bias + router.write_residual.bias])
         proj = F.linear(hidden.reshape(-1, self.hidden_size), torch.cat(parts), bias)
         hv, rw, heads = self.head_value_width, self.factor_route_width, (*lead, self.num_heads)
         geometry = dict(heads=self.num_heads, bank_size=self.bank_size, head_width=hv, route_width=rw,
                         qk_norm=self.config.qk_normalization)
-        q, k, v, g, b, w, read, write, gate = _LayerInputs.apply(proj, self.f_proj[1].weight, self.A_log, self.dt_bias,
-                                                                columns, geometry)
+        q, k, v, g, b, w, read, write = _LayerInputs.apply(proj, self.f_proj[1].weight, self.A_log, self.dt_bias,
+                                                           columns, geometry)
         (ww, wi), (rw_, ri) = self._route_both(write.view(*lead, rw), read.view(*lead, rw))
         state = self._state_heads(self.materialize_initial_state())
         operator = bank_training if self.config.routed_decay else role_bank_training
@@ -433,10 +487,11 @@ class BankedDeltaMemory(nn.Module):
                        wi, ww, ri, rw_, state, self.bank_count, self.bank_size ** -0.5,
                        compact_replay=self.compact_replay,
                        state_dtype=getattr(torch, self.config.training_state_dtype))
-        layer = self.config.output_normalization == 'layer'
-        normalized = _OutputInterface.apply(raw.reshape(-1, self.value_width), gate, self.output_norm_weight,
-                                            self.output_norm_bias if layer else None, self.norm_eps,
-                                            'layer' if layer else 'rms')
+        gate, raw = self.output_gate(hidden), raw.reshape(*lead, self.value_width)
+        if type(gate) is not Tensor or gate.dtype != raw.dtype or gate.shape != raw.shape:  # a gate of another kind
+            return self.o_proj(_output_ops(raw, gate, *self._output_norm()))
+        normalized = _OutputInterface.apply(*(t.reshape(-1, self.value_width) for t in (raw, gate)),
+                                            *self._output_norm())
         return self.o_proj(normalized.view(*lead, self.value_width))
 
     def _forward_inference(self, hidden: Tensor) -> Tensor:

@@ -675,12 +675,12 @@ def controller_backward(proj: Tensor, f: Tensor, columns: dict, a_log: Tensor, d
                         bank_size: int, head_width: int, route_width: int, qk_norm: str):
     """Gradients of ``controller_epilogue`` and of the route-score and gate
     slices of ``proj`` beside it.  ``grads``: those of (q, k, v, g, b, w, read
-    scores, write scores, gate).  Returns (grad_proj, whose f columns are left
-    unset, grad_f [N, H*S] in f's dtype, the FP32 terms [N, 2, H*S] of the
-    gradients of dt_bias and A_log)."""
+    scores, write scores, gate; the last None where ``proj`` has no gate).
+    Returns (grad_proj, whose f columns are left unset, grad_f [N, H*S] in f's
+    dtype, the FP32 terms [N, 2, H*S] of the gradients of dt_bias and A_log)."""
     _require_gpu(proj, f, a_log, dt_bias, *grads)
     n, hs = proj.shape[0], heads * bank_size
-    gq, gk, gv, gg, gb, gw, gread, gwrite, ggate = (_aligned(t) for t in grads)
+    gq, gk, gv, gg, gb, gw, gread, gwrite, ggate = (None if t is None else _aligned(t) for t in grads)
     a_log, dt_bias = a_log.contiguous(), _aligned(dt_bias)
     grad_proj = torch.empty_like(proj)
     grad_f = torch.empty(n, hs, device=proj.device, dtype=proj.dtype)
@@ -689,12 +689,12 @@ def controller_backward(proj: Tensor, f: Tensor, columns: dict, a_log: Tensor, d
     args.proj, args.f, args.a_log, args.dt_bias = (t.data_ptr() for t in (proj, f, a_log, dt_bias))
     args.grad_q, args.grad_k, args.grad_v, args.grad_b, args.grad_w, args.grad_g = (
         t.data_ptr() for t in (gq, gk, gv, gb, gw, gg))
-    args.grad_read, args.grad_write, args.grad_gate = (t.data_ptr() for t in (gread, gwrite, ggate))
+    args.grad_read, args.grad_write, args.grad_gate = gread.data_ptr(), gwrite.data_ptr(), _addr(ggate)
     args.grad_proj, args.grad_f, args.grad_terms = grad_proj.data_ptr(), grad_f.data_ptr(), terms.data_ptr()
     args.tokens, args.proj_stride, args.f_stride = n, proj.stride(0), f.stride(0)
     args.q_col, args.k_col, args.v_col = columns['q'], columns['k'], columns['v']
     args.b_col, args.w_col = columns['b'], columns['w']
-    args.read_col, args.write_col, args.gate_col = columns['read'], columns['write'], columns['gate']
+    args.read_col, args.write_col, args.gate_col = columns['read'], columns['write'], columns.get('gate', 0)
     args.heads, args.bank_size, args.head_width, args.route_width = heads, bank_size, head_width, route_width
     args.ctrl_dtype, args.param_dtype = _dtype_code(proj.dtype), _dtype_code(a_log.dtype)
     args.qk_norm = 1 if qk_norm == 'nvidia' else 0

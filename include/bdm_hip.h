@@ -398,7 +398,7 @@ int bdm_output_epilogue(const bdm_output_args *args, void *stream);
  * v], the route scores [tokens, route_width] and the output gate's projection
  * [tokens, H*v] (all contiguous, 16-byte aligned, BF16),
  *   grad_proj [tokens, proj_stride]: every column of q, k, v, b, w, read, write
- *     and gate (the other columns are left alone),
+ *     and, unless grad_gate is NULL, gate (the other columns are left alone),
  *   grad_f [tokens, H*S] BF16, grad_terms [tokens, 2, H*S] FP32: each token's
  *     d dt_bias and, summing to d A_log over tokens and rows, dg * g.
  * Columns, strides, H*v and route_width are multiples of 8, bank_size 8, 16 or

@@ -107,9 +107,115 @@ def test_router_backward(device, banks, selected, dtype):
     assert rel_err(grad, ref) < (4e-2 if dtype == torch.bfloat16 else 1e-5)
 
 
+LAYERS = [  # config class, heads, rows, options
+    ('BSDMConfig', 2, 8, {}),
+    ('BSDMConfig', 1, 16, {}),
+    ('BSDMConfig', 4, 8, dict(output_bias=False, qk_normalization='original')),
+    ('BDMConfig', 2, 8, {}),
+    ('BDMConfig', 1, 32, dict(output_normalization='layer', routed_decay=True))]
+
+
+def trained_layer(device, kind, heads, rows, options, tokens=50):
+    """A BF16 layer and its input.  Input and router are small multiples of powers of two, so that the route scores are
+    the same however a product sums them: no route depends on the path."""
+    import bdm_amd
+    cfg = getattr(bdm_amd, kind)(dim=64, bank_count=64, bank_size=rows, selected_banks=4, value_width=128, num_heads=heads,
+                                 **options)
+    gen = torch.Generator().manual_seed(rows + heads)
+    layer = bdm_amd.BankedDeltaMemory(cfg, seed=3)
+    with torch.no_grad():
+        for p in layer.shared_router.parameters():
+            p.copy_(torch.randint(-32, 33, p.shape, generator=gen) / 128)
+        layer.dt_bias += 3  # decays that are felt within the sequence
+        for p in (layer.output_norm_weight, getattr(layer, 'output_norm_bias', None), layer.output_gate.bias):
+            if p is not None:
+                p += 0.2 * torch.randn(p.shape, generator=gen)
+    layer = layer.to(device=device, dtype=torch.bfloat16)
+    x = (torch.randint(-8, 9, (2, tokens, 64), generator=gen) / 4).to(torch.bfloat16).to(device).requires_grad_(True)
+    dy = torch.randn(2, tokens, 64, generator=gen).to(torch.bfloat16).to(device)
+    return layer, x, dy
+
+
+def both_paths(layer, x, work):
+    """``work()`` with the fused training path and, behind a hook that changes nothing, with the modules' own calls."""
+    assert layer._fused_training_supported(x)
+    fused = work()
+    handle = layer.v_proj.register_forward_hook(lambda m, i, o: None)
+    assert not layer._fused_training_supported(x)
+    plain = work()
+    handle.remove()
+    torch.cuda.synchronize()
+    return fused, plain
+
+
+def norm_err(a, b):
+    a, b = a.double(), b.double()
+    return float((a - b).norm() / b.norm().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize('kind,heads,rows,options', LAYERS)
+def test_layer_gradients(device, kind, heads, rows, options):
+    """The fused training path against autograd of the modules' own calls: the output and the gradients of the input
+    and of every parameter.  Both round to BF16 at up to ten places between a parameter and the loss, 2^-9 each and
+    independent of one another: 2.5e-2 in the 2-norm is four times their root sum (each was 0.2 to 1.4 % off float64)."""
+    layer, x, dy = trained_layer(device, kind, heads, rows, options)
+    names = [n for n, _ in layer.named_parameters()] + ['input']
+    leaves = [*layer.parameters(), x]
+    print('CASE layer gradients', kind, heads, rows, options, flush=True)
+
+    def gradients():
+        y = layer(x)
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+
+    fused, plain = both_paths(layer, x, gradients)
+    assert len(names) >= 22
+    for name, ours, theirs in zip(['output', *names], fused, plain):
+        assert ours.dtype == theirs.dtype and ours.shape == theirs.shape
+        assert float(theirs.double().norm()) > 0, name
+        assert norm_err(ours, theirs) < 2.5e-2, (name, norm_err(ours, theirs))
+
+
+def test_layer_second_derivatives(device):
+    """Gradients of gradients reach what they reach without the fused path: those of the parameters behind the operator
+    are whole, those that pass the operator's own backward keep its first-order part."""
+    layer, x, dy = trained_layer(device, 'BSDMConfig', 2, 8, {})
+    behind = [layer.o_proj.weight, layer.output_norm_weight, layer.output_norm_bias, layer.output_gate.weight]
+    leaves = [*behind, layer.output_gate.bias, layer.q_proj.weight, layer.f_proj[1].weight, layer.A_log,
+              layer.shared_router.base.weight, x]
+    print('CASE second derivatives', flush=True)
+
+    def penalized(first):
+        def run():
+            loss = (layer(x).float() * dy.float()).sum()
+            grads = torch.autograd.grad(loss, first, create_graph=True)
+            penalty = sum(g.float().square().sum() for g in grads)
+            assert all(g.requires_grad for g in grads)
+            return torch.autograd.grad(penalty, leaves, allow_unused=True)
+        return run
+
+    for first in (behind, [x]):
+        fused, plain = both_paths(layer, x, penalized(first))
+        for leaf, ours, theirs in zip(leaves, fused, plain):
+            assert (ours is None) == (theirs is None), leaf.shape
+            if theirs is not None:
+                # twice the roundings of a first gradient, and the penalty doubles their share
+                assert norm_err(ours, theirs) < 5e-2, (leaf.shape, norm_err(ours, theirs))
+
+
+def test_layer_batched_gradients(device):
+    """Several output gradients at once (is_grads_batched), for the parameters whose gradients don't pass the operator."""
+    layer, x, dy = trained_layer(device, 'BSDMConfig', 2, 8, {})
+    leaves = [layer.o_proj.weight, layer.output_norm_weight, layer.output_gate.weight]
+    several = torch.stack([dy, -0.5 * dy, dy.flip(1)])
+    print('CASE batched gradients', flush=True)
+    fused, plain = both_paths(layer, x, lambda: torch.autograd.grad(layer(x), leaves, several, is_grads_batched=True))
+    for ours, theirs in zip(fused, plain):
+        assert ours.shape == theirs.shape and norm_err(ours, theirs) < 2.5e-2
+
+
 def test_training_forward_keeps_module_hooks(device):
-    """A projection that is hooked or replaced is called as a module, with the same gradients to BF16 rounding (read
-    and write routes from one projection or several agree here: well separated scores)."""
+    """A projection that is hooked is called as a module, with the same output to BF16 rounding (read and write routes
+    from one projection or several agree here: well separated scores)."""
     from bdm_amd import BSDMConfig, BankedDeltaMemory
     cfg = BSDMConfig(dim=64, bank_count=64, bank_size=8, selected_banks=4, value_width=128, num_heads=2)
     layer = BankedDeltaMemory(cfg, seed=3).to(device=device, dtype=torch.bfloat16)
