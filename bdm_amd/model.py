@@ -146,6 +146,10 @@ class _OutputInterface(torch.autograd.Function):
         return (*ops.output_backward(raw, gate, weight, bias, grad_out, eps=ctx.eps, kind=ctx.kind), None, None)
 
 
+# The methods of a layer whose work its fused training path does in another way.
+_TRAINING_METHODS = ('bank_reads', '_controllers', '_normalize_qk', '_route_projections', '_project_bank_output')
+
+
 class BankedDeltaMemory(nn.Module):
     """Shared-residual product routing around dense GDN2 memory banks."""
 
@@ -441,22 +445,31 @@ class BankedDeltaMemory(nn.Module):
     def _fused_training_supported(self, hidden: Tensor) -> bool:
         """Whether the autograd forward may project once and run the fused
         controller and output kernels: BF16 throughout (FP32 keeps torch's exact
-        exponentials and divisions), 16-byte column groups, and plain projections
-        whose own forward and hooks the one product stands for."""
-        linears = (self.q_proj, self.k_proj, self.v_proj, self.f_proj[0], self.f_proj[1], self.b_proj, self.w_proj,
-                   self.shared_router.base, self.shared_router.read_residual, self.shared_router.write_residual)
-        plain = all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                                                  or m._backward_pre_hooks) for m in linears)
-        containers = (self.f_proj, self.shared_router)
-        return (plain and hidden.dtype == torch.bfloat16 and not torch.is_autocast_enabled('cuda')
-                and type(self.f_proj) is nn.Sequential and len(self.f_proj) == 2
-                and type(self.shared_router) is SharedResidualRouter
-                and not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                            for m in containers)
-                and all(t.dtype == torch.bfloat16 and t.device == hidden.device for t in self.parameters())
-                and all(m.bias is None for m in linears[:7])
-                and self._fused_supported(hidden) and self.head_value_width % 8 == 0
-                and self.factor_route_width % 8 == 0)
+        exponentials and divisions), 16-byte column groups, and no call that the
+        one product stands for is another than this file's: the projections are
+        plain linear maps of plain tensors without hooks (their own or global
+        ones) or a forward of their instance, and neither a subclass nor the
+        instance has methods of its own for the path."""
+        def plain(m, kind):
+            return type(m) is kind and 'forward' not in m.__dict__ and not (
+                m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+        if (hidden.dtype != torch.bfloat16 or torch.is_autocast_enabled('cuda') or not self._fused_supported(hidden)
+                or self.head_value_width % 8 or self.factor_route_width % 8 or nn.modules.module._has_any_global_hook()
+                or any(getattr(type(self), n) is not getattr(BankedDeltaMemory, n) or n in self.__dict__
+                       for n in _TRAINING_METHODS)):
+            return False
+        pair, router = self.f_proj, self.shared_router
+        if not (plain(pair, nn.Sequential) and len(pair) == 2 and plain(router, SharedResidualRouter)
+                and not {'read', 'write'} & router.__dict__.keys()):
+            return False
+        unbiased = (self.q_proj, self.k_proj, self.v_proj, *pair, self.b_proj, self.w_proj)
+        biased = (router.base, router.read_residual, router.write_residual)
+        return (all(plain(m, nn.Linear) and m.bias is None for m in unbiased)
+                and all(plain(m, nn.Linear) and m.bias is not None for m in biased)
+                and type(hidden) in (Tensor, nn.Parameter)
+                and all(type(t) in (Tensor, nn.Parameter) and t.dtype == torch.bfloat16 and t.device == hidden.device
+                        for t in self.parameters()))
 
     def _forward_training(self, hidden: Tensor) -> Tensor:
         """forward under autograd: the projections that the operator reads as one,

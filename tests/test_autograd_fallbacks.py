@@ -49,3 +49,60 @@ def test_route_weights_second_derivative(router, banks, selected):
     ref = penalized(leaf, values.softmax(-1))
     # FP32 sums of at most 2K terms of the two adjoints: a few dozen roundings of 2^-24 of the largest term
     torch.testing.assert_close(penalized(scores, weights).double(), ref, rtol=0, atol=64 * 2 ** -24 * 100)
+
+
+@pytest.fixture
+def layer():
+    from bdm_amd import BSDMConfig, BankedDeltaMemory
+    config = BSDMConfig(dim=64, bank_count=64, bank_size=8, selected_banks=4, value_width=128, num_heads=2)
+    return BankedDeltaMemory(config, seed=3).to(torch.bfloat16)
+
+
+def subclass(layer, name):
+    base = type(layer)
+    layer.__class__ = type('Own', (base,), {name: lambda self, *args: getattr(base, name)(self, *args)})
+
+
+def replace_forward(module):
+    module.forward = lambda x, forward=module.forward: forward(x)
+
+
+class Marked(torch.Tensor):
+    """A tensor type of its own, as quantized or sharded weights are."""
+
+
+OWN_BEHAVIOUR = {
+    'forward of an instance': lambda m: replace_forward(m.q_proj),
+    'forward of the factor pair': lambda m: replace_forward(m.f_proj),
+    'own read map': lambda m: setattr(m.shared_router, 'read', m.shared_router.read),
+    'hook': lambda m: m.w_proj.register_forward_hook(lambda *a: None),
+    'another module': lambda m: setattr(m, 'v_proj', torch.nn.Sequential(m.v_proj)),
+    'another factor pair': lambda m: setattr(m, 'f_proj', torch.nn.Linear(64, 16, bias=False, dtype=torch.bfloat16)),
+    'another router': lambda m: setattr(m, 'shared_router', torch.nn.Identity()),
+    'method of the instance': lambda m: setattr(m, '_controllers', m._controllers),
+    'another weight type': lambda m: setattr(m.k_proj, 'weight', torch.nn.Parameter(
+        m.k_proj.weight.detach().as_subclass(Marked))),
+    **{'subclass ' + n: lambda m, n=n: subclass(m, n)
+       for n in ('bank_reads', '_controllers', '_route_projections', '_project_bank_output', '_normalize_qk')},
+}
+
+
+@pytest.mark.parametrize('change', OWN_BEHAVIOUR)
+def test_training_path_gives_way_to_own_behaviour(layer, change):
+    """Calls that the fused training path would pass by keep the modules' path."""
+    x = torch.zeros(1, 3, 64, dtype=torch.bfloat16)
+    assert layer._fused_training_supported(x)
+    OWN_BEHAVIOUR[change](layer)
+    assert not layer._fused_training_supported(x)
+
+
+@pytest.mark.parametrize('register', ['register_module_forward_hook', 'register_module_forward_pre_hook',
+                                      'register_module_full_backward_hook'])
+def test_training_path_gives_way_to_global_hooks(layer, register):
+    x = torch.zeros(1, 3, 64, dtype=torch.bfloat16)
+    handle = getattr(torch.nn.modules.module, register)(lambda *a: None)
+    try:
+        assert not layer._fused_training_supported(x)
+    finally:
+        handle.remove()
+    assert layer._fused_training_supported(x)
