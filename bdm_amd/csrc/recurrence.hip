@@ -588,11 +588,29 @@ __device__ __forceinline__ void load_vec4(const T *p, uint2 &out) {
 }
 __device__ __forceinline__ void load_vec4(const float *p, float4 &out) { out = *reinterpret_cast<const float4 *>(p); }
 
+// The segments longer than p.skip_long that lead the order of the range at
+// `base`: chain_forward_kernel's.  Of the longest-first order these are all long
+// segments; of a caller's other order MODE 4 runs the rest, so that each segment
+// is run once whatever the order.  (64 segments at a time; few are long.)
+template <typename T>
+__device__ __forceinline__ int leading_long(const ForwardParams<T> &p, int base) {
+    const int range = p.nseg / 8;
+    for (int first = 0; first < range; first += kWave) {
+        const int at = first + int(threadIdx.x) % kWave;
+        const int seg = p.seg_order[base + min(at, range - 1)];
+        const uint64_t others = __ballot(at >= range || p.cu[seg + 1] - p.cu[seg] <= p.skip_long);
+        if (others) return first + __builtin_ctzll(others);
+    }
+    return range;
+}
+
 // HB heads per workgroup of 32 * HB threads (HB = 2: one wave, so its
 // barriers never wait for other waves; HB = 8 for narrow heads, where the
 // value columns of 8 heads fit in 256 lanes).
 //
-// MODE 0 runs whole segments (one workgroup each).  Under the prefill policy
+// MODE 0 runs whole segments (one workgroup each), MODE 4 those that
+// chain_forward_kernel leaves (leading_long; as a test in MODE 0 it took 1.6 us of a
+// 422 us forward without chains).  Under the prefill policy
 // (no rounding inside the recurrence, no snapshots) a segment is an affine
 // map of its start state, M_end = P M_start + R, so segments longer than
 // kPieceEvents are cut into pieces to balance skewed routing:
@@ -634,6 +652,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
     static_assert(!BUF || (std::is_same<T, bf16_t>::value && CPL == 4), "buffer form: BF16, 4 columns per lane");
     constexpr int S = 8;
     constexpr int NE = kLazyStage;
+    constexpr bool kWhole = MODE == 0 || MODE == 4;
     // Event metadata ring: stage s lives in slot s % kRing.  The packed order
     // is loaded and decoded kGroup stages at a time (64 events, one per lane
     // of wave 0), two groups ahead of their use.
@@ -665,21 +684,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
     // Blocks reach the XCDs round-robin in dispatch order (x fastest).  With
     // p.seg_order the k-th segment block of XCD x takes item k of that XCD's
     // range: rounds of head groups (order_item), segments longest first.
+    int rank = 0;
     auto ordered_segment = [&](int64_t k, int gpr) {
         const int range = p.nseg / 8;
-        int rank;
         order_item(k / 8, range, int(gridDim.y), gpr, rank, group);
         return p.seg_order[int(k % 8) * range + rank];
     };
-    if constexpr (MODE == 0) {
+    if constexpr (kWhole) {
         if (p.seg_order) {
             seg = ordered_segment(int64_t(blockIdx.y) * gridDim.x + blockIdx.x, p.order_gpr);
         } else {
             seg = p.xcd_remap ? int((block % 8) * (p.nseg / 8) + block / 8) : block;
         }
         group += p.group_base;
-        // the stage path runs the long segments (the whole workgroup leaves together)
-        if (p.skip_long && p.cu[seg + 1] - p.cu[seg] > p.skip_long) return;
+        // the stage path or the chains run the long segments (the whole workgroup leaves together)
+        if (p.skip_long && p.cu[seg + 1] - p.cu[seg] > p.skip_long) {
+            if constexpr (MODE == 0) return;
+            else if (rank < leading_long(p, int(block % 8) * (p.nseg / 8))) return;
+        }
     } else if constexpr (MODE == 3) {
         is_piece = true;  // every piece of every long segment, one per block
     } else if constexpr (MODE == 1) {
@@ -755,7 +777,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
     // MODE 3: the slot of the piece's first stage (stage k of segment s has
     // slot cu[s] / 16 + s + k, distinct over all segments' stages)
     const int64_t stage_slot0 = start / NE + seg + int64_t(piece) * (kPieceEvents / NE);
-    if constexpr (MODE != 0) {
+    if constexpr (!kWhole) {
         if (pieces > 1) {
             start += int64_t(piece) * kPieceEvents;
             end = min(end, start + kPieceEvents);
@@ -763,7 +785,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
     }
     const int64_t write_events = p.nt * p.kw;
     const int64_t events = p.nt * (p.kw + p.kr);
-    const bool rounding = MODE == 0 && p.round_interval > 0;
+    const bool rounding = kWhole && p.round_interval > 0;
     const int nstages = int((end - start + NE - 1) / NE);
 
     // Pointers used once per stage or less live in LDS rather than in SGPRs:
@@ -1139,7 +1161,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
                 fetch_token(__builtin_amdgcn_readlane(m_wtok, k < nw ? k : nw - 1), vv, ww);
             };
             int i = 0;
-            if constexpr (MODE == 0) {
+            if constexpr (kWhole) {
                 if (nw > 0) {
                     fetch_write(0, va, wa);
                     fetch_write(1, vb, wb);
@@ -1588,21 +1610,20 @@ __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg
 
 // One workgroup of 2 NC + 1 waves per (long segment, virtual head, 64 NC
 // columns): waves 0 .. NC-1 consume, the others produce.  Items of an XCD: its
-// segments longest first; a workgroup stops at the first segment that is not
-// long.
+// segments longest first, up to the first that is not long (leading_long).
 template <typename T, int NC>
 __global__ __launch_bounds__(kWave *(2 * NC + 1)) __attribute__((amdgpu_waves_per_eu(5, 8))) void chain_forward_kernel(
     ForwardParams<T> p) {
     __shared__ __align__(16) ChainLds<NC> lds;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    const int base = int(blockIdx.x % 8) * (p.nseg / 8), count = leading_long(p, base);
     auto each_item = [&](auto run) {  // (a loop per role: no role's loop invariants live through another's)
-        const int range = p.nseg / 8, parts = p.width / (NC * kWave), per_seg = p.heads * parts;
+        const int parts = p.width / (NC * kWave), per_seg = p.heads * parts;
 #pragma unroll 1
         for (int64_t item = blockIdx.x / 8;; item += gridDim.x / 8) {
             const int64_t rank = item / per_seg;
-            if (rank >= range) return;
-            const int seg = p.seg_order[int(blockIdx.x % 8) * range + int(rank)];
-            if (p.cu[seg + 1] - p.cu[seg] <= p.skip_long) return;
+            if (rank >= count) return;
+            const int seg = p.seg_order[base + int(rank)];
             // the longest segments ahead of the others on a SIMD, which have time
             if (rank < 2) __builtin_amdgcn_s_setprio(3);
             else if (rank < 6) __builtin_amdgcn_s_setprio(2);
@@ -2273,17 +2294,17 @@ const OverlapAux *overlap_aux(hipStream_t caller) {
     return &aux[dev];
 }
 
-// The lazy kernel's MODE 0 instance: HB heads per workgroup, buffer form
-// where it applies.
-template <typename T, int CPL>
-const void *mode0_kernel(int hb, bool buf) {
+// The lazy kernel's instance for whole segments (MODE 0, or 4 beside the
+// chains): HB heads per workgroup, buffer form where it applies.
+template <typename T, int CPL, int MODE>
+const void *whole_kernel(int hb, bool buf) {
     if constexpr (std::is_same<T, bf16_t>::value && CPL == 4) {
         if (buf)
-            return hb == 2 ? reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 2, 0, true>)
-                           : reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 8, 0, true>);
+            return hb == 2 ? reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 2, MODE, true>)
+                           : reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 8, MODE, true>);
     }
-    return hb == 2 ? reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 2, 0>)
-                   : reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 8, 0>);
+    return hb == 2 ? reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 2, MODE>)
+                   : reinterpret_cast<const void *>(&lazy_forward_kernel<T, CPL, 8, MODE>);
 }
 
 // Whether the v, w rows and the read buffer fit the buffer form's 32-bit
@@ -2597,7 +2618,8 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             else
                 lazy_forward_kernel<T, CPL, 8, 2><<<g2, lthreads, 0, stream>>>(p);
         } else {
-            const void *kernel = mode0_kernel<T, CPL>(lazy_hb, buffer_form<T, CPL>(a));
+            const bool chains = pb.chain_events > 0 && a.read_banks > 0, buf = buffer_form<T, CPL>(a);
+            const void *kernel = chains ? whole_kernel<T, CPL, 4>(lazy_hb, buf) : whole_kernel<T, CPL, 0>(lazy_hb, buf);
             if (pb.seg_order) {
                 if (!pb.order_given) {
                     launch_segment_order(a.cu_seqlens, nseg, pb.seg_order, stream);
@@ -2609,7 +2631,7 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
                 const bool aligned_rounds = (int64_t(p.heads_per_block) * p.width * sizeof(T)) % 16 == 0 &&
                                             (int64_t(a.heads) * a.head_width * sizeof(T)) % 16 == 0;
                 const bool rounds = int(grid.y) > p.order_gpr && aligned_rounds;
-                if (a.read_banks > 0 && (rounds || pb.chain_events) && overlap_enabled()) {
+                if (a.read_banks > 0 && (rounds || chains) && overlap_enabled()) {
                     if (!rounds) p.order_gpr = int(grid.y);
                     if (const OverlapAux *ax = overlap_aux(stream)) {
                         // the shared events are recorded and waited for by one call at a time
@@ -2630,7 +2652,7 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             // without the auxiliary streams (switched off, or a capture that comes before
             // they exist) the long segments' chains still run, ahead of the others: the
             // same results whichever way a call goes
-            if (pb.seg_order && pb.chain_events > 0 && a.read_banks > 0) {
+            if (chains) {
                 p.skip_long = pb.chain_events;
                 if (int rc = launch_chains<T>(a, p, stream)) return rc;
             }

@@ -397,6 +397,45 @@ def test_forward_long_chains_match_oracle(device, heads, v, dtype, decay, monkey
         assert rel_err(ours, whole) < TOL, rel_err(ours, whole)
 
 
+@pytest.mark.parametrize('overlap', ['1', '0'])
+def test_forward_long_chains_in_any_order(device, overlap, monkeypatch):
+    """A caller's segment order only orders the work: with long segments behind short ones in their range (which end
+    the producer/consumer kernel's walk) and long ones of which only the first leads, every read and state is written
+    and within tolerance of the ranked order's."""
+    import dataclasses
+
+    from bdm_amd import ops
+    monkeypatch.setenv('BDM_COMBINE_OVERLAP', overlap)
+    gen = torch.Generator().manual_seed(41)
+    batch, time, heads, s, v, j = 2, 4608, 1, 8, 128, 512  # ranges of 128 segments, 4 of them to a sequence
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.05,
+                          torch.randint(0, j, (batch, time, 1), generator=gen),
+                          torch.randint(0, 2, (batch, time, 1), generator=gen) * 4) for _ in range(2))  # banks 0 and 4
+    ww, rw = (torch.rand(batch, time, 1, generator=gen).to(torch.bfloat16) for _ in range(2))
+    q, k, v_, g, b, w = controllers(batch, time, heads, s, v, gen)
+    state = initial_state(j, heads, s, v, gen)
+    dev = [t.to(device) for t in (q, k, v_, g, b, w, wi, ww, ri, rw, state)]
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    lengths = (meta.cu_seqlens[1:] - meta.cu_seqlens[:-1]).cpu()
+    assert sorted(lengths.tolist())[-4] > 4000 and int((lengths > 1000).sum()) == 4
+    ranked = 128 * torch.arange(8)[:, None] + torch.argsort(-lengths.view(8, 128), dim=1, stable=True)
+    near, far = ranked.clone(), ranked.clone()  # one long segment first, the other behind short ones
+    near[:, [1, 2]], far[:, [1, 90]] = ranked[:, [2, 1]], ranked[:, [90, 1]]
+    announce('forward long chains in any order', overlap)
+    results = []
+    for order in (ranked, near, far, ranked.flip(1), torch.arange(8 * 128).view(8, 128)):
+        final = torch.full((batch, j, heads, s, v), float('nan'), device=device, dtype=torch.float32)
+        scratch = torch.full((1 << 24,), 255, device=device, dtype=torch.uint8)  # unwritten reads are NaN
+        y = ops.routed_forward(*dev[:10], dev[10], dataclasses.replace(meta, segment_order=order.int().to(device)),
+                               bank_count=j, scale=s ** -0.5, routed_decay=True, round_interval=16, final_state=final,
+                               workspace=scratch)
+        torch.cuda.synchronize()
+        results.append((y, final))
+    for y, final in results:
+        assert torch.isfinite(y).all() and torch.isfinite(final).all()
+        assert rel_err(y, results[0][0]) < TOL and rel_err(final, results[0][1]) < TOL
+
+
 def test_forward_per_head_layout_and_determinism(device):
     from bdm_amd import bank_training
     gen = torch.Generator().manual_seed(11)
