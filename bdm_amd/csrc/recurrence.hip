@@ -2475,10 +2475,10 @@ int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void 
         pr.group_base = g0;
         pr.order_gpr = min(gpr, g1 - g0);
         if (int rc = launch_mode0<T>(kernel, dim3(nseg, unsigned(g1 - g0)), threads, pr, st)) return rc;
-        if (i == parts - 1)
-            if (int rc = record_phase(a, 1, st)) return rc;
         if (chain && hipStreamWaitEvent(st, chains_done, 0) != hipSuccess)
             return fail(BDM_ERR_LAUNCH, "forward: joining the chains");
+        if (i == parts - 1)
+            if (int rc = record_phase(a, 1, st)) return rc;
         const int h0 = g0 * p.heads_per_block;
         const int h1 = min(g1 * p.heads_per_block, p.heads);
         if (int rc = launch_combine_kernels<T>(a, zbuf, st, h0 * p.width, (h1 - h0) * p.width)) return rc;

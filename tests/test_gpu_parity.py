@@ -436,6 +436,31 @@ def test_forward_long_chains_in_any_order(device, overlap, monkeypatch):
         assert rel_err(y, results[0][0]) < TOL and rel_err(final, results[0][1]) < TOL
 
 
+def test_forward_phase_events_behind_long_chains(device):
+    """The second phase event comes after the recurrence: where a chain of 14,000 events (over 1 ms) outlasts all else,
+    what is left to the third is the combine alone (some 20 us; a quarter of the whole is the limit)."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(43)
+    batch, time, heads, s, v, j = 1, 8192, 1, 8, 128, 16
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.1,
+                          torch.randint(1, j, (batch, time, 1), generator=gen), 0) for _ in range(2))
+    ww, rw = (torch.rand(batch, time, 1, generator=gen).to(torch.bfloat16) for _ in range(2))
+    q, k, v_, g, b, w = controllers(batch, time, heads, s, v, gen)
+    state = initial_state(j, heads, s, v, gen)
+    dev = [t.to(device) for t in (q, k, v_, g, b, w, wi, ww, ri, rw, state)]
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    assert int((meta.cu_seqlens[1:] - meta.cu_seqlens[:-1]).max()) > 14000
+    announce('phase events behind long chains')
+    for _ in range(3):  # the first call creates the streams
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(3)]
+        ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
+                           round_interval=16, phase_events=events)
+        torch.cuda.synchronize()
+    recurrence, combine = (events[i].elapsed_time(events[i + 1]) for i in range(2))
+    print('recurrence', recurrence, 'combine', combine, flush=True)
+    assert 0 <= combine < 0.25 * (recurrence + combine)
+
+
 def test_forward_per_head_layout_and_determinism(device):
     from bdm_amd import bank_training
     gen = torch.Generator().manual_seed(11)
