@@ -213,6 +213,25 @@ def test_layer_batched_gradients(device):
         assert ours.shape == theirs.shape and norm_err(ours, theirs) < 2.5e-2
 
 
+def test_output_side_leaves_the_operator(device, monkeypatch):
+    """Gradients of the parameters behind the operator alone, by freezing the others or by asking for these, neither run
+    the operator's backward nor take snapshots for it."""
+    from bdm_amd import ops
+    layer, x, dy = trained_layer(device, 'BSDMConfig', 2, 8, {})
+    side = {n: p for n, p in layer.named_parameters() if n.startswith('output') or n.startswith('o_proj')}
+    assert len(side) == 6
+    print('CASE output side', flush=True)
+    whole = torch.autograd.grad(layer(x), list(side.values()), dy)
+    monkeypatch.setattr(ops, 'routed_backward', None)
+    asked = torch.autograd.grad(layer(x), list(side.values()), dy)
+    monkeypatch.setattr(ops, 'snapshot_buffer', None)
+    for n, p in layer.named_parameters():
+        p.requires_grad_(n in side)
+    frozen = torch.autograd.grad(layer(x.detach()), list(side.values()), dy)
+    for a, b, c in zip(whole, asked, frozen):
+        assert torch.equal(a, b) and torch.equal(a, c)
+
+
 def test_training_forward_keeps_module_hooks(device):
     """A projection that is hooked is called as a module, with the same output to BF16 rounding (read and write routes
     from one projection or several agree here: well separated scores)."""
