@@ -136,7 +136,7 @@ __device__ __forceinline__ void store_state(void *base, int dtype, int64_t offse
 // Bank sizes and intervals the S = 8 lazy kernel does not take: S in {4, 8,
 // 16, 32} padded rows (s_real of them live), any rounding or snapshot
 // interval, any width.  One wave per (segment, head, tile of columns); a lane
-// owns CPL value columns and R = S / RG rows (at most 8): RG groups of 64 / RG
+// owns CPL value columns and R = S / RG rows (8, or 16 at S = 16): RG groups of 64 / RG
 // lanes share a column's rows.
 //  * Stages of 16 events.  Lane e of the wave decodes event e; the loads of the
 //    next stage (columns into registers, row operands) go out before this
@@ -2810,7 +2810,15 @@ int dispatch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb,
     }
     if (a.bank_size <= 4) return launch_staged_forward<T, 4, 1, 1>(a, zbuf, pb, stream);
     if (a.bank_size <= 8) return launch_staged_forward<T, 8, 1, 1>(a, zbuf, pb, stream);
-    if (a.bank_size <= 16) return launch_staged_forward<T, 16, 2, 1>(a, zbuf, pb, stream);
+    if (a.bank_size <= 16) {
+        // Two row groups where waves of 64 columns are at most one per SIMD (256 CUs x 4): there a wave's
+        // latency counts, and halving its rows takes 102 us for 110 at 128 segments, H4 v64 (512 waves)
+        // and 105 for 114 at 256, H2 v128 (1,024).  With more waves the row operands, formed once per wave,
+        // count: 60 us for 58 at 2,048 segments, H1 v64 (2,048), 656 for 415 at 1,024, H8 v128 (16,384).
+        const int64_t waves = a.batch * a.bank_count * a.heads * ((a.head_width + kWave - 1) / kWave);
+        if (waves > 1024) return launch_staged_forward<T, 16, 1, 1>(a, zbuf, pb, stream);
+        return launch_staged_forward<T, 16, 2, 1>(a, zbuf, pb, stream);
+    }
     return launch_staged_forward<T, 32, 4, 1>(a, zbuf, pb, stream);
 }
 

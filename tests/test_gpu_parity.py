@@ -10,7 +10,7 @@ import sys
 import pytest
 import torch
 
-from _inputs import controllers, initial_state, oracle_reads, rel_err, routes
+from _inputs import controllers, global_rel_err, initial_state, oracle_reads, rel_err, routes
 from oracle import bdm_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -459,6 +459,48 @@ def test_forward_phase_events_behind_long_chains(device):
     recurrence, combine = (events[i].elapsed_time(events[i + 1]) for i in range(2))
     print('recurrence', recurrence, 'combine', combine, flush=True)
     assert 0 <= combine < 0.25 * (recurrence + combine)
+
+
+@pytest.mark.parametrize('heads,rows,v,dtype', [
+    (8, 16, 16, torch.float32), (9, 16, 16, torch.float32), (9, 9, 20, torch.float32), (5, 12, 66, torch.float32),
+    (9, 16, 24, torch.bfloat16)], ids=['1024_waves', '1152_waves', 'padded', 'two_tiles', 'bf16'])
+def test_forward_row_groups_of_16_rows(device, heads, rows, v, dtype):
+    """Banks of up to 16 rows, on both sides of 1,024 waves of 64 columns: reads, final states and the gradients behind
+    the snapshots of all heads together (beyond it, one row group) against each head alone (two)."""
+    from bdm_amd import bank_training, ops
+    gen = torch.Generator().manual_seed(heads + rows)
+    batch, time, j = 2, 33, 64
+    _, ww, wi = routes(batch, time, j, 4, gen, dtype=dtype)
+    _, rw, ri = routes(batch, time, j, 4, gen, dtype=dtype)
+    tensors = controllers(batch, time, heads, rows, v, gen, dtype)
+    state = initial_state(j, heads, rows, v, gen)
+    dy = torch.randn(batch, time, heads, v, generator=gen).to(dtype).to(device)
+    wi, ri = wi.to(device), ri.to(device)
+    meta = ops.dispatch_build(wi, ri, j)
+    announce('row groups', heads, rows, v)
+
+    def run(h):
+        leaves = [t.to(device).requires_grad_(True) for t in (*(t[:, :, h] for t in tensors), ww, rw, state[:, h])]
+        n = leaves[0].shape[2]
+        y = bank_training(*leaves[:6], wi, leaves[6], ri, leaves[7], leaves[8], j, rows ** -0.5)
+        final = torch.empty(batch, j, n, rows, v, device=device)
+        with torch.no_grad():
+            ops.routed_forward(*leaves[:6], wi, leaves[6], ri, leaves[7], leaves[8], meta, bank_count=j,
+                               scale=rows ** -0.5, routed_decay=True, final_state=final)
+        grads = torch.autograd.grad(y, leaves, dy[:, :, h].reshape(batch, time, -1))
+        torch.cuda.synchronize()
+        return y.detach().view(batch, time, n, v), final, grads
+
+    y, final, grads = run(slice(0, heads))
+    one = [run(slice(h, h + 1)) for h in range(heads)]
+    pairs = [(y, torch.cat([o[0] for o in one], 2)), (final, torch.cat([o[1] for o in one], 2))]
+    for i, g in enumerate(grads):
+        dim = {6: None, 7: None, 8: 1}.get(i, 2)  # the route weights' gradients sum over the heads
+        pairs.append((g, sum(o[2][i] for o in one) if dim is None else torch.cat([o[2][i] for o in one], dim)))
+    for ours, theirs in pairs:
+        # FP32 sums of up to 16 rows and 66 columns in another order along some tens of events; in BF16 values that
+        # round apart by an ulp of 2^-8, the heads' route-weight gradients rounded one by one
+        assert global_rel_err(ours, theirs) < (2e-5 if dtype == torch.float32 else 1e-2)
 
 
 def test_forward_per_head_layout_and_determinism(device):
