@@ -465,11 +465,14 @@ class BankedDeltaMemory(nn.Module):
             return False
         unbiased = (self.q_proj, self.k_proj, self.v_proj, *pair, self.b_proj, self.w_proj)
         biased = (router.base, router.read_residual, router.write_residual)
-        return (all(plain(m, nn.Linear) and m.bias is None for m in unbiased)
-                and all(plain(m, nn.Linear) and m.bias is not None for m in biased)
-                and type(hidden) in (Tensor, nn.Parameter)
+        if not all(plain(m, nn.Linear) and m._parameters.keys() == {'weight', 'bias'}
+                   and (m._parameters['bias'] is None) is without
+                   for group, without in ((unbiased, True), (biased, False)) for m in group):
+            return False
+        own = [t for m in (self, *unbiased, *biased) for t in m._parameters.values() if t is not None]
+        return (type(hidden) in (Tensor, nn.Parameter)
                 and all(type(t) in (Tensor, nn.Parameter) and t.dtype == torch.bfloat16 and t.device == hidden.device
-                        for t in self.parameters()))
+                        for t in own))
 
     def _forward_training(self, hidden: Tensor) -> Tensor:
         """forward under autograd: the projections that the operator reads as one,
