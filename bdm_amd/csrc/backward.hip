@@ -33,6 +33,7 @@
 // reference's rounding (role_bank_dispatch.py:99-131); route-weight
 // gradients add the heads' contributions in head order in FP32.
 // token_vjp_kernel: the same for shapes outside that kernel's limits.
+#include <algorithm>
 #include <type_traits>
 
 #include "bdm_common.h"
@@ -658,27 +659,35 @@ __device__ __forceinline__ float reduce_columns(const float (&x)[N], int lane, i
 
 // Chunk replay for the shapes the S = 8 chunk kernel does not take: S in {4,
 // 8, 16, 32} padded rows (s_real of them live), replay intervals C of 4, 8 or
-// 16 events.  One wave per (segment, head, tile of columns); chunks in
-// reverse.  A lane owns CPL value columns and R = S / RG rows (at most 8): RG
-// groups of 64 / RG lanes share a column's rows.
+// 16 events.  One workgroup of WAVES waves per (segment, head, tile of columns);
+// chunks in reverse.  A lane owns CPL value columns and R = S / RG
+// rows (at most 8): RG groups of 64 / RG lanes share a column's rows.
 //  * All C states of a chunk sit in registers (C*R*CPL of them, at most 128),
 //    so each write is replayed once.
 //  * The operands of the next chunk (columns, row operands, start state) are
 //    loaded when half of the chunk's events remain and put in LDS after them,
 //    so no event waits for a load; the row operands (exp, bf(b p) k, bf(q r))
 //    are formed once per event, spread over the lanes, not by every lane.
-//  * The sums over columns (U, X, P, dq) are permlane swaps and DPP adds.
+//  * The sums over columns (U, X, P, dq) are permlane swaps and DPP adds.  The
+//    waves of a tile add theirs in LDS, so that a wave of 16 or 32 columns has
+//    no rows of partial sums of its own in the workspace: with a row per wave it
+//    was three times as large at S = 32, and the training step of 8,192 tokens,
+//    H8 S16 v128, 256 banks took 3,148 us for 2,840, of 2,002 tokens, H4 S32
+//    v64, 64 banks 635 for 544.
 // Bound: instruction issue of the event loop.  Before it, one kernel loaded
 // every operand at its event and reduced by shuffles: 813 -> 103 us at 16,384
-// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 1,934 -> 229
-// us at 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events); of
-// these, addresses and route slots by readlane took 115 -> 103 and 239 -> 229.  Two
-// row groups at S = 16 (32 columns per wave) double the waves, which the
-// second size needs to fill the chip, and halve a lane's states.
-template <typename T, int S, int RG, int CPL, int C>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void staged_backward_kernel(
+// tokens, H1 S4 v128, 1024 banks (8,192 segments of 32 events), 1,934 -> 245
+// us at 2,002 tokens, H4 S16 v64, 64 banks (128 segments of 250 events; 231
+// with two one-wave workgroups in place of one of two, whose halves of the sums
+// token_vjp_kernel read in 47 us for 38); of these, addresses and route slots by
+// readlane took 115 -> 103 and 239 -> 229.  Two row groups at S = 16 (32 columns
+// per wave) double the waves, which the second size needs to fill the chip, and
+// halve a lane's states.
+template <typename T, int S, int RG, int CPL, int C, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2))) void staged_backward_kernel(
     BackwardParams<T> p) {
     constexpr int R = S / RG, kCols = kLanes / RG;
+    constexpr bool kShared = WAVES > 1;
     constexpr int NR = (C * S + kLanes - 1) / kLanes;  // (event, row) operands per lane
     constexpr int kKey = 0, kDecay = S, kErase = 2 * S, kStride = 3 * S + 4;
     struct Staged {
@@ -687,18 +696,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         float g[NR];
         uint32_t m0[R][CPL];  // start state (BF16 or FP32 bits)
     };
-    __shared__ int4 s_meta[2][C];
-    __shared__ __align__(16) float s_rows[C][kStride];
-    __shared__ float s_cols[C][2 * CPL][kCols];  // write: v, bf(w p); read: dy
+    // each wave's own, but for the sums of a tile's waves by chunk % 3 (write: U, X, P; read: dq)
+    __shared__ int4 s_meta_[WAVES][2][C];
+    __shared__ __align__(16) float s_rows_[WAVES][C][kStride];
+    __shared__ float s_cols_[WAVES][C][2 * CPL][kCols];  // write: v, bf(w p); read: dy
+    __shared__ float s_part[kShared ? 3 : 1][WAVES][C][kShared ? 3 * S : 1];
+    const int wave = kShared ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kLanes) : 0;
+    auto &s_meta = s_meta_[wave];
+    auto &s_rows = s_rows_[wave];
+    auto &s_cols = s_cols_[wave];
 
     int seg, head, tile;
     block_item(p, seg, head, tile);
     const int bank = seg % p.banks;
     const int64_t bidx = seg / p.banks;
-    const int lane = threadIdx.x;
+    const int lane = kShared ? int(threadIdx.x) % kLanes : int(threadIdx.x);
     const int row0 = lane / kCols * R, col = lane % kCols;
-    const int col0 = (tile * kCols + col) * CPL;
+    const int col0 = ((tile * WAVES + wave) * kCols + col) * CPL;
     const bool live = col0 < p.width;
+    // waves of the tile with columns
+    const int busy = min(WAVES, (p.width - tile * WAVES * kCols * CPL + kCols * CPL - 1) / (kCols * CPL));
     const int colc = live ? col0 : p.width - CPL;  // lanes past the width load valid columns and zero them
     const int64_t start = p.cu[seg], end = p.cu[seg + 1];
     const int count = int((end - start + C - 1) / C);
@@ -833,6 +850,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc) dm[r][cc] = 0.f;
 
+    int sums = 0;  // the chunk's buffer of s_part
     // Route slot of event e from the chunk's metadata, lane e holding event e's.
     auto slot_of = [&](int e, const int4 &meta, int per_token) {
         return int64_t(__builtin_amdgcn_readlane(meta.x, e)) * per_token + __builtin_amdgcn_readlane(meta.y, e);
@@ -884,7 +902,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
             bool mine;
             const float o = reduce_columns<RG, 12>(red, lane, at, mine);
             const int r = row0 + 4 * g + (at & 3);
-            if (mine && r < p.s_real) wp[(at >> 2) * p.s_real + r] = o;
+            if constexpr (kShared) {
+                if (mine) s_part[sums][wave][e][(at >> 2) * S + r] = o;
+            } else {
+                if (mine && r < p.s_real) wp[(at >> 2) * p.s_real + r] = o;
+            }
         }
     };
     // Adjoint of read e with the state st it read: dq = scale st dy, dm += scale eq dy^T.
@@ -906,24 +928,93 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         int at;
         bool mine;
         const float o = reduce_columns<RG, R>(red, lane, at, mine) * p.scale;
-        if (mine && row0 + at < p.s_real) rp[row0 + at] = o;
+        if constexpr (kShared) {
+            if (mine) s_part[sums][wave][e][row0 + at] = o;
+        } else {
+            if (mine && row0 + at < p.s_real) rp[row0 + at] = o;
+        }
+    };
+    // The chunk's sums over the tile's waves, in wave order: wave w takes the events
+    // w, w + WAVES, ..., a lane one or two of an event's 3S sums.  rows: lane e event
+    // e's row of the workspace.
+    auto store_sums = [&](int from, uint64_t rows, uint32_t wmask, uint32_t rmask) {
+        constexpr int kEvents = C / WAVES, kPer = (3 * S + kLanes - 1) / kLanes;
+        float sum[kEvents][kPer];
+#pragma unroll
+        for (int n = 0; n < kEvents; ++n)
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                const int i = min(lane + q * kLanes, 3 * S - 1);
+                sum[n][q] = s_part[from][0][wave + n * WAVES][i];
+#pragma unroll
+                for (int w = 1; w < WAVES; ++w) sum[n][q] += w < busy ? s_part[from][w][wave + n * WAVES][i] : 0.f;
+            }
+#pragma unroll
+        for (int n = 0; n < kEvents; ++n) {
+            const int e = wave + n * WAVES;
+            const int count = wmask >> e & 1u ? 3 * S : (rmask >> e & 1u ? S : 0);  // (a read has dq in U's place)
+            float *row = reinterpret_cast<float *>(const_cast<char *>(lane_ptr(rows, e)));
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                const int i = lane + q * kLanes, r = i % S;
+                if (i < count && r < p.s_real) row[i / S * p.s_real + r] = sum[n][q];
+            }
+        }
+    };
+    // (bases, strides and the difference in registers: a choice between two kernel arguments becomes a load of one)
+    const int64_t wsums = (int64_t(tile) * p.nt * p.kw * p.heads + head) * 3 * p.s_real, wstride = int64_t(p.heads) * 3 * p.s_real;
+    const int64_t rsums = (int64_t(tile) * p.nt * p.kr * p.heads + head) * p.s_real, rstride = int64_t(p.heads) * p.s_real;
+    const uint64_t wbase = reinterpret_cast<uint64_t>(p.wpart + wsums), rbase = reinterpret_cast<uint64_t>(p.rpart + rsums);
+    const int more = p.kr - p.kw;
+    auto sums_row = [&](const int4 &meta) {
+        const int64_t slot = int64_t(meta.x) * (p.kw + (meta.z ? more : 0)) + meta.y;
+        return (meta.z ? rbase : wbase) + uint64_t(slot * (meta.z ? rstride : wstride)) * sizeof(float);
     };
 
+    // The sums of the chunk before, stored once every wave of the tile has passed it: half a chunk later, so
+    // that no wave waits for another's last event (a third buffer, since the others may be a chunk further).
+    uint64_t done_rows = 0;
+    uint32_t done_writes = 0, done_reads = 0;
+    auto finish_sums = [&] {
+        __syncthreads();
+        store_sums(sums ? sums - 1 : 2, done_rows, done_writes, done_reads);
+    };
+    auto keep_sums = [&](const int4 &meta, uint32_t wmask, uint32_t rmask) {
+        done_rows = sums_row(meta), done_writes = wmask, done_reads = rmask;
+        sums = sums == 2 ? 0 : sums + 1;
+    };
+    if constexpr (kShared) {
+        if (wave >= busy) {  // no columns: only its share of the sums
+            for (int c = count - 1; c >= 0; --c) {
+                const int4 mine = load_meta(c);
+                const bool valid = lane < chunk_len(c);
+                if (c < count - 1) finish_sums();
+                keep_sums(mine, uint32_t(__ballot(valid && mine.z == 0)), uint32_t(__ballot(valid && mine.z != 0)));
+            }
+            if (count > 0) finish_sums();
+            return;
+        }
+    }
+    // Order among a wave's own LDS accesses (which run in order).
+    auto sync_wave = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     float m0[R][CPL];
     if (count > 0) {
         store_meta(count - 1, load_meta(count - 1));
         int4 prev = make_int4(0, 0, 0, 0);
         if (count > 1) prev = load_meta(count - 2);
-        __syncthreads();
+        sync_wave();
         Staged sg;
         issue_stage(count - 1, sg);
         if (count > 1) store_meta(count - 2, prev);
-        __syncthreads();
+        sync_wave();
         finish_stage(count - 1, sg, m0);
     }
 #pragma unroll 1
     for (int c = count - 1; c >= 0; --c) {
-        __syncthreads();
+        sync_wave();
         const int len = chunk_len(c);
         const int4 mine = s_meta[c & 1][lane & (C - 1)];
         const uint32_t wmask = uint32_t(__ballot(lane < len && mine.z == 0)) & ((1u << C) - 1);
@@ -947,15 +1038,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void st
         Staged sg;
         if (c >= 2) meta2 = load_meta(c - 2);
         if (c >= 1) issue_stage(c - 1, sg);
+        if (kShared && c < count - 1) finish_sums();
 #pragma unroll
         for (int e = C / 2 - 1; e >= 0; --e) {
             if (wmask & (1u << e)) write_back(e, mine, st[e]);
             else if (rmask & (1u << e)) read_back(e, mine, st[e]);
         }
-        __syncthreads();
+        sync_wave();
         if (c >= 2) store_meta(c - 2, meta2);
         if (c >= 1) finish_stage(c - 1, sg, m0);
+        if constexpr (kShared) keep_sums(mine, wmask, rmask);
     }
+    if (kShared && count > 0) finish_sums();
     // adjoint of the segment's initial state (FP32, per sequence)
     if (live) {
         const int64_t off = ((bidx * p.banks + bank) * p.heads + head) * p.s_real * p.width + col0;
@@ -1360,9 +1454,16 @@ int columns_per_lane(const bdm_backward_args &a) {
     return a.bank_size <= 4 && a.head_width % 2 == 0 && a.head_width > kLanes ? 2 : 1;
 }
 
-int column_tiles(const bdm_backward_args &a) {
+// Columns of a tile, the unit of the partial sums over columns in the
+// workspace, and the waves of a workgroup that share it.
+int tile_columns(const bdm_backward_args &a) { return a.bank_size <= 8 ? 2 * kLanes : kLanes; }
+
+int column_tiles(const bdm_backward_args &a) { return (a.head_width + tile_columns(a) - 1) / tile_columns(a); }
+
+int tile_waves(const bdm_backward_args &a) {
     const int columns = kLanes / (chunk_path(a) ? 1 : row_groups(a)) * columns_per_lane(a);
-    return (a.head_width + columns - 1) / columns;
+    const int waves = std::min(tile_columns(a) / columns, (a.head_width + columns - 1) / columns);
+    return waves == 3 ? 4 : waves;
 }
 
 // The per-token gradient kernel: one wave per head and one lane per (slot, row).
@@ -1439,6 +1540,7 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
     const int64_t nseg = a.batch * a.bank_count;
     p.xcd_remap = (nseg % 8 == 0) ? 1 : 0;
     const dim3 grid(unsigned(nseg), unsigned(a.heads), unsigned(p.tiles));
+    const int threads = tile_waves(a) * kLanes;
     if constexpr (CHUNK) {
         const int64_t events = p.nt * (p.kw + p.kr);
         const unsigned blocks = unsigned((events + 255) / 256);
@@ -1450,10 +1552,10 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
         launch_segment_order(p.cu, nseg, ws.seg_order, stream);
         if (int rc = check_launch("segment_order_kernel")) return rc;
         p.seg_order = ws.seg_order;
-        p.order_gpr = order_groups_per_round(reinterpret_cast<const void *>(kernel), kLanes, nseg,
+        p.order_gpr = order_groups_per_round(reinterpret_cast<const void *>(kernel), threads, nseg,
                                              int(grid.y * grid.z));
     }
-    kernel<<<grid, kLanes, 0, stream>>>(p);
+    kernel<<<grid, threads, 0, stream>>>(p);
     if (int rc = check_launch(CHUNK ? "chunk_backward_kernel" : "staged_backward_kernel")) return rc;
 
     VjpParams<T> v{};
@@ -1498,7 +1600,7 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
                 token_grad_kernel<T, CPL, false, WAVES><<<blocks, threads, 0, stream>>>(v);
         };
         constexpr std::integral_constant<int, 4> four{};
-        // the head's waves share its tiles of 128 columns (the tiles of the kernels of pairs, up to 8 rows)
+        // the head's waves share its tiles of 128 columns (tile_columns up to 8 rows)
         if (v.wph > 1 && p.tiles <= 2 * v.wph)
             launch(four, std::true_type{});
         else if (v.wph > 1 || a.head_width > 2 * kLanes)
@@ -1528,10 +1630,19 @@ int launch_backward(const bdm_backward_args &a, const Workspace &ws, void (*kern
 template <typename T, int S, int C>
 int launch_staged(const bdm_backward_args &a, const Workspace &ws, hipStream_t stream) {
     constexpr int RG = S <= 8 ? 1 : S / 8;  // row_groups
+    auto launch = [&](auto cpl, auto waves) {
+        return launch_backward<T, false>(
+            a, ws, &staged_backward_kernel<T, S, RG, decltype(cpl)::value, C, decltype(waves)::value>, stream);
+    };
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, 2> two{};
     if constexpr (S == 4) {
-        if (columns_per_lane(a) == 2) return launch_backward<T, false>(a, ws, &staged_backward_kernel<T, S, 1, 2, C>, stream);
+        if (columns_per_lane(a) == 2) return launch(two, one);
     }
-    return launch_backward<T, false>(a, ws, &staged_backward_kernel<T, S, RG, 1, C>, stream);
+    if constexpr (S == 32) {
+        if (tile_waves(a) == 4) return launch(one, std::integral_constant<int, 4>{});
+    }
+    return tile_waves(a) == 2 ? launch(one, two) : launch(one, one);
 }
 
 template <typename T>

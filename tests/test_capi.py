@@ -128,6 +128,23 @@ def test_backward_rejects_bad_arguments(lib):
     assert lib.bdm_snapshot_rows(1000, 16) == 62 and lib.bdm_snapshot_rows(0, 16) == 0
 
 
+@pytest.mark.parametrize('rows,width,interval', [(4, 130, 16), (4, 129, 16), (6, 128, 16), (8, 200, 8), (16, 64, 8),
+                                                 (12, 100, 8), (32, 64, 4), (32, 130, 4)])
+def test_backward_partial_sums_per_tile(lib, rows, width, interval):
+    """The workspace holds one row of partial sums per tile of columns, 128 of them for banks of up to 8 rows and 64
+    for larger ones, however many waves a tile's columns take."""
+    from bdm_amd import _lib
+    args = _lib.BackwardArgs()
+    args.batch, args.time, args.heads, args.bank_size, args.head_width = 1, 50, 3, rows, width
+    args.bank_count, args.write_banks, args.read_banks = 12, 4, 2
+    args.ctrl_dtype = args.initial_dtype = _lib.BDM_BF16
+    args.snapshot_dtype, args.snapshot_interval = _lib.BDM_F32, interval
+    tiles = -(-width // (128 if rows <= 8 else 64))
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    assert lib.bdm_backward_workspace_size(ctypes.byref(args)) == (
+        up(50 * 4 * 3 * width * 4) + up(tiles * 3 * 50 * 4 * 3 * rows * 4) + up(tiles * 50 * 2 * 3 * rows * 4))
+
+
 def test_struct_layouts_match_the_header(tmp_path):
     """sizeof/offsetof of every argument struct, compiled from the header with
     gcc, equal the ctypes mirrors the Python layer passes."""

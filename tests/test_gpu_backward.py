@@ -151,6 +151,15 @@ def test_staged_backward_fp32(device, case):
     check_against_oracle(device, (*case, True, torch.float32, torch.float32), 500 + case[3] + case[4])
 
 
+@pytest.mark.parametrize('case', [(1, 21, 1, 16, 80, 6, 2), (1, 21, 2, 32, 64, 6, 2), (1, 19, 1, 32, 70, 4, 4),
+                                  (2, 17, 1, 4, 131, 6, 2), (1, 40, 1, 8, 193, 4, 4)],
+                         ids=lambda c: f's{c[3]}v{c[4]}')
+def test_staged_backward_tile_waves(device, case):
+    """Tiles whose columns take two or four waves, all of them with columns or some without."""
+    announce('staged backward tile waves', case)
+    check_against_oracle(device, (*case, True, torch.float32, torch.float32), 700 + case[3] + case[4])
+
+
 @pytest.mark.parametrize('s,compact', [(4, None), (4, True), (8, True), (16, None), (32, None)])
 def test_staged_backward_bf16(device, s, compact):
     """BF16 state rounded every 16, 8 or 4 events (an odd width keeps S = 8 off the chunk kernel)."""
