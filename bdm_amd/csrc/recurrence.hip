@@ -1538,7 +1538,8 @@ __device__ __forceinline__ void chain_columns(const ForwardParams<T> &p, int seg
     __syncthreads();
 }
 
-// The consumer of a 64-column tile: the state of one column per lane.
+// The consumer of a 64-column tile: the state of one column per lane, rounded
+// every stage (chain_events takes no other policy, and no snapshots).
 template <typename T, int NC>
 __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg, int vhead, int tile, int which,
                                               ChainLds<NC> &lds) {
@@ -1548,7 +1549,6 @@ __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg
     const int64_t bidx = seg / p.banks;
     const int64_t start = p.cu[seg], end = p.cu[seg + 1];
     const int nstages = int((end - start + NE - 1) / NE);
-    const bool rounding = p.round_interval > 0;
     const int64_t head_cols = int64_t(vhead / p.split) * S * p.row_stride + int64_t(vhead % p.split) * p.width +
                               tile * kWave + lane;
     const int64_t state_offset = int64_t(bank) * p.s_heads * S * p.row_stride + head_cols;
@@ -1558,16 +1558,8 @@ __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg
         const int64_t at = bidx * p.init_bstride + state_offset + int64_t(r) * p.row_stride;
         const float x = p.init_dtype == BDM_BF16 ? to_f32(static_cast<const bf16_t *>(p.initial)[at])
                                                  : static_cast<const float *>(p.initial)[at];
-        h[r] = rounding ? round_bf16(x) : x;
+        h[r] = round_bf16(x);
     }
-    auto store_h = [&](void *base, int dtype, int64_t offset) {
-#pragma unroll
-        for (int r = 0; r < S; ++r) {
-            const int64_t at = offset + int64_t(r) * p.row_stride;
-            if (dtype == BDM_BF16) static_cast<bf16_t *>(base)[at] = from_f32<bf16_t>(h[r]);
-            else static_cast<float *>(base)[at] = h[r];
-        }
-    };
     auto load8 = [&](const float *row, float (&x)[S]) {
         const float4 lo = reinterpret_cast<const float4 *>(row)[0], hi = reinterpret_cast<const float4 *>(row)[1];
         x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w, x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
@@ -1582,13 +1574,8 @@ __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg
         const uint32_t writes = __builtin_amdgcn_readfirstlane(lds.writes[buf]);
         const int eager = __builtin_amdgcn_readfirstlane(lds.eager[buf]);
         if (s > 0) {
-            if (rounding) {
 #pragma unroll
-                for (int r = 0; r < S; ++r) h[r] = round_bf16(h[r]);
-            }
-            // snapshot of the state before event 16 s of the segment (see staged_forward_kernel)
-            if (p.snap)
-                store_h(p.snap, p.snap_dtype, (start / NE + s - 1) * p.s_heads * S * p.row_stride + head_cols);
+            for (int r = 0; r < S; ++r) h[r] = round_bf16(h[r]);
         }
         if (!eager) {
             chain_stage<false>(h, coef, beta, coef, lds.x[buf][which], writes, lds.z[buf][which], lane);
@@ -1603,8 +1590,15 @@ __device__ __forceinline__ void chain_consume(const ForwardParams<T> &p, int seg
         for (int r = 0; r < S; ++r) h[r] *= fold[r];
         __syncthreads();
     }
-    if (p.final_state)
-        store_h(p.final_state, p.final_dtype, bidx * (int64_t(p.banks) * p.s_heads * S * p.row_stride) + state_offset);
+    if (p.final_state) {
+        const int64_t offset = bidx * (int64_t(p.banks) * p.s_heads * S * p.row_stride) + state_offset;
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const int64_t at = offset + int64_t(r) * p.row_stride;
+            if (p.final_dtype == BDM_BF16) static_cast<bf16_t *>(p.final_state)[at] = from_f32<bf16_t>(h[r]);
+            else static_cast<float *>(p.final_state)[at] = h[r];
+        }
+    }
     __syncthreads();
 }
 
