@@ -29,9 +29,15 @@ def _dtype_code(dtype: torch.dtype) -> int:
     raise ValueError(f'unsupported dtype {dtype}; expected bfloat16 or float32')
 
 
+# The raw handle of a device's current stream without a Stream object per launch; torch's binding for
+# compiled code, which a build may lack.
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+
+
 def _stream(device: torch.device) -> int:
-    # the raw handle of the current stream, without a Stream object per launch
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _require_gpu(*tensors: Tensor) -> torch.device:

@@ -231,3 +231,17 @@ def test_router_backward_without_rows(lib):
     assert lib.bdm_router_backward(None, None, None, None, 0, 8, 8, 4, 0, None) == 0
     assert lib.bdm_router_backward(None, None, None, None, -1, 8, 8, 4, 0, None) != 0
     assert lib.bdm_router_backward(None, None, None, None, 1, 8, 8, 4, 0, None) != 0
+
+
+def test_stream_handle_without_the_raw_binding(monkeypatch):
+    """Launches take the public Stream object's handle where torch has no raw one, and for a device without an index."""
+    import types
+
+    import torch
+
+    from bdm_amd import ops
+    monkeypatch.setattr(torch.cuda, 'current_stream', lambda device: types.SimpleNamespace(cuda_stream=17))
+    monkeypatch.setattr(ops, '_raw_stream', lambda index: 5)
+    assert ops._stream(torch.device('cuda', 0)) == 5 and ops._stream(torch.device('cuda')) == 17
+    monkeypatch.setattr(ops, '_raw_stream', None)
+    assert ops._stream(torch.device('cuda', 0)) == 17
