@@ -2429,6 +2429,24 @@ int launch_overlapped_stage(const bdm_forward_args &a, ForwardParams<T> p, const
     return record_phase(a, 2, stream);
 }
 
+// The chains of a forward whose other segments are one launch: on an auxiliary
+// stream, the others and the combine on the caller's, which a routing without
+// long segments then leaves only for the wait after the others.
+template <typename T>
+int launch_beside_chains(const bdm_forward_args &a, ForwardParams<T> p, const void *kernel, dim3 grid, int threads,
+                         const T *zbuf, const OverlapAux &ax, const PieceBuffers &pb, hipStream_t stream) {
+    p.skip_long = pb.chain_events;
+    if (hipEventRecord(ax.fork, stream) != hipSuccess || hipStreamWaitEvent(ax.stream[0], ax.fork, 0) != hipSuccess)
+        return fail(BDM_ERR_LAUNCH, "forward: forking the chains");
+    if (int rc = launch_chains<T>(a, p, ax.stream[0])) return rc;
+    if (int rc = launch_mode0<T>(kernel, grid, threads, p, stream)) return rc;
+    if (hipEventRecord(ax.join[0], ax.stream[0]) != hipSuccess || hipStreamWaitEvent(stream, ax.join[0], 0) != hipSuccess)
+        return fail(BDM_ERR_LAUNCH, "forward: joining the chains");
+    if (int rc = record_phase(a, 1, stream)) return rc;
+    if (int rc = launch_combine_kernels<T>(a, zbuf, stream)) return rc;
+    return record_phase(a, 2, stream);
+}
+
 template <typename T, int CPL>
 int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void *kernel, unsigned nseg, int groups,
                       int threads, const T *zbuf, const OverlapAux &ax, const PieceBuffers &pb, hipStream_t stream) {
@@ -2436,7 +2454,7 @@ int launch_overlapped(const bdm_forward_args &a, ForwardParams<T> p, const void 
         return launch_overlapped_stage<T, CPL>(a, p, kernel, nseg, groups, threads, zbuf, ax, pb, stream);
     const int gpr = p.order_gpr;
     const bool chain = pb.chain_events > 0;
-    int parts = groups > gpr ? overlap_parts((groups + gpr - 1) / gpr, groups) : 1;
+    int parts = overlap_parts((groups + gpr - 1) / gpr, groups);
     if (chain) parts = min(parts, kOverlapAux - 1);
     hipEvent_t chains_done = ax.join[kOverlapAux - 1];
     // part i's stream: the caller's and the auxiliary ones, or behind the chains the auxiliary ones
@@ -2612,8 +2630,9 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             else
                 lazy_forward_kernel<T, CPL, 8, 2><<<g2, lthreads, 0, stream>>>(p);
         } else {
-            const bool chains = pb.chain_events > 0 && a.read_banks > 0, buf = buffer_form<T, CPL>(a);
-            const void *kernel = chains ? whole_kernel<T, CPL, 4>(lazy_hb, buf) : whole_kernel<T, CPL, 0>(lazy_hb, buf);
+            const bool buf = buffer_form<T, CPL>(a);
+            const void *kernel = whole_kernel<T, CPL, 0>(lazy_hb, buf);
+            bool chains = pb.chain_events > 0 && a.read_banks > 0;
             if (pb.seg_order) {
                 if (!pb.order_given) {
                     launch_segment_order(a.cu_seqlens, nseg, pb.seg_order, stream);
@@ -2625,11 +2644,20 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
                 const bool aligned_rounds = (int64_t(p.heads_per_block) * p.width * sizeof(T)) % 16 == 0 &&
                                             (int64_t(a.heads) * a.head_width * sizeof(T)) % 16 == 0;
                 const bool rounds = int(grid.y) > p.order_gpr && aligned_rounds;
+                // Without rounds to overlap, the fork for the chains costs a routing without long segments 10 us
+                // of GPU time and 25 of the host's: only where the calls are long, by their sequences (4 x 4,096
+                // tokens, 1,024 columns, 256 banks: uniform 227 -> 240 us, Zipf 1.1 1,670 -> 637) or their
+                // segments (2 x 3,000, 512 columns, 64 banks: 242 -> 260, 1,217 -> 705).  Below, a call is as long
+                // as its host work: 2,048 tokens, 256 banks 77 us, 105 with the fork (Zipf 1.1: 807, 566).
+                const int64_t mean = a.time * (int64_t(a.write_banks) + a.read_banks) / a.bank_count;
+                chains = chains && (rounds || a.time >= 4096 || mean >= 256);
+                if (chains) kernel = whole_kernel<T, CPL, 4>(lazy_hb, buf);
                 if (a.read_banks > 0 && (rounds || chains) && overlap_enabled()) {
                     if (!rounds) p.order_gpr = int(grid.y);
                     if (const OverlapAux *ax = overlap_aux(stream)) {
                         // the shared events are recorded and waited for by one call at a time
                         std::lock_guard<std::mutex> lock(overlap_launch_mutex());
+                        if (!rounds) return launch_beside_chains<T>(a, p, kernel, grid, lthreads, zbuf, *ax, pb, stream);
                         return launch_overlapped<T, CPL>(a, p, kernel, grid.x, int(grid.y), lthreads, zbuf, *ax, pb,
                                                          stream);
                     }
@@ -2710,14 +2738,16 @@ int64_t stage_slots(const bdm_forward_args &a) {
 // others (0: the path is off).  MODE 0 takes ~0.21 us per event of a lone
 // segment, 2T events at most, and ~0.63 ns per event and 1,024 columns over the
 // whole chip, (KW + KR) B T events: where batch * columns is small the longest
-// segment of a skewed routing outlasts everything else.  At 65,536 columns times
-// route slots (B = 4, 1,024 columns, 8 + 8 banks, T = 8,192, 2,048 banks, Zipf
-// 1.1: 15,000 of 524,288 events in one segment) the whole forward went from 3.53
-// to 1.21 ms; at twice that a fork costs 3 us of a uniform routing's 424, and
-// the path is left out.  Long is 2,048 events, a third of the time of everything
-// else there (1,024: 1.28 ms, 3,072: 1.22), or 4 times the mean.  Without
-// snapshots only: a training step's backward walks the same chain at its own
-// pace.
+// segment of a skewed routing outlasts everything else.  B = 4, 1,024 columns, 8 +
+// 8 banks, T = 8,192, 2,048 banks, Zipf 1.1: 15,000 of 524,288 events in one
+// segment, the whole forward 3.53 -> 1.21 ms.  The line at 98,304 columns times
+// route slots spares larger calls the chains' launch, not because these gain
+// nothing: at 131,072 (B = 8, T = 4,096, 256 banks) it costs a uniform routing 3 us
+// of 396 and would take a skewed one (Zipf 1.1) from 1,756 to 822.  Below T =
+// 2,048 it would cost 25 us of 83 (B = 4, T = 1,024, 256 banks).  Long is 2,048
+// events, a third of the time of everything else at the first size (1,024: 1.28
+// ms, 3,072: 1.22), or 4 times the mean.  Without snapshots only: a training step's
+// backward walks the same chain at its own pace.
 bool order_path(const bdm_forward_args &a);
 int chain_events(const bdm_forward_args &a) {
     const int64_t columns = int64_t(a.heads) * a.head_width, slots = int64_t(a.write_banks) + a.read_banks;

@@ -397,17 +397,18 @@ def test_forward_long_chains_match_oracle(device, heads, v, dtype, decay, monkey
         assert rel_err(ours, whole) < TOL, rel_err(ours, whole)
 
 
-@pytest.mark.parametrize('overlap', ['1', '0'])
-def test_forward_long_chains_in_any_order(device, overlap, monkeypatch):
+@pytest.mark.parametrize('heads,overlap', [(1, '1'), (1, '0'), (16, '1'), (16, '0')])
+def test_forward_long_chains_in_any_order(device, heads, overlap, monkeypatch):
     """A caller's segment order only orders the work: with long segments behind short ones in their range (which end
     the producer/consumer kernel's walk) and long ones of which only the first leads, every read and state is written
-    and within tolerance of the ranked order's."""
+    and within tolerance of the ranked order's, and that of the forward without it.  The other segments of 16 heads are
+    two rounds of launches, those of one head one beside the chains."""
     import dataclasses
 
     from bdm_amd import ops
     monkeypatch.setenv('BDM_COMBINE_OVERLAP', overlap)
     gen = torch.Generator().manual_seed(41)
-    batch, time, heads, s, v, j = 2, 4608, 1, 8, 128, 512  # ranges of 128 segments, 4 of them to a sequence
+    batch, time, s, v, j = 2, 4608, 8, 128, 512  # ranges of 128 segments, 4 of them to a sequence
     wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.05,
                           torch.randint(0, j, (batch, time, 1), generator=gen),
                           torch.randint(0, 2, (batch, time, 1), generator=gen) * 4) for _ in range(2))  # banks 0 and 4
@@ -421,11 +422,14 @@ def test_forward_long_chains_in_any_order(device, overlap, monkeypatch):
     ranked = 128 * torch.arange(8)[:, None] + torch.argsort(-lengths.view(8, 128), dim=1, stable=True)
     near, far = ranked.clone(), ranked.clone()  # one long segment first, the other behind short ones
     near[:, [1, 2]], far[:, [1, 90]] = ranked[:, [2, 1]], ranked[:, [90, 1]]
-    announce('forward long chains in any order', overlap)
+    announce('forward long chains in any order', heads, overlap)
     results = []
-    for order in (ranked, near, far, ranked.flip(1), torch.arange(8 * 128).view(8, 128)):
+    for order in (ranked, near, far, ranked.flip(1), torch.arange(8 * 128).view(8, 128), None):
+        if order is None:
+            monkeypatch.setenv('BDM_SEGMENT_ORDER', '0')
+            order = ranked
         final = torch.full((batch, j, heads, s, v), float('nan'), device=device, dtype=torch.float32)
-        scratch = torch.full((1 << 24,), 255, device=device, dtype=torch.uint8)  # unwritten reads are NaN
+        scratch = torch.full((1 << 26,), 255, device=device, dtype=torch.uint8)  # unwritten reads are NaN
         y = ops.routed_forward(*dev[:10], dev[10], dataclasses.replace(meta, segment_order=order.int().to(device)),
                                bank_count=j, scale=s ** -0.5, routed_decay=True, round_interval=16, final_state=final,
                                workspace=scratch)
@@ -434,6 +438,42 @@ def test_forward_long_chains_in_any_order(device, overlap, monkeypatch):
     for y, final in results:
         assert torch.isfinite(y).all() and torch.isfinite(final).all()
         assert rel_err(y, results[0][0]) < TOL and rel_err(final, results[0][1]) < TOL
+
+
+def test_forward_long_chains_in_a_graph(device):
+    """The chains on an auxiliary stream beside the other segments, captured: replays with eager work between them give
+    the eager results, also after new inputs in the same buffers."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(47)
+    batch, time, heads, s, v, j = 1, 4224, 2, 8, 128, 16
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.1,
+                          torch.randint(1, j, (batch, time, 1), generator=gen), 0) for _ in range(2))
+    ww, rw = (torch.rand(batch, time, 1, generator=gen).to(torch.bfloat16) for _ in range(2))
+    sets = [[t.to(device) for t in (*controllers(batch, time, heads, s, v, gen),)] for _ in range(2)]
+    fixed = [t.to(device) for t in (wi, ww, ri, rw, initial_state(j, heads, s, v, gen))]
+    meta = ops.dispatch_build(fixed[0], fixed[2], j)
+
+    def run(tensors):
+        final = torch.empty(batch, j, heads, s, v, device=device)
+        y = ops.routed_forward(*tensors, *fixed, meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
+                               round_interval=16, final_state=final)
+        return y, final
+
+    announce('chains in a graph')
+    eager = [run(tensors) for tensors in sets]  # (also creates the streams)
+    torch.cuda.synchronize()
+    inputs = [t.clone() for t in sets[0]]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run(inputs)
+    for which in (0, 1, 0, 1, 1):
+        for buffer, t in zip(inputs, sets[which]):
+            buffer.copy_(t)
+        graph.replay()
+        torch.cuda.synchronize()
+        again = run(sets[which])
+        for ours, theirs, live in zip(captured, eager[which], again):
+            assert torch.equal(ours, theirs) and torch.equal(live, theirs)
 
 
 def test_forward_phase_events_behind_long_chains(device):
