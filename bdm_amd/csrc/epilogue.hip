@@ -31,14 +31,17 @@ struct ControllerParams {
     int heads, hv, param_dtype, qk_norm;
 };
 
-// A workgroup takes TB consecutive tokens: the 8-column chunks of v and w,
-// chunk by chunk for all TB tokens at once (TB loads in flight per thread),
-// then the 4H rows of q, k, b, g of each token (S values, 8 at a time).  VEC:
-// every 8-element group of the inputs and outputs is 16-byte aligned.  Bound:
-// HBM.  As one-wave workgroups of one item per thread it was bound by their
-// number (163,840 at 32,768 tokens, H8 S8 v128): 101 -> 71 us there, 305 MB.
+// Items of a token: the 4H rows of q, k, b, g (S values, 8 at a time) and the
+// 8-column chunks of v and w.  TB = 1: one-wave workgroups, one item per thread
+// (grid: tokens, items / 64).  TB = 4: a workgroup takes four consecutive
+// tokens, first their chunks, four loads in flight per thread, then their rows.
+// VEC: every 8-element group of the inputs and outputs is 16-byte aligned.
+// Bound: HBM for many tokens, where TB = 1 is bound by the number of its
+// workgroups (163,840 at 32,768 tokens, H8 S8 v128: 101 -> 71 us, 305 MB; at 8,192
+// 24.3 -> 20.3), latency for few, where its spread over them counts (1,024 tokens:
+// 7.8 us, 9.4 with a workgroup per token; H1 S8 v2048: 8.2, 12.4).
 template <typename T, int S, bool VEC, int TB>
-__global__ __launch_bounds__(256) void controller_epilogue_kernel(ControllerParams<T> p) {
+__global__ __launch_bounds__(TB == 1 ? 64 : 256) void controller_epilogue_kernel(ControllerParams<T> p) {
     static_assert(S % 8 == 0, "S");
     const int chunks = p.heads * p.hv / 8;
     const int64_t token0 = int64_t(blockIdx.x) * TB;
@@ -57,7 +60,7 @@ __global__ __launch_bounds__(256) void controller_epilogue_kernel(ControllerPara
                 for (int j = 0; j < 8; ++j) dst[r0 + j] = from_f32<std::remove_pointer_t<decltype(dst)>>(t[j]);
         }
     };
-    for (int c = threadIdx.x; c < 2 * chunks; c += int(blockDim.x)) {
+    auto chunk = [&](int c) {
         const bool is_v = c < chunks;
         const int col = (is_v ? c : c - chunks) * 8;
         const T *src = p.proj + (is_v ? p.v_col : p.w_col) + col;
@@ -73,12 +76,10 @@ __global__ __launch_bounds__(256) void controller_epilogue_kernel(ControllerPara
             for (int j = 0; j < 8; ++j) x[t][j] = is_v ? silu_f(x[t][j]) : sigmoid_f(x[t][j]);
             store_row<8>(dst + (token0 + t) * total, x[t]);
         }
-    }
-    for (int i = threadIdx.x; i < 4 * p.heads * TB; i += int(blockDim.x)) {
-        const int64_t token = token0 + i / (4 * p.heads);
-        if (token >= p.tokens) break;
+    };
+    auto row_item = [&](int64_t token, int it) {
         const T *row = p.proj + token * p.proj_stride;
-        const int it = i % (4 * p.heads), h = it % p.heads;
+        const int h = it % p.heads;
         float y[S];
         if (it < 2 * p.heads) {
             // q or k: silu, rounded, then the l2 normalization over the head's S values
@@ -92,6 +93,16 @@ __global__ __launch_bounds__(256) void controller_epilogue_kernel(ControllerPara
             decay_row<T, S, VEC>(p.f + token * p.f_stride + h * S, p.a_log, p.dt_bias, p.param_dtype, h, y);
             store(p.g + token * hs + h * S, y);
         }
+    };
+    const int rows = 4 * p.heads;
+    if constexpr (TB == 1) {
+        const int it = int(blockIdx.y) * 64 + int(threadIdx.x);
+        if (it < rows) row_item(token0, it);
+        else if (it < rows + 2 * chunks) chunk(it - rows);
+    } else {
+        for (int c = threadIdx.x; c < 2 * chunks; c += int(blockDim.x)) chunk(c);
+        for (int i = threadIdx.x; i < rows * TB && token0 + i / rows < p.tokens; i += int(blockDim.x))
+            row_item(token0 + i / rows, i % rows);
     }
 }
 
@@ -197,16 +208,18 @@ int launch_controller(const bdm_controller_args &a, hipStream_t stream) {
     p.hv = a.head_width;
     p.param_dtype = a.param_dtype;
     p.qk_norm = a.qk_norm;
-    // four tokens a workgroup where that still leaves four workgroups per CU
-    const bool many = a.tokens >= 4096;
-    const unsigned blocks = unsigned(many ? (a.tokens + 3) / 4 : a.tokens);
+    // four tokens a workgroup where that still leaves four workgroups per CU and a head has more than two
+    // chunks (H16 S8 v16, whose 64 rows a token outweigh them, 8,192 tokens: 17.8 us, 20.5 with four)
+    const bool many = a.tokens >= 4096 && a.head_width > 16;
+    const unsigned items = unsigned(4 * a.heads + 2 * (int64_t(a.heads) * a.head_width / 8));
+    const dim3 blocks(unsigned(many ? (a.tokens + 3) / 4 : a.tokens), many ? 1 : (items + 63) / 64);
     // 16-byte groups everywhere: aligned bases, strides and column offsets in multiples of 8 elements
     const bool vec = aligned(a.proj, 16) && aligned(a.f, 16) && aligned(a.q, 16) && aligned(a.k, 16) &&
                      aligned(a.b, 16) && aligned(a.g, 16) && aligned(a.dt_bias, 16) && a.proj_stride % 8 == 0 &&
                      a.f_stride % 8 == 0 && a.q_col % 8 == 0 && a.k_col % 8 == 0 && a.v_col % 8 == 0 &&
                      a.b_col % 8 == 0 && a.w_col % 8 == 0;
 #define BDM_CTRL_TB(S, V) (many ? (controller_epilogue_kernel<T, S, V, 4><<<blocks, 256, 0, stream>>>(p), 0) \
-                                : (controller_epilogue_kernel<T, S, V, 1><<<blocks, 256, 0, stream>>>(p), 0))
+                                : (controller_epilogue_kernel<T, S, V, 1><<<blocks, 64, 0, stream>>>(p), 0))
 #define BDM_CTRL(S) (vec ? BDM_CTRL_TB(S, true) : BDM_CTRL_TB(S, false))
     switch (a.bank_size) {
         case 8: BDM_CTRL(8); break;
