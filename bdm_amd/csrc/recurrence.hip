@@ -2595,7 +2595,20 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
     {
         // the prep role needs one lane per (event, head, half): 32 per head
         const int lthreads = lazy_hb == 2 ? 64 : 256;
-        if (pb.max_pieces > 0) {
+        const bool buf = buffer_form<T, CPL>(a);
+        const void *kernel = whole_kernel<T, CPL, 0>(lazy_hb, buf);
+        p.order_gpr = int(grid.y);
+        if (pb.seg_order && (pb.max_pieces == 0 || a.time <= kPieceEvents))
+            p.order_gpr = order_groups_per_round(kernel, lthreads, nseg, int(grid.y));
+        // rounds whose heads' columns split y in whole 16-byte groups
+        const bool aligned_rounds = (int64_t(p.heads_per_block) * p.width * sizeof(T)) % 16 == 0 &&
+                                    (int64_t(a.heads) * a.head_width * sizeof(T)) % 16 == 0;
+        const bool rounds = int(grid.y) > p.order_gpr && aligned_rounds;
+        // A token of this router writes and reads a bank once, so a segment holds at most 2T events: up to two
+        // pieces' worth it runs whole, in one launch instead of four (two pieces cost two passes over theirs: 512
+        // tokens, H4 v64, 27 + 4.5 + 4 + 4 us).  Not as several launches with overlapped combines (512 tokens,
+        // one head of 2,048 columns, 1,024 banks: 76 us in pieces, 109), which longer calls without pieces gain by.
+        if (pb.max_pieces > 0 && (a.time > kPieceEvents || rounds)) {
             // prefill policy: long segments run as balanced pieces
             p.items = pb.items;
             p.n_items = pb.count;
@@ -2630,8 +2643,6 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
             else
                 lazy_forward_kernel<T, CPL, 8, 2><<<g2, lthreads, 0, stream>>>(p);
         } else {
-            const bool buf = buffer_form<T, CPL>(a);
-            const void *kernel = whole_kernel<T, CPL, 0>(lazy_hb, buf);
             bool chains = pb.chain_events > 0 && a.read_banks > 0;
             if (pb.seg_order) {
                 if (!pb.order_given) {
@@ -2639,11 +2650,6 @@ int launch_forward(const bdm_forward_args &a, T *zbuf, const PieceBuffers &pb, h
                     if (int rc = check_launch("segment_order_kernel")) return rc;
                 }
                 p.seg_order = pb.seg_order;
-                p.order_gpr = order_groups_per_round(kernel, lthreads, nseg, int(grid.y));
-                // rounds whose heads' columns split y in whole 16-byte groups
-                const bool aligned_rounds = (int64_t(p.heads_per_block) * p.width * sizeof(T)) % 16 == 0 &&
-                                            (int64_t(a.heads) * a.head_width * sizeof(T)) % 16 == 0;
-                const bool rounds = int(grid.y) > p.order_gpr && aligned_rounds;
                 // Without rounds to overlap, the fork for the chains costs a routing without long segments 10 us
                 // of GPU time and 25 of the host's: only where the calls are long, by their sequences (4 x 4,096
                 // tokens, 1,024 columns, 256 banks: uniform 227 -> 240 us, Zipf 1.1 1,670 -> 637) or their
@@ -2949,11 +2955,6 @@ extern "C" int bdm_forward(const bdm_forward_args *a, void *workspace, size_t wo
     PieceBuffers pb;
     pb.max_pieces = max_pieces(*a);
     if (pb.max_pieces > INT32_MAX / 2) return fail(BDM_ERR_UNSUPPORTED, "forward: too many pieces");
-    // A token writes and reads a bank at most once, so a segment holds at most
-    // 2T events: up to two pieces' worth it runs whole, in one launch instead of
-    // four (two pieces cost two passes over theirs: 512 tokens, H4 v64, 27 + 4.5
-    // + 4 + 4 us), and the combine may run beside it.
-    if (2 * a->time <= 2 * kPieceEvents) pb.max_pieces = 0;
     if (pb.max_pieces) {
         char *at = ws + forward_zbuf_bytes(a);
         const size_t n = size_t(pb.max_pieces);

@@ -543,6 +543,34 @@ def test_forward_row_groups_of_16_rows(device, heads, rows, v, dtype):
         assert global_rel_err(ours, theirs) < (2e-5 if dtype == torch.float32 else 1e-2)
 
 
+@pytest.mark.parametrize('time', [300, 512, 513])
+def test_short_forward_in_pieces_matches_whole(device, time, monkeypatch):
+    """FP32 state, up to two pieces' worth of events a segment: with 32 heads in two rounds a call runs in pieces, in bank
+    order (one launch) whole; the piece sums differ from the whole chain's in FP32 association only."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(time)
+    batch, heads, s, v, j = 1, 32, 8, 128, 512
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.1,
+                          torch.randint(1, j, (batch, time, 1), generator=gen), 0) for _ in range(2))
+    ww, rw = (torch.rand(batch, time, 1, generator=gen) for _ in range(2))
+    q, k, v_, g, b, w = controllers(batch, time, heads, s, v, gen, torch.float32)
+    state = initial_state(j, heads, s, v, gen)
+    dev = [t.to(device) for t in (q, k, v_, g, b, w, wi, ww, ri, rw, state)]
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    assert int((meta.cu_seqlens[1:] - meta.cu_seqlens[:-1]).max()) > 512
+    announce('short forward in pieces', time)
+    results = []
+    for order in ('1', '0'):
+        monkeypatch.setenv('BDM_SEGMENT_ORDER', order)
+        final = torch.empty(batch, j, heads, s, v, device=device)
+        y = ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,
+                               final_state=final)
+        torch.cuda.synchronize()
+        results.append((y, final))
+    for ours, theirs in zip(*results):
+        assert torch.isfinite(ours).all() and global_rel_err(ours, theirs) < 1e-4
+
+
 def test_forward_per_head_layout_and_determinism(device):
     from bdm_amd import bank_training
     gen = torch.Generator().manual_seed(11)
