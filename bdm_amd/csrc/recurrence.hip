@@ -1279,7 +1279,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 3 ?
 //    load (lanes 0..31 the column pairs of event 2i, lanes 32..63 of 2i + 1),
 //    leaves x = bf(w p) v in LDS and stores the z of the stage before.
 // The arithmetic is lazy_forward_kernel's, in its order, apart from the rounding
-// of x + sum.  Bound: the consumer's issue and one barrier, ~75 ns per event
+// of x + sum.  Bound: the consumer's issue and one barrier, ~79 ns per event
 // (lazy_forward_kernel: 211).  Measured on the way there (1,000-stage chain, one
 // launch alone): row operands read from LDS at each event 2,780 us (each event
 // waits for LDS), by row_newbcast 2,240; the preparation moved to producers
@@ -2717,7 +2717,10 @@ int64_t max_pieces(const bdm_forward_args &a) {
 // BDM_STAGE_PATH=1 runs segments longer than kPieceEvents under the
 // rounding policy on the stage path; otherwise they run whole (the default:
 // its launches cost a forward without long segments ~3 % at C2, and its
-// buffers ~2-3 GiB of workspace at the C2 and C4 sizes).
+// buffers ~2-3 GiB of workspace at the C2 and C4 sizes).  It pays for short
+// skewed calls that the chains leave out (Zipf 1.1, 1,024 columns, 256 banks, 2 x
+// 2,048 tokens: 820 us whole, 547 so), not where the chains run (4 x 4,096: 633,
+// 1,204) nor where the chip is full (8 x 4,096: 1,753, 2,133).
 bool stage_enabled() {
     const char *e = getenv("BDM_STAGE_PATH");
     return e && e[0] == '1' && e[1] == 0;

@@ -152,7 +152,9 @@ inline int order_groups_per_round(const void *kernel, int block_threads, int64_t
 // Whether a launch over `nseg` segments can take the order.
 inline bool order_geometry(int64_t nseg) { return nseg > 0 && nseg % 8 == 0 && nseg / 8 <= kOrderMaxRange; }
 
-// BDM_SEGMENT_ORDER=0 keeps bank order (results are identical either way).
+// BDM_SEGMENT_ORDER=0 keeps bank order.  Results are identical either way but for a
+// forward's long segments, which run on chain_forward_kernel only with the order
+// (another FP32 association).
 inline bool order_enabled() {
     const char *e = getenv("BDM_SEGMENT_ORDER");
     return !(e && e[0] == '0' && e[1] == 0);

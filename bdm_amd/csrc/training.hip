@@ -6,10 +6,10 @@
 // projections and rounded once, in one pass instead of the chains of
 // elementwise, cast, reduce and scatter kernels that autograd makes of them.
 // At 8,192 tokens, 1,024 columns, H8 S8 v128 the layer's training step (the
-// input projected once, by the concatenated weights) went from 2,800 to 1,564
-// us: 48 us here for the controllers, 31 for the output interface and 6 for
-// each role's routes, where the chains took ~600 us and the separate products'
-// gradients ~600.
+// input projected by the concatenated weights, apart from the output gate) took
+// 2,370 us and takes 1,560: 46 us here for the controllers, 31 for the output
+// interface and 6 for each role's routes, where the chains took ~600 us and the
+// separate products' gradients ~600.
 #include "epilogue_ops.h"
 
 namespace bdm {
@@ -39,9 +39,9 @@ __device__ __forceinline__ void sigmoid8(const float (&t)[8], float (&s)[8]) {
 // One workgroup per token; a thread takes items of 8 columns (S for the rows
 // of a head): 4H rows of q, k, b, g, then the chunks of v, w, gate, read and
 // write.  Bound: HBM, the projection and every gradient read once and the
-// projection's gradient written once (59 MB of each at 8,192 tokens and 3,520
-// columns); the last three kinds are copies into the one gradient that the two
-// backward GEMMs read.
+// projection's gradient written once (40 MB of each at 8,192 tokens and the 2,432
+// columns of H8 S8 v128, 256 banks, without the gate); the last three kinds are
+// copies into the one gradient that the two backward GEMMs read.
 template <typename T, int S>
 __global__ __launch_bounds__(256) void controller_backward_kernel(ControllerGradParams<T> p) {
     const int64_t token = blockIdx.x;

@@ -63,13 +63,18 @@ def _output_ops(raw, gate, weight, bias, eps, kind):
     return normalized * torch.sigmoid(gate).to(raw.dtype)
 
 
+# Tests for the wrapped tensors of batched gradients, as far as this torch has them, and the one for global module
+# hooks (without it every module counts as hooked).
+_WRAPPED = [f for f in (getattr(getattr(torch._C, '_functorch', None), name, None)
+                        for name in ('is_legacy_batchedtensor', 'is_functorch_wrapped_tensor')) if f is not None]
+_global_hooks = getattr(nn.modules.module, '_has_any_global_hook', lambda: True)
+
+
 def _differentiable(grads) -> bool:
     """Whether a backward has to run in torch ops: its result is differentiated
     again (create_graph; a kernel's would end the graph), or the gradients are
     batched (is_grads_batched)."""
-    wrapped = torch._C._functorch
-    return torch.is_grad_enabled() or any(wrapped.is_legacy_batchedtensor(t) or wrapped.is_functorch_wrapped_tensor(t)
-                                          for t in grads)
+    return torch.is_grad_enabled() or any(wrapped(t) for t in grads for wrapped in _WRAPPED)
 
 
 def _torch_gradients(form, inputs, grads):
@@ -455,7 +460,7 @@ class BankedDeltaMemory(nn.Module):
                 m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
 
         if (hidden.dtype != torch.bfloat16 or torch.is_autocast_enabled('cuda') or not self._fused_supported(hidden)
-                or self.head_value_width % 8 or self.factor_route_width % 8 or nn.modules.module._has_any_global_hook()
+                or self.head_value_width % 8 or self.factor_route_width % 8 or _global_hooks()
                 or any(getattr(type(self), n) is not getattr(BankedDeltaMemory, n) or n in self.__dict__
                        for n in _TRAINING_METHODS)):
             return False

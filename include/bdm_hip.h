@@ -206,11 +206,15 @@ typedef struct bdm_forward_args {
     /* Profiling: NULL, or three hipEvent_t the call records: before the
      * recurrence kernels, after the last recurrence launch (the last head-group
      * round, whose read combine follows it; the earlier rounds' combines run
-     * beside the later rounds on an auxiliary stream) and after the combine,
-     * so a caller can time the recurrence and the combine left after it. */
+     * beside the later rounds on an auxiliary stream; the long segments' chains
+     * have ended too) and after the combine, so a caller can time the recurrence
+     * and the combine left after it. */
     void *phase_events[3];
     /* NULL, or the longest-first segment order bdm_route_dispatch wrote for
-     * this dispatch ([batch*J] int32); the call computes it itself otherwise. */
+     * this dispatch ([batch*J] int32); the call computes it itself otherwise.
+     * Any order that permutes each eighth of the segments within itself gives
+     * every result; long segments that do not lead theirs run on another kernel,
+     * in another FP32 association. */
     const int32_t *segment_order;
 } bdm_forward_args;
 
@@ -442,7 +446,7 @@ int bdm_output_backward(const bdm_output_grad_args *args, void *stream);
 /*
  * Gradient of bdm_router_select's weights with respect to its scores (autograd
  * of gdn2_banks.py:104-114): weights, indices, grad_weights [rows, selected],
- * grad_scores [rows, J1 + J2], contiguous.
+ * grad_scores [rows, J1 + J2], contiguous.  No rows are no work.
  */
 int bdm_router_backward(const void *weights, const int64_t *indices, const void *grad_weights, void *grad_scores,
                         int64_t rows, int32_t factor_first, int32_t factor_second, int32_t selected, int32_t dtype,
