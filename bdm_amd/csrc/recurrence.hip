@@ -2259,9 +2259,21 @@ std::mutex &overlap_launch_mutex() {
     return mu;
 }
 
+// Whether the auxiliary streams are the caller's to use: not part of a capture,
+// or of the caller's own.  (One that has used them holds them to its end.)
+bool aux_free(const OverlapAux &ax, hipStream_t caller) {
+    hipStreamCaptureStatus theirs = hipStreamCaptureStatusNone, mine = hipStreamCaptureStatusNone;
+    unsigned long long their_id = 0, my_id = 0;
+    if (hipStreamGetCaptureInfo(ax.stream[0], &theirs, &their_id) != hipSuccess) return false;
+    if (theirs == hipStreamCaptureStatusNone) return true;
+    return hipStreamGetCaptureInfo(caller, &mine, &my_id) == hipSuccess && mine == hipStreamCaptureStatusActive &&
+           theirs == mine && my_id == their_id;
+}
+
 // The device's auxiliary streams and events, or null (then the serial order
-// runs): creation failed, or the caller's stream is being captured and they
-// do not exist yet (resources are not created under capture).
+// runs): creation failed, the caller's stream is being captured and they do not
+// exist yet (resources are not created under capture), or another capture holds
+// them.
 const OverlapAux *overlap_aux(hipStream_t caller) {
     constexpr int kMaxDev = 64;
     static std::mutex mu;
@@ -2270,7 +2282,7 @@ const OverlapAux *overlap_aux(hipStream_t caller) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return nullptr;
     std::lock_guard<std::mutex> lock(mu);
-    if (aux[dev].fork) return &aux[dev];
+    if (aux[dev].fork) return aux_free(aux[dev], caller) ? &aux[dev] : nullptr;
     if (failed[dev]) return nullptr;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(caller, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;

@@ -152,8 +152,8 @@ def test_staged_backward_fp32(device, case):
 
 
 @pytest.mark.parametrize('case', [(1, 21, 1, 16, 80, 6, 2), (1, 21, 2, 32, 64, 6, 2), (1, 19, 1, 32, 70, 4, 4),
-                                  (2, 17, 1, 4, 131, 6, 2), (1, 40, 1, 8, 193, 4, 4), (1, 20, 1, 5, 300, 6, 2),
-                                  (1, 15, 1, 4, 517, 6, 2), (1, 20, 2, 3, 514, 6, 2)],
+                                  (2, 17, 1, 4, 131, 6, 2), (1, 40, 1, 8, 193, 4, 4), (1, 20, 1, 5, 304, 6, 2),
+                                  (1, 15, 1, 4, 520, 6, 2), (1, 20, 2, 7, 776, 6, 2)],
                          ids=lambda c: f's{c[3]}v{c[4]}')
 def test_staged_backward_tile_waves(device, case):
     """Tiles whose columns take two or four waves, all of them with columns or some without, and heads of more than 256

@@ -476,6 +476,42 @@ def test_forward_long_chains_in_a_graph(device):
             assert torch.equal(ours, theirs) and torch.equal(live, theirs)
 
 
+def test_forward_beside_another_capture(device):
+    """A capture that used the auxiliary streams holds them to its end: a forward on a stream outside it meanwhile runs in
+    the serial order, with the same results, and leaves the capture whole."""
+    from bdm_amd import ops
+    gen = torch.Generator().manual_seed(53)
+    batch, time, heads, s, v, j = 1, 4224, 1, 8, 128, 16
+    wi, ri = (torch.where(torch.rand(batch, time, 1, generator=gen) < 0.1,
+                          torch.randint(1, j, (batch, time, 1), generator=gen), 0) for _ in range(2))
+    ww, rw = (torch.rand(batch, time, 1, generator=gen).to(torch.bfloat16) for _ in range(2))
+    dev = [t.to(device) for t in (*controllers(batch, time, heads, s, v, gen), wi, ww, ri, rw,
+                                  initial_state(j, heads, s, v, gen))]
+    meta = ops.dispatch_build(dev[6], dev[8], j)
+    run = lambda: ops.routed_forward(*dev[:10], dev[10], meta, bank_count=j, scale=s ** -0.5, routed_decay=True,  # noqa: E731
+                                     round_interval=16)
+    announce('beside another capture')
+    other = torch.cuda.Stream()
+    expected = run().clone()
+    with torch.cuda.stream(other):
+        run()  # (the allocator's blocks of that stream)
+    torch.cuda.synchronize()
+    graph, capturing = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(capturing):
+        graph.capture_begin(capture_error_mode='relaxed')
+        captured = run()
+        with torch.cuda.stream(other):
+            outside = run()
+        graph.capture_end()
+    torch.cuda.synchronize()
+    assert torch.equal(outside, expected)
+    for _ in range(2):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, expected)
+
+
 def test_forward_phase_events_behind_long_chains(device):
     """The second phase event comes after the recurrence: where a chain of 14,000 events (over 1 ms) outlasts all else,
     what is left to the third is the combine alone (some 20 us; a quarter of the whole is the limit)."""
