@@ -511,7 +511,7 @@ class BankedDeltaMemory(nn.Module):
         gate, raw = self.output_gate(hidden), raw.reshape(*lead, self.value_width)
         if type(gate) is not Tensor or gate.dtype != raw.dtype or gate.shape != raw.shape:  # a gate of another kind
             return self.o_proj(_output_ops(raw, gate, *self._output_norm()))
-        normalized = _OutputInterface.apply(*(t.reshape(-1, self.value_width) for t in (raw, gate)),
+        normalized = _OutputInterface.apply(*(ops._aligned(t.reshape(-1, self.value_width)) for t in (raw, gate)),
                                             *self._output_norm())
         return self.o_proj(normalized.view(*lead, self.value_width))
 

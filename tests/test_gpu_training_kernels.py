@@ -213,6 +213,30 @@ def test_layer_batched_gradients(device):
         assert ours.shape == theirs.shape and norm_err(ours, theirs) < 2.5e-2
 
 
+GATES = {  # what a hook on the output gate returns
+    'another stride': lambda o: torch.cat([o, o], -1)[..., :o.shape[-1]],
+    'another order': lambda o: o.transpose(1, 2).contiguous().transpose(1, 2),
+    'unaligned': lambda o: torch.cat([o, o], -1)[..., 3:3 + o.shape[-1]],
+    'FP32': lambda o: o.float(),
+    'broadcast': lambda o: o[..., :1]}
+
+
+@pytest.mark.parametrize('kind', GATES)
+def test_hooked_output_gate(device, kind):
+    """The output gate is called as a module on the fused path too: whatever its hook makes of the projection."""
+    layer, x, dy = trained_layer(device, 'BSDMConfig', 2, 8, {})
+    layer.output_gate.register_forward_hook(lambda m, i, o: GATES[kind](o))
+    leaves = [x, layer.output_gate.weight, layer.output_norm_weight, layer.q_proj.weight]
+    print('CASE hooked gate', kind, flush=True)
+
+    def gradients():
+        y = layer(x)
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+
+    for ours, theirs in zip(*both_paths(layer, x, gradients)):
+        assert ours.shape == theirs.shape and norm_err(ours, theirs) < 2.5e-2
+
+
 def test_output_side_leaves_the_operator(device, monkeypatch):
     """Gradients of the parameters behind the operator alone, by freezing the others or by asking for these, neither run
     the operator's backward nor take snapshots for it."""
